@@ -10,22 +10,9 @@
 // attention that reference/vllm/v1/attention/backends/mla/prefill/
 // sm70_triton.py:54-187 (_varlen_attention) computes per sequence in fp32.
 //
-// Workgroup = (query tile of 64 QB rows, sequence, head), 4 waves; wave w
-// owns query rows [16 QB w, +16 QB).  Key tiles of KT keys stream through
-// two LDS stages by LDS-DMA (K and V rows at padded pitches, so that the rows
-// of an MFMA operand spread over the banks), the next tile in flight while
-// the current one is used; two workgroups share a CU.  Per tile and wave:
-//   * S^T = K Q^T (v_mfma_f32_16x16x32): keys are the A operand read from
-//     LDS, the wave's queries the B operand resident in registers;
-//   * online softmax per query column in exp2 with the scale folded in; the
-//     tile maximum is the only cross-lane reduction (the row sums stay
-//     per-lane partials until the end);
-//   * O^T += V^T P^T: the S^T accumulator layout is the B-operand layout of
-//     P^T (keys 4g..4g+3 of two 16-key blocks per lane), so P never leaves
-//     registers; V^T comes from ds_read_b64_tr_b16 transpose reads in the
-//     same key order.
-// bf16 inputs use the bf16 MFMA; their P is split into two bf16 parts
-// (p = hi + lo), so the PV product keeps ~16 bits of P.
+// Three kernels: 16-bit inputs at head dims up to (192, 128) (LDS ring, 32
+// query rows per wave), 16-bit inputs at (256, 256), whose Q and O rows leave
+// no registers for that form, and fp32 inputs.
 #include <float.h>
 
 #include "capi_internal.h"
@@ -53,6 +40,8 @@ struct VaArgs {
   const int32_t* cu_k;
   int64_t q_st, q_sh, k_st, k_sh, v_st, v_sh, o_st, o_sh;  // element strides
   int H, total_q, n_qtiles, causal;
+  int o16;    // output rows are 16-byte aligned
+  int pairs;  // > 0: 1-D grid in pair-major order over this many (sequence, head) pairs
   float scale_log2;  // softmax scale * log2(e)
   float scale;
 };
@@ -98,6 +87,13 @@ __device__ __forceinline__ void va_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// 16-bit inputs at (256, 256).  Workgroup = (query tile of 64 QB rows,
+// sequence, head), 4 waves; wave w owns query rows [16 QB w, +16 QB).  Key
+// tiles of KT keys stream through two LDS stages by LDS-DMA, the next tile in
+// flight while the current one is used.  Per tile and wave: S^T = K Q^T
+// (v_mfma_f32_16x16x32, keys the A operand read from LDS, queries resident in
+// registers), online softmax per query column, O^T += V^T P^T with P in
+// registers and V^T from ds_read_b64_tr_b16.  bf16 P is split into hi + lo.
 template <bool BF16, int DQK, int DV, int QB, int KT, int MINB>
 __global__ void __launch_bounds__(kVaThreads, MINB) varlen_attn_kernel(VaArgs a) {
   using Sh = VaShape<DQK, DV, KT>;
@@ -321,14 +317,412 @@ int launch_va(const VaArgs& a0, int num_seqs, int max_q_len, hipStream_t st) {
   return check_launch("varlen_attention");
 }
 
+// ---------------------------------------------------------------------------
+// 16-bit inputs, head dims (192, 128), (128, 128) and (64, 64).
+//
+// Workgroup = (query tile of 128 rows, sequence, head), 4 waves of 32 rows;
+// two workgroups share a CU.  Steps of 32 keys stream through a four-slot LDS
+// ring by LDS-DMA, three steps ahead, one barrier per step.  A wave's step i:
+//   * S^T(i+1) = K Q^T (v_mfma_f32_32x32x16: keys the A operand from LDS, the
+//     wave's 32 queries the B operand resident in registers) beside the
+//     exponentials of step i: independent work for the matrix cores and the
+//     VALU in one basic block;
+//   * O^T += V^T P^T: the S^T accumulator layout (query = lane % 32, keys
+//     8 (e / 4) + 4 (lane / 32) + e % 4) is the B-operand layout of P^T, so P
+//     stays in registers; V^T comes from ds_read_b64_tr_b16 transpose reads in
+//     the same key order; the maximum of S^T(i+1) is taken beside it.
+// A query's 32 scores of a step sit in two lanes, so its maximum is one lane
+// swap.  O is rescaled only when a maximum grows by more than kVaLazy binades
+// over the one in use (p then stays <= 2^kVaLazy, far inside fp16), and the
+// causal / tail masks run only in steps that hold a masked key.
+// bf16 inputs keep P as two bf16 parts (p = hi + lo, two PV MFMAs), ~16 bits.
+//
+// LDS layouts, free of bank conflicts without pads: K as 64-byte blocks
+// (4 pieces of 16 B) per key, block-major (block b of key r at 2048 b + 64 r),
+// piece p at p ^ ((r >> 2) & 3): the 32 rows of a QK read cover every bank
+// once per 16-lane phase.  V rows are whole, 64-byte group u of key r at
+// u ^ (r & 3) (DV = 64: u ^ ((r >> 1) & 1)): the 4 keys x 64 bytes of a
+// half-wave's transpose read cover the 64 banks.  Both are applied to the
+// DMA's source address, so every DMA instruction writes 1 KB in order and
+// reads 64-byte or longer runs.
+//
+// Bound: the matrix cores, with the softmax's VALU work beside them (per step
+// and wave 20 MFMAs of 32 clk at (192, 128) fp16, 28 in bf16, against ~120-160
+// VALU instructions, 16 of them exponentials at a quarter rate); on short
+// sequences the first Q and K reads of each workgroup.  Measured, 64 heads,
+// (192, 128), against the two-stage kernel kept for (256, 256): causal 16k
+// 11.08 -> 5.66 ms fp16 (972 TFLOP/s; a large library product reaches 1180
+// here), 12.90 -> 6.86 ms bf16; causal 800-3203-token prompts, 10007 tokens,
+// 1386 -> 815 us fp16, 1460 -> 855 us bf16.  Of that, the 32-row waves, the
+// ring and the lazy rescale gave 6.3 ms, whole (sequence, head) pairs per XCD
+// 5.9 ms, the grouped MFMA / VALU order 5.66 ms (the compiler's own order put
+// the exponentials before the MFMAs).  Measured level: 2 K reads ahead instead
+// of 3, two steps per loop iteration, groups of 4-16 query tiles per pair.
+// ---------------------------------------------------------------------------
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+constexpr float kVaLazy = 8.f;
+constexpr int kVaAhead = 3;  // K reads in flight ahead of their MFMA
+
+template <bool BF16>
+__device__ __forceinline__ f32x16 mma32x32(const u32x4& a, const u32x4& b, f32x16 c) {
+  if constexpr (BF16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+// two fp32 values as one packed pair of 16-bit values (RNE)
+template <bool BF16>
+__device__ __forceinline__ uint32_t pack16(float x, float y) {
+  if constexpr (BF16) {
+    const bf16x2 p = {(__bf16)x, (__bf16)y};
+    return __builtin_bit_cast(uint32_t, p);
+  } else {
+    const f16x2 p = {(f16)x, (f16)y};
+    return __builtin_bit_cast(uint32_t, p);
+  }
+}
+
+// max of a lane's value and the lane's ^ 32, in both
+__device__ __forceinline__ float xor32_max(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                                  false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+template <int DQK, int DV>
+struct VaRing {
+  static constexpr int KT = 32;              // keys per step
+  static constexpr int SLOTS = 4;
+  static constexpr int KBYTES = KT * DQK * 2;
+  static constexpr int VBYTES = KT * DV * 2;
+  static constexpr int SLOT = KBYTES + VBYTES;
+  static constexpr int NKD = DQK / 64;       // K DMA instructions per wave and step
+  static constexpr int NVD = DV / 64;        // V DMA instructions per wave and step
+  static constexpr int ND = NKD + NVD;
+};
+
+template <bool BF16, int DQK, int DV>
+__global__ void __launch_bounds__(kVaThreads, 2) varlen_attn_ring_kernel(VaArgs a) {
+  using R = VaRing<DQK, DV>;
+  constexpr int KT = R::KT;
+  constexpr int NS = DQK / 16;  // QK k-steps
+  constexpr int NDT = DV / 32;  // O^T dim tiles
+  constexpr int QROWS = 32 * kVaWaves;
+  constexpr int VROWS = 1024 / (2 * DV);  // V rows per DMA instruction
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int c = lane & 31, hf = lane >> 5;
+  int seq = blockIdx.y, h = blockIdx.z, bt = blockIdx.x;
+  if (a.pairs > 0) {
+    // consecutive workgroups go to the eight XCDs in turn: each XCD takes
+    // whole (sequence, head) pairs, one after another, so that the query
+    // tiles in flight on it stream the same K and V through its L2
+    const int r = blockIdx.x >> 3, pair = 8 * (r / a.n_qtiles) + (blockIdx.x & 7);
+    if (pair >= a.pairs) return;
+    bt = r % a.n_qtiles;
+    seq = pair / a.H;
+    h = pair % a.H;
+  }
+  const int qs = a.cu_q[seq], q_len = a.cu_q[seq + 1] - qs;
+  const int ks = a.cu_k[seq], k_len = a.cu_k[seq + 1] - ks;
+  // heaviest (latest) query tiles first under a causal mask
+  const int tile = a.causal ? a.n_qtiles - 1 - bt : bt;
+  const int q0 = tile * QROWS;
+  if (q0 >= q_len) return;
+  const int offset = a.causal ? k_len - q_len : 0;
+  const int kend = a.causal ? max(0, min(k_len, q0 + QROWS + offset)) : k_len;
+  const int n = (kend + KT - 1) / KT;
+
+  // ---- Q (B operand): row q0 + 32 w + c, dims 16 s + 8 hf .. +7; rows past
+  // q_len read row 0 of the sequence (their columns are not stored) ----
+  const int qi = q0 + 32 * w + c;
+  u32x4 qf[NS];
+  {
+    const uint16_t* qrow = a.q + (int64_t)(qs + (qi < q_len ? qi : 0)) * a.q_st +
+                           (int64_t)h * a.q_sh + 8 * hf;
+#pragma unroll
+    for (int s = 0; s < NS; s++) qf[s] = *reinterpret_cast<const u32x4*>(qrow + 16 * s);
+  }
+
+  // ---- this wave's share of a step's DMA: K rows 16 (w & 1) + lane / 4 of
+  // blocks NKD (w >> 1) .. , V rows VROWS (NVD w + u) + lane / (DV / 8) ----
+  const int kr = 16 * (w & 1) + (lane >> 2);
+  const int kb0 = R::NKD * (w >> 1);
+  const uint16_t* kp = a.k + (int64_t)(ks + kr) * a.k_st + (int64_t)h * a.k_sh + 32 * kb0 +
+                       8 * ((lane & 3) ^ ((lane >> 4) & 3));
+  const int vl = lane / (DV / 8), vr = VROWS * R::NVD * w + vl;
+  const int vsw = DV == 64 ? (vl >> 1) & 1 : vl & 3;
+  const uint16_t* vp = a.v + (int64_t)(ks + vr) * a.v_st + (int64_t)h * a.v_sh +
+                       8 * ((lane & (DV / 8 - 1)) ^ (4 * vsw));
+  unsigned char* const kdst = smem_raw + 2048 * kb0 + 1024 * (w & 1);
+  unsigned char* const vdst = smem_raw + R::KBYTES + 1024 * R::NVD * w;
+
+  auto issue = [&](int i) {
+    const int so = (i & (R::SLOTS - 1)) * R::SLOT;
+    const int k0 = i * KT;
+    const uint16_t* kq = kp + (int64_t)k0 * a.k_st;
+    const uint16_t* vq = vp + (int64_t)k0 * a.v_st;
+    if (k0 + KT <= kend) {
+#pragma unroll
+      for (int u = 0; u < R::NKD; u++) dma16(kq + 32 * u, kdst + so + 2048 * u);
+#pragma unroll
+      for (int u = 0; u < R::NVD; u++)
+        dma16(vq + (int64_t)(VROWS * u) * a.v_st, vdst + so + 1024 * u);
+    } else {  // rows past the last key read zeros
+      const bool kok = k0 + kr < kend;
+#pragma unroll
+      for (int u = 0; u < R::NKD; u++)
+        dma16(kok ? kq + 32 * u : kVaZero, kdst + so + 2048 * u);
+#pragma unroll
+      for (int u = 0; u < R::NVD; u++)
+        dma16(k0 + vr + VROWS * u < kend ? vq + (int64_t)(VROWS * u) * a.v_st : kVaZero,
+              vdst + so + 1024 * u);
+    }
+  };
+
+  // ---- LDS read offsets within a slot ----
+  const uint32_t lds0 = (uint32_t)(uintptr_t)smem_raw;
+  const uint32_t ka0 = 64 * c + 16 * (hf ^ ((c >> 2) & 3));  // QK steps 0, 2, ..; ka0 ^ 32: 1, 3, ..
+  const int ti = lane & 15, trow = 4 * hf + (ti >> 2);
+  const int tsw = DV == 64 ? (ti >> 3) & 1 : ti >> 2;
+  uint32_t va0[NDT];
+#pragma unroll
+  for (int t = 0; t < NDT; t++)
+    va0[t] = R::KBYTES + trow * (2 * DV) + 64 * (t ^ tsw) + 32 * ((lane >> 4) & 1) + 8 * (ti & 3);
+
+  // keys < jmax are visible to this lane's query; steps that end at or below
+  // jmin hold no masked key for any query of the wave
+  const int jmax = a.causal ? min(kend, qi + offset + 1) : kend;
+  const int jmin = a.causal ? min(kend, q0 + 32 * w + offset + 1) : kend;
+  const float lazy = kVaLazy / a.scale_log2;
+
+  f32x16 oacc[NDT], s;
+  float m_run, l_part;
+
+  auto qk = [&](int i) {
+    const uint32_t kb = lds0 + (i & (R::SLOTS - 1)) * R::SLOT + ka0;
+    f32x16 acc = {};
+#pragma unroll
+    for (int t = 0; t < NS; t++) {
+      const u32x4 kf = *(const __attribute__((address_space(3))) u32x4*)(
+          ((t & 1) ? (kb ^ 32u) : kb) + 2048u * (t >> 1));
+      acc = mma32x32<BF16>(kf, qf[t], acc);
+    }
+    return acc;
+  };
+
+  // the ring's first three steps
+  auto prologue = [&]() {
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+      if (i < n) issue(i);
+  };
+  auto max16 = [&](const f32x16& x) {
+    float m = fmaxf(x[0], x[1]);
+#pragma unroll
+    for (int e = 2; e < 16; e++) m = fmaxf(m, x[e]);
+    return xor32_max(m);
+  };
+  prologue();
+  // Q completes here, beside the first steps.  The compiler does not count
+  // the DMAs issued by inline asm, so a wait for Q left to the loop would
+  // drain the steps in flight.
+#pragma unroll
+  for (int t = 0; t < NS; t++) asm volatile("" : "+v"(qf[t]));
+
+  // NaN scores count as masked.  They show as a NaN row sum, and the tile is
+  // then run again with every score tested, so the usual pass tests none.
+  for (bool safe = false;; safe = true) {
+#pragma unroll
+    for (int t = 0; t < NDT; t++) oacc[t] = (f32x16){};
+    m_run = -1e30f;
+    l_part = 0.f;
+    va_wait<0>();
+    lds_barrier();
+    s = qk(0);
+    float mt = max16(s);
+    for (int i = 0; i < n; i++) {
+      if (i + 2 < n) va_wait<R::ND>();
+      else va_wait<0>();
+      lds_barrier();  // K(i + 1) and V(i) are in; nobody reads slot (i - 1) any more
+      if (i + 3 < n) issue(i + 3);
+
+      const int k0 = i * KT;
+      if (k0 + KT > jmin || safe) {
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+          const int j = k0 + 8 * (e >> 2) + 4 * hf + (e & 3);
+          if (j >= jmax || s[e] != s[e]) s[e] = -INFINITY;
+        }
+        mt = max16(s);
+      }
+      if (__any(mt > m_run + lazy)) {
+        const float m_new = fmaxf(m_run, mt);
+        const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2);
+        m_run = m_new;
+        l_part *= alpha;
+#pragma unroll
+        for (int t = 0; t < NDT; t++) oacc[t] *= alpha;
+      }
+
+      // S^T(i + 1) beside p(i), then O(i) beside the row sums and the maximum
+      // of S^T(i + 1).  Each group holds one MFMA (pair), the LDS read of a
+      // later one and a share of the VALU work; sched_barrier keeps the
+      // groups apart.  Past the last step QK multiplies a slot's old keys,
+      // and nothing reads the result.
+      f32x16 sn = {};
+      const float mb = m_run * a.scale_log2;
+      u32x4 pb[2], pl[2];
+      {
+        const uint32_t kb = lds0 + ((i + 1) & (R::SLOTS - 1)) * R::SLOT + ka0;
+        auto kread = [&](int t) {
+          return *(const __attribute__((address_space(3))) u32x4*)(
+              ((t & 1) ? (kb ^ 32u) : kb) + 2048u * (t >> 1));
+        };
+        u32x4 kf[kVaAhead + 1];
+#pragma unroll
+        for (int t = 0; t < kVaAhead; t++) kf[t] = kread(t);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < NS; t++) {
+          if (t + kVaAhead < NS) kf[(t + kVaAhead) % (kVaAhead + 1)] = kread(t + kVaAhead);
+          sn = mma32x32<BF16>(kf[t % (kVaAhead + 1)], qf[t], sn);
+#pragma unroll
+          for (int e = 16 * t / NS; e < 16 * (t + 1) / NS; e++) {
+            s[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e], a.scale_log2, -mb));
+            if (e & 1) {
+              const uint32_t hi = pack16<BF16>(s[e - 1], s[e]);
+              pb[e >> 3][(e >> 1) & 3] = hi;
+              if constexpr (BF16)
+                pl[e >> 3][(e >> 1) & 3] =
+                    pack16<true>(s[e - 1] - __uint_as_float(hi << 16),
+                                 s[e] - __uint_as_float(hi & 0xffff0000u));
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      {
+        const uint32_t vb = lds0 + (i & (R::SLOTS - 1)) * R::SLOT;
+        auto vread = [&](int u) {
+          const int t = u % NDT, t2 = u / NDT;
+          const s16x4v v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds_s16x4v*)(vb + va0[t] + 32 * DV * t2));
+          const s16x4v v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds_s16x4v*)(vb + va0[t] + 32 * DV * t2 + 16 * DV));
+          const u32x2 x0 = __builtin_bit_cast(u32x2, v0), x1 = __builtin_bit_cast(u32x2, v1);
+          return (u32x4){x0[0], x0[1], x1[0], x1[1]};
+        };
+        constexpr int NP = 2 * NDT;
+        u32x4 vf[3];
+        vf[0] = vread(0);
+        vf[1] = vread(1);
+        __builtin_amdgcn_sched_barrier(0);
+        float ls[4] = {s[0], s[1], s[2], s[3]};
+        mt = -1e30f;
+#pragma unroll
+        for (int u = 0; u < NP; u++) {
+          if (u + 2 < NP) vf[(u + 2) % 3] = vread(u + 2);
+          oacc[u % NDT] = mma32x32<BF16>(vf[u % 3], pb[u / NDT], oacc[u % NDT]);
+          if constexpr (BF16) oacc[u % NDT] = mma32x32<BF16>(vf[u % 3], pl[u / NDT], oacc[u % NDT]);
+          constexpr int H = NP / 2;
+#pragma unroll
+          for (int e = 4 + 12 * u / NP; e < 4 + 12 * (u + 1) / NP; e++) ls[e & 3] += s[e];
+          if (u >= H) {
+#pragma unroll
+            for (int e = 16 * (u - H) / H; e < 16 * (u - H + 1) / H; e++) mt = fmaxf(mt, sn[e]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        l_part += (ls[0] + ls[1]) + (ls[2] + ls[3]);
+        mt = xor32_max(mt);
+      }
+      s = sn;
+    }
+    if (safe) break;
+    volatile int* redo = reinterpret_cast<int*>(smem_raw);  // the ring is idle here
+    const int bad = __any(l_part != l_part);  // of all 64 lanes
+    lds_barrier();
+    if (lane == 0) redo[w] = bad;
+    lds_barrier();
+    if (!(redo[0] | redo[1] | redo[2] | redo[3])) break;
+    lds_barrier();
+    prologue();
+  }
+
+  // ---- outputs: lane c's query, dims 32 t + 8 u + 4 hf .. +3, turned into
+  // whole rows in the wave's part of the idle ring (16-byte piece j of row r
+  // at j ^ (r & 7)), so that every store writes full rows ----
+  float l = l_part;
+  l += __shfl_xor(l, 32, 64);
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  if (a.lse != nullptr && hf == 0 && qi < q_len)
+    a.lse[(int64_t)h * a.total_q + qs + qi] = l > 0.f ? m_run * a.scale + logf(l) : -INFINITY;
+  lds_barrier();
+  constexpr int NP16 = DV / 8;  // 16-byte pieces of an output row
+  unsigned char* const ow = smem_raw + w * (32 * 2 * DV);
+#pragma unroll
+  for (int t = 0; t < NDT; t++)
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const u32x2 pk = {pack16<BF16>(oacc[t][4 * u] * inv, oacc[t][4 * u + 1] * inv),
+                        pack16<BF16>(oacc[t][4 * u + 2] * inv, oacc[t][4 * u + 3] * inv)};
+      *reinterpret_cast<u32x2*>(ow + c * (2 * DV) + 16 * ((4 * t + u) ^ (c & 7)) + 8 * hf) = pk;
+    }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own rows
+#pragma unroll
+  for (int u = 0; u < NP16 / 2; u++) {
+    const int r = (64 / NP16) * u + lane / NP16, j = lane % NP16;
+    const u32x4 x = *reinterpret_cast<const u32x4*>(ow + r * (2 * DV) + 16 * (j ^ (r & 7)));
+    const int i = q0 + 32 * w + r;
+    if (i >= q_len) continue;
+    uint16_t* dst = a.o + (int64_t)(qs + i) * a.o_st + (int64_t)h * a.o_sh + 8 * j;
+    if (a.o16) {
+      *reinterpret_cast<u32x4*>(dst) = x;
+    } else {  // an output aligned to 8 bytes only
+      *reinterpret_cast<u32x2*>(dst) = (u32x2){x[0], x[1]};
+      *reinterpret_cast<u32x2*>(dst + 4) = (u32x2){x[2], x[3]};
+    }
+  }
+}
+
+template <bool BF16, int DQK, int DV>
+int launch_ring(const VaArgs& a0, int num_seqs, int max_q_len, hipStream_t st) {
+  using R = VaRing<DQK, DV>;
+  constexpr int QROWS = 32 * kVaWaves;
+  auto kern = varlen_attn_ring_kernel<BF16, DQK, DV>;
+  const int lds = R::SLOTS * R::SLOT;
+  const int rc = reserve_lds(reinterpret_cast<const void*>(kern), lds, "varlen_attention");
+  if (rc) return rc;
+  VaArgs a = a0;
+  a.n_qtiles = (max_q_len + QROWS - 1) / QROWS;
+  if (a.n_qtiles == 0) return MI355_DSA_OK;
+  // pair-major order where it leaves no XCD idle (a multiple of 8 pairs, or
+  // enough of them that the last round is small: at most one pair in nine
+  // runs beside idle XCDs) and a 1-D grid can hold it.  Causal 16k, 64 heads:
+  // 5.90 against 6.32 ms with consecutive workgroups on different heads.
+  const int64_t pairs = (int64_t)num_seqs * a.H, n1 = (pairs + 7) / 8 * 8 * a.n_qtiles;
+  const bool by_pair = (pairs % 8 == 0 || pairs >= 64) && n1 <= (1 << 23);
+  a.o16 = aligned_to(a.o, 16) && a.o_st % 8 == 0 && a.o_sh % 8 == 0;
+  a.pairs = by_pair ? (int)pairs : 0;
+  const dim3 grid = by_pair ? dim3((unsigned)n1) : dim3(a.n_qtiles, num_seqs, a.H);
+  kern<<<grid, kVaThreads, lds, st>>>(a);
+  return check_launch("varlen_attention");
+}
+
 template <bool BF16>
 int dispatch_va(const VaArgs& a, int d_qk, int d_v, int num_seqs, int max_q_len, hipStream_t st) {
-  // 32-key tiles and two workgroups per CU: two waves per SIMD, so one
-  // wave's softmax overlaps the other's MFMAs (1.7x the 64-key tile at one
-  // wave per SIMD on the (192, 128) causal prefill)
-  if (d_qk == 192 && d_v == 128) return launch_va<BF16, 192, 128, 2, 32, 2>(a, num_seqs, max_q_len, st);
-  if (d_qk == 128 && d_v == 128) return launch_va<BF16, 128, 128, 2, 32, 2>(a, num_seqs, max_q_len, st);
-  if (d_qk == 64 && d_v == 64) return launch_va<BF16, 64, 64, 2, 32, 2>(a, num_seqs, max_q_len, st);
+  // (256, 256): the ring kernel would hold 64 + 128 registers of Q and O per
+  // wave beside the scores, one wave per SIMD instead of two
+  if (d_qk == 192 && d_v == 128) return launch_ring<BF16, 192, 128>(a, num_seqs, max_q_len, st);
+  if (d_qk == 128 && d_v == 128) return launch_ring<BF16, 128, 128>(a, num_seqs, max_q_len, st);
+  if (d_qk == 64 && d_v == 64) return launch_ring<BF16, 64, 64>(a, num_seqs, max_q_len, st);
   if (d_qk == 256 && d_v == 256) return launch_va<BF16, 256, 256, 1, 32, 2>(a, num_seqs, max_q_len, st);
   return set_error(MI355_DSA_EINVAL,
                    "varlen_attention: head dims (%d, %d) not built; supported (qk, v): "

@@ -110,6 +110,61 @@ def test_equal_scores_closed_form(pkg, dev):
         torch.testing.assert_close(out[t], v[ks:ks + n].float().mean(0), rtol=2e-3, atol=1e-3)
 
 
+# (q_len, k_len) around the ring kernel's 32-key steps and 128-row tiles (and
+# its three-step prologue); H = 3 takes the plain grid order, H = 8 whole
+# (sequence, head) pairs per XCD
+EDGES = [(1, 1), (31, 33), (32, 32), (33, 31), (127, 95), (128, 96), (129, 97), (257, 129), (5, 161)]
+
+
+@pytest.mark.parametrize("H,dims", [(3, (192, 128)), (8, (128, 128)), (8, (64, 64))])
+@pytest.mark.parametrize("causal", [True, False])
+def test_ring_kernel_edges(pkg, dev, H, dims, causal):
+    """All edge lengths in one ragged batch; q scaled by 6 on half the rows, so
+    that the running maximum grows past the lazy rescale's threshold."""
+    cu_q = [sum(a for a, _ in EDGES[:i]) for i in range(len(EDGES) + 1)]
+    cu_k = [sum(b for _, b in EDGES[:i]) for i in range(len(EDGES) + 1)]
+    for dtype in (torch.float16, torch.bfloat16):
+        q, k, v = make(20 + H, cu_q, cu_k, H, *dims, dtype)
+        q[::2] *= 6
+        k *= torch.linspace(0.2, 1.5, cu_k[-1])[:, None, None].to(dtype)  # later keys score higher
+        scale = dims[0] ** -0.5
+        out, lse = run(pkg, dev, q, k, v, cu_q, cu_k, scale, causal)
+        ro, rl = O.varlen_attention(q, k, v, cu_q, cu_k, scale, causal)
+        check(out, lse, ro, rl, dtype)
+
+
+def test_nan_scores_are_masked(pkg, dev):
+    """A key with a NaN element is left out; a query with one sees no key."""
+    q, k, v = make(31, [0, 140], [0, 200], 8, 192, 128, torch.float16)
+    k[77, :, 5] = float("nan")
+    keep = [j for j in range(200) if j != 77]
+    ro, rl = O.varlen_attention(q, k[keep], v[keep], [0, 140], [0, 199], 0.07, False)
+    out, lse = run(pkg, dev, q, k, v, [0, 140], [0, 200], 0.07, False)
+    check(out, lse, ro, rl, torch.float16)
+    q[3, 2, 9] = float("nan")
+    out, lse = run(pkg, dev, q, k, v, [0, 140], [0, 200], 0.07, False)
+    assert torch.all(out[3, 2] == 0) and lse[2, 3] == -math.inf
+    ro[3, 2], rl[2, 3] = 0, -math.inf
+    check(out, lse, ro, rl, torch.float16)
+
+
+def test_output_aligned_to_8_bytes(pkg, dev):
+    """The C entry takes outputs aligned to 8 bytes only: the same values."""
+    q, k, v = (x.to(dev) for x in make(32, [0, 150], [0, 150], 8, 192, 128, torch.float16))
+    cu = torch.tensor([0, 150], dtype=torch.int32, device=dev)
+    want = pkg.mla_prefill.varlen_attention(q, k, v, cu, cu, 0.07, True, False)
+    buf = torch.zeros(150 * 8 * 128 + 4, dtype=torch.float16, device=dev)
+    out = buf[4:].view(150, 8, 128)
+    assert out.data_ptr() % 16 == 8
+    pkg._lib.call("mi355_dsa_varlen_attention", out.data_ptr(), None, q.data_ptr(), k.data_ptr(),
+                  v.data_ptr(), 0, 1, 8, 192, 128, q.stride(0), q.stride(1), k.stride(0),
+                  k.stride(1), v.stride(0), v.stride(1), out.stride(0), out.stride(1),
+                  cu.data_ptr(), cu.data_ptr(), 150, 150, 0.07, 1,
+                  torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and torch.all(buf[:4] == 0)
+
+
 F32_RTOL, F32_ATOL, F32_LSE = 2e-5, 2e-5, 2e-5
 
 
