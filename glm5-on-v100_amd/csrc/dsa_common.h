@@ -213,6 +213,12 @@ __device__ __forceinline__ float xor32_sum(float v) {
                                                   false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
+// max of v and v of lane ^ 32, the same way
+__device__ __forceinline__ float xor32_max(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                                  false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
 // max(d, 0) of an MFMA result in one instruction: such a value is never a
 // signalling NaN, so the quieting max the compiler puts before fmaxf is not
 // needed (a NaN gives 0, as d > 0 ? d : 0 does).

@@ -48,8 +48,10 @@
 //    every gathered 32-key tile; consecutive tokens map to the same XCD so
 //    their overlapping top-k sets hit in L2.
 #include <float.h>
+#include <stddef.h>
 
 #include <mutex>
+#include <utility>
 
 #include "capi_internal.h"
 #include "dsa_common.h"
@@ -207,10 +209,12 @@ __device__ __forceinline__ void resolve_bt(const MlaParams& p, int b, int seq_le
 // p.zero_unresolved is set -- it reads as a zero row and stays in the
 // softmax with score 0, as the reference's dense kernel (sm70_mla_decode.cu:
 // 762-771) and split-decode kernel (:970-992, :1047-1053) do.
+// Returns the key count up to this thread's last unmasked key (0: none).
 template <int NT>
-__device__ __forceinline__ void resolve_store(const MlaParams& p, int n, int base, int seq_len,
-                                              const int pos[kResU], const int pg[kResU],
-                                              const int blk[kResU], int32_t* rows) {
+__device__ __forceinline__ int resolve_store(const MlaParams& p, int n, int base, int seq_len,
+                                             const int pos[kResU], const int pg[kResU],
+                                             const int blk[kResU], int32_t* rows) {
+  int last = 0;
 #pragma unroll
   for (int u = 0; u < kResU; u++) {
     const int j = base + u * NT + (int)threadIdx.x;
@@ -219,8 +223,24 @@ __device__ __forceinline__ void resolve_store(const MlaParams& p, int n, int bas
       const bool bad = blk[u] < 0 || row >= p.n_kv_rows;
       const bool in_range = pos[u] >= 0 && pos[u] < seq_len && pg[u] < p.max_blocks;
       rows[j] = bad ? ((p.zero_unresolved && in_range) ? -2 : -1) : (int32_t)row;
+      if (!bad || (p.zero_unresolved && in_range)) last = j + 1;
     }
   }
+  return last;
+}
+
+// Token of workgroup bid of n.  Consecutive workgroups run on the eight XCDs in
+// turn; runs of 32 consecutive tokens, one per CU, share an XCD and its L2
+// (neighbouring tokens' lists overlap).  The runs go round the XCDs from the
+// last token down: the lists of a prompt's first top-k tokens are short, and
+// long ones then neither pile up on a few XCDs nor start last (3333 tokens of
+// three prompts, lists of up to 1667 keys, 64 heads, fp16 rows: 912 -> 750 us
+// against one eighth of the tokens per XCD).  The last n % 256 workgroups,
+// which take the first tokens, go one by one.
+__device__ __forceinline__ int token_of(int bid, int n) {
+  const int full = n & ~255;
+  const int x = bid < full ? (bid & ~255) + 32 * (bid & 7) + ((bid & 255) >> 3) : bid;
+  return n - 1 - x;
 }
 
 template <bool KVFP8, int HW, int KW, int NB>
@@ -614,7 +634,7 @@ __device__ __forceinline__ int dpt_at(int c, int key) {  // key % 4 == 0
 constexpr int kDimsPerWave = kValueDim / kDmaWaves;                      // 64
 constexpr int kTilesPerWave = kDimsPerWave / 16;                         // 4
 
-__device__ __align__(16) const uint8_t kZeroRow[kDsmlaRowBytes] = {};
+__device__ __align__(16) const uint8_t kZeroRow[kLatentDim * 2] = {};  // either row format
 
 struct DmaSmem {
   uint8_t rows[kDmaWaves][kDecWaveBytes];  // raw rows: wave w's keys 16w .. 16w+15
@@ -1002,6 +1022,7 @@ struct WsSmem {
   f32x4 lsum[16];
   int rescale[2];
   int tmask[kSegKeys / kPfTileKeys];  // tile of the segment holds a masked key (row -1)
+  int last[kWsWaves];                 // keys of the segment up to each wave's last unmasked one
 };
 static_assert(sizeof(WsSmem) <= 160 * 1024, "one workgroup per CU");
 
@@ -1055,10 +1076,7 @@ struct WsCtx {
 
 __device__ __forceinline__ WsCtx ws_ctx(const MlaParams& p) {
   WsCtx x;
-  const int nx = gridDim.x, bid = blockIdx.x;
-  const int xcd = bid & 7, j = bid >> 3;
-  const int per = nx >> 3, rem = nx & 7;
-  x.b = xcd * per + (xcd < rem ? xcd : rem) + j;  // consecutive tokens share an XCD
+  x.b = token_of(blockIdx.x, gridDim.x);
   x.hbase = blockIdx.y * 64;
   x.split = blockIdx.z;
   x.seq_len = p.seq_lens[x.b];
@@ -1069,11 +1087,29 @@ __device__ __forceinline__ WsCtx ws_ctx(const MlaParams& p) {
   return x;
 }
 
+// Tiles of a segment up to its last unmasked key (at least one), from the key counts up to
+// each wave's last unmasked key (every wave computes the same).  The tiles
+// past it hold masked keys only (the -1 padding of a list longer than its
+// token's context) and would change no result: they are not gathered or
+// multiplied.  Prompts shorter than top-k, 64 heads, fp16 rows, 3333 tokens with
+// lists a third full on average: 1535 -> 1214 us by this alone, before token_of
+// spread the long lists.
+template <int NW>
+__device__ __forceinline__ int used_tiles(const int (&last)[NW]) {
+  int n = 1;
+#pragma unroll
+  for (int w = 0; w < NW; w++) n = max(n, last[w]);
+  return __builtin_amdgcn_readfirstlane((n + kPfTileKeys - 1) / kPfTileKeys);
+}
+
 // idx -> block table -> row of the segment's keys, by all 768 threads, then
-// a barrier.  The caller's previous barrier ended every use of rows and ring.
-__device__ __forceinline__ void ws_resolve(const MlaParams& p, const WsCtx& x, int seg_lo,
-                                           int nkeys, int ntiles, int32_t* rows) {
-  for (int base = 0; base < ntiles * kPfTileKeys; base += kWsThreads * kResU) {
+// a barrier; returns the tiles to run (used_tiles).  The caller's previous
+// barrier ended every use of rows, last and ring.
+__device__ __forceinline__ int ws_resolve(const MlaParams& p, const WsCtx& x, int seg_lo,
+                                          int nkeys, WsSmem& sh) {
+  const int n = (nkeys + kPfTileKeys - 1) / kPfTileKeys * kPfTileKeys;
+  int last = 0;
+  for (int base = 0; base < n; base += kWsThreads * kResU) {
     int pos[kResU], pg[kResU], blk[kResU];
 #pragma unroll
     for (int u = 0; u < kResU; u++) {
@@ -1084,15 +1120,20 @@ __device__ __forceinline__ void ws_resolve(const MlaParams& p, const WsCtx& x, i
 #pragma unroll
     for (int u = 0; u < kResU; u++) {
       const int j = base + u * kWsThreads + (int)threadIdx.x;
-      if (j < ntiles * kPfTileKeys) {
+      if (j < n) {
         const int64_t row = (int64_t)blk[u] * p.page_size + (pos[u] - pg[u] * p.page_size);
         const bool in_range = pos[u] >= 0 && pos[u] < x.seq_len && pg[u] < p.max_blocks;
-        rows[j] = (blk[u] < 0 || row >= p.n_kv_rows)
-                      ? ((in_range && p.zero_unresolved) ? -2 : -1) : (int32_t)row;
+        const int code = (blk[u] < 0 || row >= p.n_kv_rows)
+                             ? ((in_range && p.zero_unresolved) ? -2 : -1) : (int32_t)row;
+        sh.rows[j] = code;
+        if (code != -1) last = j + 1;
       }
     }
   }
+  last = wave_max_i32(last);
+  if ((threadIdx.x & 63) == 0) sh.last[threadIdx.x >> 6] = last;
   lds_barrier();
+  return used_tiles(sh.last);
 }
 
 // ---- QK waves ----
@@ -1149,8 +1190,7 @@ __device__ __forceinline__ void ws_qk_role(const MlaParams& p, const WsCtx& x, W
   };
   for (int seg_lo = x.k_lo; seg_lo < x.k_hi; seg_lo += kSegKeys) {
     const int nkeys = min(x.k_hi - seg_lo, kSegKeys);
-    const int ntiles = (nkeys + kPfTileKeys - 1) / kPfTileKeys;
-    ws_resolve(p, x, seg_lo, nkeys, ntiles, sh.rows);
+    const int ntiles = ws_resolve(p, x, seg_lo, nkeys, sh);
     lds_barrier();  // tile 0 landed
     for (int s = -1; s < ntiles; s++) {
       f32x4 v[2][4];
@@ -1216,8 +1256,7 @@ __device__ __forceinline__ void ws_pv_role(const MlaParams& p, const WsCtx& x, W
   };
   for (int seg_lo = x.k_lo; seg_lo < x.k_hi; seg_lo += kSegKeys) {
     const int nkeys = min(x.k_hi - seg_lo, kSegKeys);
-    const int ntiles = (nkeys + kPfTileKeys - 1) / kPfTileKeys;
-    ws_resolve(p, x, seg_lo, nkeys, ntiles, sh.rows);
+    const int ntiles = ws_resolve(p, x, seg_lo, nkeys, sh);
     ws_dma_nope(kv, sh.rows, sh.ring[0], pw, lane);
     if (ntiles > 1) ws_dma_nope(kv, sh.rows + kPfTileKeys, sh.ring[1], pw, lane);
     ws_wait_pv(ntiles > 1);
@@ -1366,8 +1405,7 @@ __device__ __forceinline__ void ws_sm_role(const MlaParams& p, const WsCtx& x, W
   };
   for (int seg_lo = x.k_lo; seg_lo < x.k_hi; seg_lo += kSegKeys) {
     const int nkeys = min(x.k_hi - seg_lo, kSegKeys);
-    const int ntiles = (nkeys + kPfTileKeys - 1) / kPfTileKeys;
-    ws_resolve(p, x, seg_lo, nkeys, ntiles, sh.rows);
+    const int ntiles = ws_resolve(p, x, seg_lo, nkeys, sh);
     {  // which tiles hold a masked key: thread ts checks rows 8 ts .. +7 (tile ts / 4)
       const bool in = 8 * ts < ntiles * kPfTileKeys;
       int m = 0;
@@ -1714,6 +1752,439 @@ __global__ void __launch_bounds__(kPfThreads) mla_attn_f16_kernel(MlaParams p) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// 64-head attention with whole-head waves: the prefill configuration, batches
+// split over keys, and dense decode (idx == nullptr: positions [0, seq_len)).
+//
+// Workgroup = (token, 64 heads, key split), 4 waves, one per SIMD (512
+// registers each).  Wave (hw, kw) owns heads [32 hw, +32) and every second
+// 32-key tile (tiles 2 r + kw), end to end: its Q (32 heads x 576 dims) and
+// its O^T (512 dims x 32 heads, fp32) stay in registers, so scores and P never
+// leave the wave and no barrier separates QK, softmax and PV.
+//   * S^T = K Q^T, v_mfma_f32_32x32x16: 32 keys x 32 heads, keys from LDS;
+//   * softmax per head: lane (head c, half) holds 16 of its 32 scores, so the
+//     maximum is one lane swap; lazy running max (kPfLazyMax);
+//   * O^T += V^T P^T: the S^T accumulator layout (keys 8 a + 4 half + r) is
+//     P^T's operand layout; V^T comes from transpose LDS reads in that order.
+// A round is one tile of each key group; its tiles arrive by LDS-DMA one round
+// ahead, behind one barrier per round.  At the end the two key groups merge O
+// through LDS, each finishing half of the dims.
+//
+// Tile layout: 64-byte blocks, block-major (block b of key r at 2048 b + 64 r),
+// 16-byte piece p of a block at p ^ ((r >> 2) & 3).  A QK read (one piece of 32
+// keys per half-wave) and a transpose read (a block of 4 keys per half-wave)
+// then cover the 64 banks without conflicts, and every DMA instruction fetches
+// a block of 16 keys: four adjacent lanes read 64 contiguous bytes.  (With one
+// 16-byte piece of 64 scattered rows' halves per instruction the address unit
+// takes a cycle per lane, and the gather alone bounded the kernel: 1830 us for
+// 4096 tokens of 64 heads against 1460 us.)
+//
+// Bound: LDS bandwidth (a round's four waves read 278 KB and receive 74 KB,
+// ~2800 cycles at 128 B/clk) and the softmax between QK and PV; waits for tiles
+// and barriers are under 3 % (stamps: QK 1650, softmax 720, PV 1290 cycles of a
+// 3940-cycle round, 2176 of MFMA).  4096 tokens at 64k, 64 heads: 1904 us with
+// mla_attn_f16_kernel -> 1335-1460 us (800-875 TFLOP/s); 3000-token prompt
+// 1373 -> 750 us.  Measured level: two S accumulators, LDS reads five ahead, one
+// wait per four MFMAs.  fp8_ds_mla rows in this form took 1635 us against 1638
+// us of the wave-role kernel above: a wave alone on its SIMD issues one VALU
+// instruction in 8 cycles, and the e4m3 conversions of 32 heads per wave fill
+// them; splits were slower (31.7 against 26.5 us at 16 tokens).
+// ---------------------------------------------------------------------------
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int kHwWaves = 4;
+constexpr int kHwThreads = 64 * kHwWaves;
+constexpr int kHwChunks = kLatentDim / 8;                        // 72 per fp16 row
+constexpr int kHwBlocks = kHwChunks / 4;                         // 64-byte blocks per row
+constexpr int kHwSlotBytes = kHwBlocks * kPfTileKeys * 64;       // 36864
+constexpr int kHwAhead = 3;                                      // LDS reads ahead of their MFMA
+
+// O^T of a wave: 16 tiles of 16 registers, tile t in a[16 t : 16 t + 15].  All
+// 256 accumulation registers are named here and kept from the compiler, which
+// needs the other 256 for Q, scores, P and the operands in flight: left to it,
+// O moved between the two files every round and Q spilled.  It never
+// allocates an accumulation register itself in a kernel that does not exceed
+// 256 VGPRs (hw_own_agprs, once a round, lists them all as overwritten).
+#define HW_AGPRS \
+  "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", \
+  "a14", "a15", "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", \
+  "a27", "a28", "a29", "a30", "a31", "a32", "a33", "a34", "a35", "a36", "a37", "a38", "a39", \
+  "a40", "a41", "a42", "a43", "a44", "a45", "a46", "a47", "a48", "a49", "a50", "a51", "a52", \
+  "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63", "a64", "a65", \
+  "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", \
+  "a79", "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", \
+  "a92", "a93", "a94", "a95", "a96", "a97", "a98", "a99", "a100", "a101", "a102", "a103", \
+  "a104", "a105", "a106", "a107", "a108", "a109", "a110", "a111", "a112", "a113", "a114", \
+  "a115", "a116", "a117", "a118", "a119", "a120", "a121", "a122", "a123", "a124", "a125", \
+  "a126", "a127", "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", \
+  "a137", "a138", "a139", "a140", "a141", "a142", "a143", "a144", "a145", "a146", "a147", \
+  "a148", "a149", "a150", "a151", "a152", "a153", "a154", "a155", "a156", "a157", "a158", \
+  "a159", "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", \
+  "a170", "a171", "a172", "a173", "a174", "a175", "a176", "a177", "a178", "a179", "a180", \
+  "a181", "a182", "a183", "a184", "a185", "a186", "a187", "a188", "a189", "a190", "a191", \
+  "a192", "a193", "a194", "a195", "a196", "a197", "a198", "a199", "a200", "a201", "a202", \
+  "a203", "a204", "a205", "a206", "a207", "a208", "a209", "a210", "a211", "a212", "a213", \
+  "a214", "a215", "a216", "a217", "a218", "a219", "a220", "a221", "a222", "a223", "a224", \
+  "a225", "a226", "a227", "a228", "a229", "a230", "a231", "a232", "a233", "a234", "a235", \
+  "a236", "a237", "a238", "a239", "a240", "a241", "a242", "a243", "a244", "a245", "a246", \
+  "a247", "a248", "a249", "a250", "a251", "a252", "a253", "a254", "a255"
+__device__ __forceinline__ void hw_own_agprs() { asm volatile("" ::: HW_AGPRS); }
+template <class F, int... I>
+__device__ __forceinline__ void unroll_seq(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+// f(0), f(1), .. f(N - 1), the index a compile-time constant
+template <int N, class F>
+__device__ __forceinline__ void unroll(F&& f) {
+  unroll_seq(f, std::make_integer_sequence<int, N>{});
+}
+template <int T>
+__device__ __forceinline__ void hw_mma(f16x8 a, f16x8 b) {
+  asm volatile("v_mfma_f32_32x32x16_f16 a[%0:%1], %2, %3, a[%0:%1]" ::"n"(16 * T),
+               "n"(16 * T + 15), "v"(a), "v"(b));
+}
+// S accumulators stay out of the accumulation registers the same way; the
+// first step starts from 0
+__device__ __forceinline__ void hw_qk0(f32x16& s, f16x8 a, f16x8 b) {
+  asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=&v"(s) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void hw_qk(f32x16& s, f16x8 a, f16x8 b) {
+  asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(s) : "v"(a), "v"(b));
+}
+template <int I>
+__device__ __forceinline__ void hw_zero() {
+  asm volatile("v_accvgpr_write_b32 a[%0], 0" ::"n"(I));
+}
+template <int I>
+__device__ __forceinline__ float hw_read() {
+  float v;
+  asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(v) : "n"(I));
+  return v;
+}
+template <int I>
+__device__ __forceinline__ void hw_scale(float f) {
+  float t0, t1, t2, t3;
+  asm volatile(
+      "v_accvgpr_read_b32 %0, a[%5]\n\tv_accvgpr_read_b32 %1, a[%6]\n\t"
+      "v_accvgpr_read_b32 %2, a[%7]\n\tv_accvgpr_read_b32 %3, a[%8]\n\t"
+      "v_mul_f32 %0, %0, %4\n\tv_mul_f32 %1, %1, %4\n\t"
+      "v_mul_f32 %2, %2, %4\n\tv_mul_f32 %3, %3, %4\n\t"
+      "v_accvgpr_write_b32 a[%5], %0\n\tv_accvgpr_write_b32 a[%6], %1\n\t"
+      "v_accvgpr_write_b32 a[%7], %2\n\tv_accvgpr_write_b32 a[%8], %3"
+      : "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
+      : "v"(f), "n"(I), "n"(I + 1), "n"(I + 2), "n"(I + 3));
+}
+// MFMA results of the last tiles are readable, VALU writes reach the next MFMA
+__device__ __forceinline__ void hw_settle() { asm volatile("s_nop 15\n\ts_nop 7"); }
+
+struct HwSmem {
+  uint8_t ring[2][2][kHwSlotBytes];   // [key group][round parity]; with rows: O exchange at the end
+  int32_t rows[kSegKeys];
+  float m[2][64], l[2][64];           // [key group][head]
+  int tmask[kSegKeys / kPfTileKeys];  // tile of the segment holds a masked key (row -1)
+  int last[kHwWaves];
+};
+static_assert(sizeof(HwSmem) <= 160 * 1024, "one workgroup per CU");
+static_assert(offsetof(HwSmem, m) >= kHwWaves * 8 * 64 * 64, "the O exchange ends below m and l");
+
+// DMA instruction I of a tile: block I of 16 keys (lane l: key l / 4, 64
+// contiguous bytes per 4 lanes)
+template <int I>
+__device__ __forceinline__ void hw_dma1(const uint8_t* src, uint8_t* slot, int hw) {
+  dma16_at<64 * I>(src, slot + 2048 * I + 1024 * hw);
+}
+typedef __attribute__((address_space(3))) f16x8 lds_f16x8;
+
+// S^T of a tile of fp16 rows: step t covers dims 16 t + 8 hf .. +7
+__device__ __forceinline__ void hw_qk_f16(f32x16& s, const f16x8 (&qf)[36], uint32_t slot,
+                                          uint32_t ka0, const uint8_t* src, uint8_t* dst, int hw) {
+  const uint32_t kb = slot + ka0;
+  auto kread = [&](int t) {
+    return *(const lds_f16x8*)(((t & 1) ? (kb ^ 32u) : kb) + 2048u * (t >> 1));
+  };
+  constexpr int NS = 36;
+  f16x8 kf[kHwAhead + 1];
+#pragma unroll
+  for (int t = 0; t < kHwAhead; t++) kf[t] = kread(t);
+  __builtin_amdgcn_sched_barrier(0);
+  unroll<NS>([&](auto tc) {
+    constexpr int t = tc;
+    if constexpr (t + kHwAhead < NS) kf[(t + kHwAhead) % (kHwAhead + 1)] = kread(t + kHwAhead);
+    if constexpr (t == 0) hw_qk0(s, kf[0], qf[0]);
+    else hw_qk(s, kf[t % (kHwAhead + 1)], qf[t]);
+    if constexpr (t % 2 == 0) hw_dma1<t / 2>(src, dst, hw);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+}
+
+// O^T += V^T P^T of a tile of fp16 rows, p = 2^(s log2 e - ml); returns this
+// lane's sum of p.  The second half of P is computed beside the first's MFMAs.
+__device__ __forceinline__ float hw_pv_f16(const f32x16& s, float ml, uint32_t slot, uint32_t va0) {
+  constexpr float kLog2e = 1.4426950408889634f;
+  const uint32_t vb0 = slot + va0, vb1 = (vb0 + 512u) ^ 32u;
+  auto vread = [&](int u) {
+    const int t = u % 16, t2 = u / 16;
+    const s16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (lds_s16x4*)(vb0 + 2048u * t + 1024u * t2));
+    const s16x4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (lds_s16x4*)(vb1 + 2048u * t + 1024u * t2));
+    const f16x4 x0 = __builtin_bit_cast(f16x4, x), x1 = __builtin_bit_cast(f16x4, y);
+    return (f16x8){x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+  };
+  f16x8 vf[kHwAhead + 1], pb[2];
+#pragma unroll
+  for (int u = 0; u < kHwAhead; u++) vf[u] = vread(u);
+  __builtin_amdgcn_sched_barrier(0);
+  float ls = 0.f;
+  auto pexp = [&](int e) {
+    const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e], kLog2e, -ml));
+    ls += x;
+    pb[e >> 3][e & 7] = (f16)x;
+  };
+#pragma unroll
+  for (int e = 0; e < 8; e++) pexp(e);
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_nop 1");  // P is written
+  unroll<32>([&](auto uc) {
+    constexpr int u = uc;
+    if constexpr (u + kHwAhead < 32) vf[(u + kHwAhead) % (kHwAhead + 1)] = vread(u + kHwAhead);
+    hw_mma<u % 16>(vf[u % (kHwAhead + 1)], pb[u / 16]);
+    if constexpr (u < 8) pexp(8 + u);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+  return ls;
+}
+
+__global__ void __launch_bounds__(kHwThreads, 1) mla_hw_f16_kernel(MlaParams p) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  HwSmem& sh = *reinterpret_cast<HwSmem*>(smem_raw);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hw = w & 1, kw = w >> 1;
+  const int c = lane & 31, hf = lane >> 5;
+  const int b = token_of(blockIdx.x, gridDim.x);
+  const int hbase = blockIdx.y * 64;
+  const int split = blockIdx.z;
+  const uint8_t* kv = reinterpret_cast<const uint8_t*>(p.kv);
+  const int seq_len = p.seq_lens[b];
+  constexpr float kLog2e = 1.4426950408889634f;
+
+  const int n_keys = p.idx ? p.topk : max(0, min(p.topk, seq_len));
+  const int kps = ((n_keys + p.n_splits - 1) / p.n_splits + kPfTileKeys - 1) / kPfTileKeys *
+                  kPfTileKeys;
+  const int k_lo = min(split * kps, n_keys);
+  const int k_hi = min(k_lo + kps, n_keys);
+
+  // the first segment's idx entries load beside Q
+  int pos[kResU];
+  resolve_idx<kHwThreads>(p, b, k_lo, min(k_hi - k_lo, kSegKeys), 0, pos);
+
+  // ---- Q (B operand): head c, dims 16 s + 8 hf .. +7 of step s;
+  // scaled in fp16 once the first tile is on its way ----
+  f16x8 qf[kLatentDim / 16];
+  {
+    const int h = hbase + 32 * hw + c;
+    const f16* qrow = p.q + ((int64_t)b * p.n_head + (h < p.n_head ? h : 0)) * kLatentDim;
+#pragma unroll
+    for (int s = 0; s < kLatentDim / 16; s++)
+      qf[s] = *reinterpret_cast<const f16x8*>(qrow + 16 * s + 8 * hf);
+  }
+
+  // O^T tile t: dims 32 t + 8 a + 4 hf + r (element 4 a + r), head c
+  hw_own_agprs();
+  unroll<256>([&](auto i) { hw_zero<i>(); });
+  float m_run = -1e30f, l_part = 0.f;  // l: this lane's keys only
+
+  // LDS addresses within a slot
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(&sh.ring[kw][0][0]);
+  const uint32_t ka0 = 64 * c + 16 * (hf ^ ((c >> 2) & 3));  // QK steps 0, 2, ..; ^ 32: 1, 3, ..
+  // transpose reads: keys 4 hf + ti / 4 (+ 8, + 16 t2), dims 32 t + 16 td + 4 (ti % 4) .. +3
+  const int ti = lane & 15, td = (lane >> 4) & 1;
+  const uint32_t va0 =
+      64 * (4 * hf + (ti >> 2)) + 16 * ((2 * td + ((ti >> 1) & 1)) ^ hf) + 8 * (ti & 1);
+  const int drow = 16 * hw + (lane >> 2);  // the key whose blocks this lane fetches
+
+  // this lane's source in a tile (zeros for a masked key, and past the end)
+  auto source = [&](int tile, int n) {
+    const int row = tile < n ? sh.rows[tile * kPfTileKeys + drow] : -1;
+    return (row >= 0 ? kv + (int64_t)row * (kLatentDim * 2) : kZeroRow) +
+           16 * ((lane & 3) ^ ((lane >> 4) & 3));
+  };
+  // rows and flags of the segment at seg_lo (its idx entries in pos), the first
+  // tiles on their way; returns the tiles to run
+  auto start_segment = [&](int seg_lo) {
+    const int nkeys = min(k_hi - seg_lo, kSegKeys);
+    const int n_res = (nkeys + kPfTileKeys - 1) / kPfTileKeys * kPfTileKeys;
+    int pg[kResU], blk[kResU];
+    resolve_bt<kHwThreads>(p, b, seq_len, pos, pg, blk);
+    int last = resolve_store<kHwThreads>(p, n_res, 0, seq_len, pos, pg, blk, sh.rows);
+    last = wave_max_i32(last);
+    if (lane == 0) sh.last[w] = last;
+    lds_barrier();
+    const int n = used_tiles(sh.last);
+    const uint8_t* src = source(kw, n);
+    unroll<kHwBlocks>([&](auto i) { hw_dma1<i>(src, sh.ring[kw][0], hw); });
+    {  // which tiles hold a masked key: thread t checks rows 8 t .. +7 (tile t / 4)
+      const int t8 = 8 * (int)threadIdx.x;
+      int mk = 0;
+      if (t8 < n_res) {
+        const int4 x = *reinterpret_cast<const int4*>(sh.rows + t8);
+        const int4 y = *reinterpret_cast<const int4*>(sh.rows + t8 + 4);
+        mk = (x.x == -1) | (x.y == -1) | (x.z == -1) | (x.w == -1) | (y.x == -1) | (y.y == -1) |
+             (y.z == -1) | (y.w == -1);
+      }
+      const unsigned long long bal = __ballot(mk);
+      if ((threadIdx.x & 3) == 0) sh.tmask[threadIdx.x >> 2] = ((bal >> (lane & ~3)) & 0xfull) != 0;
+    }
+    return n;
+  };
+  int ntiles = k_lo < k_hi ? start_segment(k_lo) : 0;
+  {
+    const f16 sc = (f16)p.scale_h;
+    const f16x8 sc8 = {sc, sc, sc, sc, sc, sc, sc, sc};
+#pragma unroll
+    for (int s = 0; s < kLatentDim / 16; s++) qf[s] *= sc8;
+    // every load that the compiler counts has landed: a wait that it placed
+    // later would drain the tiles in flight
+    __builtin_amdgcn_s_waitcnt(0x0f70);
+  }
+  for (int seg_lo = k_lo; seg_lo < k_hi; seg_lo += kSegKeys) {
+    for (int t0 = 0; t0 < ntiles; t0 += 2) {
+      const int tile = t0 + kw, par = (t0 >> 1) & 1;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_barrier();  // this round's tiles are in; the other parity's slots are free
+      if (tile < ntiles) {
+        const uint32_t slot = lds0 + par * kHwSlotBytes;
+        const int masked = sh.tmask[tile];
+
+        // ---- S^T, beside the next round's DMA ----
+        f32x16 s;
+        hw_qk_f16(s, qf, slot, ka0, source(tile + 2, ntiles), sh.ring[kw][1 - par], hw);
+        hw_settle();
+        asm volatile("" : "+v"(s));  // no use of S above the wait
+
+        // ---- softmax ----
+        if (masked) {  // wave-uniform; row code -2 is a zero row, a valid key
+#pragma unroll
+          for (int a = 0; a < 4; a++) {
+            const int4 rc =
+                *reinterpret_cast<const int4*>(sh.rows + tile * kPfTileKeys + 8 * a + 4 * hf);
+            if (rc.x == -1) s[4 * a + 0] = -INFINITY;
+            if (rc.y == -1) s[4 * a + 1] = -INFINITY;
+            if (rc.z == -1) s[4 * a + 2] = -INFINITY;
+            if (rc.w == -1) s[4 * a + 3] = -INFINITY;
+          }
+        }
+        float mt = fmaxf(s[0], s[1]);
+#pragma unroll
+        for (int e = 2; e < 16; e++) mt = fmaxf(mt, s[e]);
+        mt = xor32_max(mt);
+        if (__any(mt > m_run + kPfLazyMax)) {
+          const float m_new = mt > m_run + kPfLazyMax ? mt : m_run;
+          const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * kLog2e);
+          m_run = m_new;
+          l_part *= alpha;
+          hw_settle();
+          unroll<64>([&](auto i) { hw_scale<4 * i>(alpha); });
+        }
+        // ---- O^T += V^T P^T ----
+        l_part += hw_pv_f16(s, m_run * kLog2e, slot, va0);
+        hw_own_agprs();
+      }
+    }
+    if (seg_lo + kSegKeys < k_hi) {
+      resolve_idx<kHwThreads>(p, b, seg_lo + kSegKeys, min(k_hi - seg_lo - kSegKeys, kSegKeys), 0, pos);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last round's DMA past the end too
+      lds_barrier();  // rows, flags and the ring are free
+      ntiles = start_segment(seg_lo + kSegKeys);
+      __builtin_amdgcn_s_waitcnt(0x0f70);
+    }
+  }
+
+  // ---- merge the key groups: wave (hw, kw) finishes dims [256 kw, +256) of
+  // its heads and hands the other half to wave (hw, 1 - kw) ----
+  const float l_own = l_part + __shfl_xor(l_part, 32, 64);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  lds_barrier();  // the ring is idle
+  if (hf == 0) {
+    sh.m[kw][32 * hw + c] = m_run;
+    sh.l[kw][32 * hw + c] = l_own;
+  }
+  f32x4* const xout = reinterpret_cast<f32x4*>(smem_raw) + (2 * (1 - kw) + hw) * 2048 + lane;
+  f32x4* const xin = reinterpret_cast<f32x4*>(smem_raw) + (2 * kw + hw) * 2048 + lane;
+  hw_settle();
+  auto hand_over = [&](auto hc) {  // tiles 8 hc .. +7
+    unroll<32>([&](auto uc) {
+      constexpr int i = 128 * decltype(hc)::value + 4 * decltype(uc)::value;
+      xout[64 * uc] = (f32x4){hw_read<i>(), hw_read<i + 1>(), hw_read<i + 2>(), hw_read<i + 3>()};
+    });
+  };
+  if (kw == 0) hand_over(std::integral_constant<int, 1>{});
+  else hand_over(std::integral_constant<int, 0>{});
+  lds_barrier();
+  const float m2 = sh.m[1 - kw][32 * hw + c], l2 = sh.l[1 - kw][32 * hw + c];
+  const float M = fmaxf(m_run, m2);
+  // the sum in the order of the key groups, so that both waves get the same l
+  const float w_own = __expf(m_run - M), w_oth = __expf(m2 - M);
+  const float L = kw == 0 ? l_own * w_own + l2 * w_oth : l2 * w_oth + l_own * w_own;
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const float f_own = w_own * inv, f_oth = w_oth * inv;
+  const int h = hbase + 32 * hw + c;
+  const int64_t bh = (int64_t)b * p.n_head + h;
+  const bool final_out = p.n_splits == 1;
+  const int64_t ps = bh * p.n_splits + split;
+  auto finish = [&](auto tc) {  // tiles t and t + 1, one 64-dim chunk
+    constexpr int t = decltype(tc)::value;
+    u32x2 q2[2][4];  // dims 32 (t + tt) + 8 a + 4 hf .. +3
+    unroll<8>([&](auto ec) {
+      constexpr int tt = ec / 4, a = ec % 4, i = 16 * (t + tt) + 4 * a;
+      const f32x4 x = xin[64 * (4 * ((t + tt) & 7) + a)];
+      const f32x4 own = {hw_read<i>(), hw_read<i + 1>(), hw_read<i + 2>(), hw_read<i + 3>()};
+      f16x4 v;
+#pragma unroll
+      for (int r = 0; r < 4; r++) v[r] = (f16)(own[r] * f_own + x[r] * f_oth);
+      q2[tt][a] = __builtin_bit_cast(u32x2, v);
+    });
+    if (final_out) {
+      // lane halves swap quads: half 0 gets dims 16 v + 0..7, half 1 16 v + 8..15
+#pragma unroll
+      for (int tt = 0; tt < 2; tt++)
+#pragma unroll
+        for (int v = 0; v < 2; v++) {
+          const auto d0 = __builtin_amdgcn_permlane32_swap(q2[tt][2 * v][0], q2[tt][2 * v + 1][0],
+                                                           false, false);
+          const auto d1 = __builtin_amdgcn_permlane32_swap(q2[tt][2 * v][1], q2[tt][2 * v + 1][1],
+                                                           false, false);
+          if (h < p.n_head) {
+            u32x2* dst = reinterpret_cast<u32x2*>(p.o + bh * kValueDim + 32 * (t + tt) + 16 * v +
+                                                  8 * hf);
+            dst[0] = (u32x2){d0[0], d1[0]};
+            dst[1] = (u32x2){d0[1], d1[1]};
+          }
+        }
+    } else if (h < p.n_head) {
+      // the split merge's partial layout: 64-dim chunk t / 2, dim 16 t' + 4 g + r
+      // at 16 g + 4 t' + r, with g = 2 (a & 1) + hf, t' = 2 tt + a / 2
+#pragma unroll
+      for (int a1 = 0; a1 < 2; a1++) {
+        u32x4* dst = reinterpret_cast<u32x4*>(p.part_o + ps * kValueDim + 32 * t +
+                                              16 * (2 * a1 + hf));
+        dst[0] = (u32x4){q2[0][a1][0], q2[0][a1][1], q2[0][2 + a1][0], q2[0][2 + a1][1]};
+        dst[1] = (u32x4){q2[1][a1][0], q2[1][a1][1], q2[1][2 + a1][0], q2[1][2 + a1][1]};
+      }
+    }
+  };
+  if (kw == 0) unroll<4>([&](auto i) { finish(std::integral_constant<int, 2 * i>{}); });
+  else unroll<4>([&](auto i) { finish(std::integral_constant<int, 8 + 2 * i>{}); });
+  if (kw == 0 && hf == 0 && h < p.n_head) {
+    if (final_out) {
+      p.lse[bh] = (L > 0.f) ? (M + logf(L)) : p.empty_lse;
+    } else {
+      p.part_ml[ps * 2 + 0] = M;
+      p.part_ml[ps * 2 + 1] = L;
+    }
+  }
+}
+
 // Flash-decode merge of S partial states (reference :1138-1184):
 // m = max_s m_s, w_s = l_s > 0 ? exp(m_s - m) l_s : 0, o = sum w_s o_s / sum w_s
 // (o_s is the split's own normalised output, stored in fp16).
@@ -1967,7 +2438,21 @@ static int dense_splits(int B, int n_head, int max_kv) {
   return s;
 }
 
+// fp16 rows over 64 heads: whole-head waves where a workgroup has 16 tiles or
+// more of its split's list (or context), mla_attn_f16_kernel below that, where
+// the larger prologue and the final merge of O weigh more (us per call at 64
+// heads, mla_attn_f16_kernel / whole-head waves: 4 tiles, 16 tokens, 27.8 / 29.9;
+// dense 4 x 4k 24.8 / 26.2; 16 tiles, 64 tokens, 58.0 / 57.5; dense 4 x 32k ragged
+// 47.9 / 45.5; 64 tiles, 200 tokens, 134.3 / 116.6).
+constexpr int kHwMinTiles = 16;
 static int launch_attn_f16(const MlaParams& prm, dim3 grid, hipStream_t st) {
+  if ((prm.topk + prm.n_splits - 1) / prm.n_splits > (kHwMinTiles - 1) * kPfTileKeys) {
+    const int rc = reserve_lds(reinterpret_cast<const void*>(mla_hw_f16_kernel), sizeof(HwSmem),
+                               "mla_hw_f16");
+    if (rc) return rc;
+    mla_hw_f16_kernel<<<grid, kHwThreads, sizeof(HwSmem), st>>>(prm);
+    return check_launch("mla_hw_f16");
+  }
   const int rc = reserve_lds(reinterpret_cast<const void*>(mla_attn_f16_kernel), sizeof(HfSmem),
                              "mla_attn_f16");
   if (rc) return rc;

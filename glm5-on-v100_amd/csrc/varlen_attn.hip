@@ -387,13 +387,6 @@ __device__ __forceinline__ uint32_t pack16(float x, float y) {
   }
 }
 
-// max of a lane's value and the lane's ^ 32, in both
-__device__ __forceinline__ float xor32_max(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                  false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
 template <int DQK, int DV>
 struct VaRing {
   static constexpr int KT = 32;              // keys per step

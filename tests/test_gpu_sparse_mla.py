@@ -193,6 +193,29 @@ def test_prefill_config_segments_partial_heads(ops, dev, fp8):
     check(o, lse, ro, rl)
 
 
+# slots [lo, hi) of a list that hold keys, the rest -1: around the 32-key
+# tiles, the kernels' 1024- and 2048-key segments, leading gaps, none at all
+VALID_SLOTS = [(0, 0), (0, 1), (0, 32), (0, 33), (31, 32), (63, 65), (0, 1023), (0, 1025),
+               (1024, 1056), (1500, 2048), (2047, 2049), (2048, 2080), (2079, 2112), (0, 2112),
+               (1000, 1001), (2111, 2112)]
+
+
+@pytest.mark.parametrize("fp8", [True, False], ids=["fp8", "fp16"])
+@pytest.mark.parametrize("H", [64, 16])
+def test_lists_with_unused_tiles(ops, dev, fp8, H):
+    """Tiles past a list's last key are not run: every position of the last
+    key around a tile or segment edge, and keys behind leading gaps."""
+    B, topk = 256, 2112
+    q, kv, idx, bt, seq = make(60 + H, B, H, 60, 64, fp8, topk, [3000] * B, shared_bt=True)
+    slot = torch.arange(topk)
+    for b in range(B):
+        lo, hi = VALID_SLOTS[b % len(VALID_SLOTS)]
+        idx[b, (slot < lo) | (slot >= hi)] = -1
+    o, lse = run(ops, dev, q, kv, idx, bt, seq)
+    ro, rl = O.sparse_mla(q, kv, idx, bt, seq, SCALE)
+    check(o, lse, ro, rl)
+
+
 PIPE_SPLIT = [
     # seed, B, H, fp8, topk, seqs: batches of 8..255 tokens at > 32 heads run the
     # 64-head pipelined kernels with round(256 / (B * ceil(H / 64))) key splits
