@@ -213,7 +213,12 @@ __device__ __forceinline__ float xor32_sum(float v) {
                                                   false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
-// max of v and v of lane ^ 32, the same way
+// max of v and v of lane ^ 16, and of lane ^ 32, the same way
+__device__ __forceinline__ float xor16_max(float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                                  false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
 __device__ __forceinline__ float xor32_max(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
                                                   false);

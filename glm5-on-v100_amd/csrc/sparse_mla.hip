@@ -19,7 +19,7 @@
 // S^T's accumulator layout (lane c = head, rows 4g..4g+3 = keys) is the
 // B-operand layout of the PV step, so P never leaves registers and the
 // softmax reductions over keys are two lane shuffles.  V^T operands come
-// straight from the row-major key tile with ds_read_b64_tr_b16 (in a 16-lane
+// straight from the key tile with transpose LDS reads (ds_read_b64_tr_b16: in a 16-lane
 // group, lane j element k = lane (4k + j/4)'s element j%4), one LDS
 // instruction per MFMA operand.  O^T lives in 32 accumulator tiles.
 //
@@ -32,21 +32,12 @@
 // e4m3*scale to fp16 before the dot (dsmla_load4 + half store), which the
 // tolerance of the parity tests covers.
 //
-// Memory pipeline: every workgroup first resolves idx -> block table ->
-// cache row for all its keys in one batched pass (rows kept in LDS), then
-// streams key tiles with the global loads of tile t+1 held in registers
-// while tile t is computed.
-//
-// Launch configurations of one kernel template:
-//  * decode (HW=1, KW=4, NB=1): workgroup = (split, 16-head group, token);
-//    its 4 waves take interleaved 16-key tiles of the split's range, each in
-//    its own LDS tile, and are merged in LDS; splits write unnormalised
-//    partials combined by sparse_mla_merge_kernel (flash-decode reduction,
-//    :1138-1184).  Workgroups of one (token, split) differ by a multiple of 8
-//    in launch order, so they share an XCD and its L2 for the gathered rows.
-//  * prefill (HW=4, KW=1, NB=2): workgroup = token x 64 heads; 4 waves share
-//    every gathered 32-key tile; consecutive tokens map to the same XCD so
-//    their overlapping top-k sets hit in L2.
+// Kernels, picked by plan_decode: sparse_mla_decode_dma_kernel (fp8 split decode
+// of small batches), sparse_mla_prefill_fp8_ws_kernel (fp8, 64 heads per
+// workgroup), mla_hw_f16_kernel and mla_attn_f16_kernel (fp16, 64 heads, sparse
+// and dense), sparse_mla_few_kernel (16 heads per workgroup: few heads, and small
+// fp16 batches).  Splits write partials combined by sparse_mla_merge_kernel
+// (flash-decode reduction, :1138-1184).
 #include <float.h>
 #include <stddef.h>
 
@@ -58,8 +49,6 @@
 
 namespace mi355dsa {
 
-constexpr int kPitch = kLatentDim + 8;   // LDS row pitch (halves) of Q / key tiles
-constexpr int kOTiles = kValueDim / 16;  // 32 O^T accumulator tiles
 constexpr int kSegKeys = 2048;           // keys resolved per segment
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -90,81 +79,6 @@ struct MlaParams {
   int xcd_map;  // decode workgroup order (grid a multiple of 8): 0 plain; 1 a (token,
                 // split)'s head groups share an XCD
 };
-
-template <int HW, int KW, int NB>
-struct MlaSmem {
-  static constexpr int TN = 16 * NB;  // keys per tile per key-wave group
-  struct Main {
-    f16 q[HW * 16 * kPitch];
-    f16 k[KW * TN * kPitch];
-    float sc[KW * TN * 4];  // fp8 tile scales of the tile's rows
-  };
-  // key-wave merge: wave w owns dims [128w, 128w+128) (8 O^T tiles) and
-  // receives the other waves' tiles of that quarter: [quarter][source][tile][lane]
-  static constexpr int XSRC = KW > 1 ? KW - 1 : 1;
-  union {
-    Main main;
-    f32x4 xbuf[KW > 1 ? KW : 1][XSRC][kOTiles / (KW > 1 ? KW : 1)][64];
-  } u;
-  int32_t rows[kSegKeys];
-  float m[KW * 16];
-  float l[KW * 16];
-};
-
-// Per-thread register stage of one tile's global loads.  Chunks of invalid
-// rows are loaded from row 0 and zeroed only when stored to LDS (bit u of
-// `bad`), so issuing the loads never waits for them.
-template <bool KVFP8, int TN, int GT>
-struct TileStage {
-  static constexpr int NCH = KVFP8 ? 41 : kLatentDim / 8;  // 16-B chunks per row
-  static constexpr int PER = (TN * NCH + GT - 1) / GT;
-  u32x4 v[PER];
-  uint32_t bad;
-};
-
-// Writes the staged chunks into the LDS key tile (and fp8 scales).
-template <bool KVFP8, int TN, int GT>
-__device__ __forceinline__ void tile_store(const TileStage<KVFP8, TN, GT>& st, f16* ktile,
-                                           float* sc, int t0) {
-  constexpr int NCH = TileStage<KVFP8, TN, GT>::NCH;
-  constexpr int PER = TileStage<KVFP8, TN, GT>::PER;
-#pragma unroll
-  for (int u = 0; u < PER; u++) {
-    const int i = t0 + u * GT;
-    if (i >= TN * NCH) continue;
-    const int r = i / NCH, ch = i - r * NCH;
-    f16* d = ktile + r * kPitch;
-    const u32x4 val = ((st.bad >> u) & 1u) ? (u32x4){0u, 0u, 0u, 0u} : st.v[u];
-    if constexpr (KVFP8) {
-      if (ch < 32) {
-        // 16 e4m3 bytes -> 16 exact fp16 values (dims 16ch .. 16ch+15)
-        u32x4 h0, h1;
-#pragma unroll
-        for (int w = 0; w < 4; w++) {
-          const f16x2 lo = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)val[w], 1.0f, false);
-          const f16x2 hi = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)val[w], 1.0f, true);
-          const uint32_t a = __builtin_bit_cast(uint32_t, lo);
-          const uint32_t b = __builtin_bit_cast(uint32_t, hi);
-          if (w < 2) {
-            h0[2 * w] = a;
-            h0[2 * w + 1] = b;
-          } else {
-            h1[2 * (w - 2)] = a;
-            h1[2 * (w - 2) + 1] = b;
-          }
-        }
-        *reinterpret_cast<u32x4*>(d + 16 * ch) = h0;
-        *reinterpret_cast<u32x4*>(d + 16 * ch + 8) = h1;
-      } else if (ch == 32) {
-        *reinterpret_cast<u32x4*>(sc + 4 * r) = val;  // 4 fp32 tile scales
-      } else {
-        *reinterpret_cast<u32x4*>(d + 512 + 8 * (ch - 33)) = val;  // RoPE fp16
-      }
-    } else {
-      *reinterpret_cast<u32x4*>(d + 8 * ch) = val;
-    }
-  }
-}
 
 // Resolves idx -> block table -> cache row for keys [j0, j0+n) of token b
 // into rows[0..n).  Work is done in batches of NT*8 keys; each batch issues
@@ -243,347 +157,6 @@ __device__ __forceinline__ int token_of(int bid, int n) {
   return n - 1 - x;
 }
 
-template <bool KVFP8, int HW, int KW, int NB>
-__global__ void __launch_bounds__(HW * KW * 64) sparse_mla_kernel(MlaParams p) {
-  using Smem = MlaSmem<HW, KW, NB>;
-  constexpr int TN = Smem::TN;
-  constexpr int NT = HW * KW * 64;
-  constexpr int GT = HW * 64;  // gather team = the HW waves of a key-wave group
-  constexpr int NACC = KVFP8 ? 5 : 1;  // QK accumulators: 4 scale tiles + RoPE
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  Smem& sh = *reinterpret_cast<Smem*>(smem_raw);
-
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int hw = wave % HW, kw = wave / HW;
-  const int c = lane & 15, g = lane >> 4;
-
-  // ---- work item ----
-  int b, h0, split;
-  if constexpr (KW == 1) {
-    // prefill: XCD-aware token order (consecutive tokens share an XCD)
-    const int nx = gridDim.x, bid = blockIdx.x;
-    const int xcd = bid & 7, j = bid >> 3;
-    const int per = nx >> 3, rem = nx & 7;
-    b = xcd * per + (xcd < rem ? xcd : rem) + j;
-    h0 = blockIdx.y * (16 * HW);
-    split = 0;
-  } else {
-    split = blockIdx.x;
-    h0 = blockIdx.y * (16 * HW);
-    b = blockIdx.z;
-  }
-  const int seq_len = p.seq_lens[b];
-
-  // ---- this workgroup's key range (tiles of TN) ----
-  // Dense mode (idx == nullptr) attends to positions [0, seq_len): the
-  // token's own length is split, not the table's width.
-  const int n_keys = p.idx ? p.topk : max(0, min(p.topk, seq_len));
-  const int n_tiles_all = (n_keys + TN - 1) / TN;
-  const int tps = (n_tiles_all + p.n_splits - 1) / p.n_splits;  // tiles per split
-  const int tile_lo = split * tps;
-  const int tile_hi = min(tile_lo + tps, n_tiles_all);
-  constexpr int SEG_TILES = kSegKeys / TN;
-
-  // first index batch in flight while Q is staged
-  int pos0[kResU];
-  const int nkeys0 = tile_lo < tile_hi ? min(min(tile_lo + SEG_TILES, tile_hi) * TN, n_keys) - tile_lo * TN : 0;
-  resolve_idx<NT>(p, b, tile_lo * TN, nkeys0, 0, pos0);
-
-  // ---- scaled Q of this workgroup's heads into LDS; the block-table loads
-  // of the first index batch are issued between the Q loads and the Q
-  // stores so both latencies overlap ----
-  int pg0[kResU], blk0[kResU];
-  {
-    constexpr int QCH = HW * 16 * (kLatentDim / 8);
-    constexpr int QPER = (QCH + NT - 1) / NT;
-    const f16* qb = p.q + ((int64_t)b * p.n_head) * kLatentDim;
-    f16x8 raw[QPER];
-#pragma unroll
-    for (int u = 0; u < QPER; u++) {
-      const int i = threadIdx.x + u * NT;
-      const int hh = i / (kLatentDim / 8), ch = i - hh * (kLatentDim / 8);
-      raw[u] = (f16x8){0, 0, 0, 0, 0, 0, 0, 0};
-      if (i < QCH && h0 + hh < p.n_head)
-        raw[u] = *reinterpret_cast<const f16x8*>(qb + (int64_t)(h0 + hh) * kLatentDim + 8 * ch);
-    }
-    resolve_bt<NT>(p, b, seq_len, pos0, pg0, blk0);
-#pragma unroll
-    for (int u = 0; u < QPER; u++) {
-      const int i = threadIdx.x + u * NT;
-      if (i < QCH) {
-        const int hh = i / (kLatentDim / 8), ch = i - hh * (kLatentDim / 8);
-        f16x8 v;
-#pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = (f16)((float)raw[u][e] * p.scale_h);
-        *reinterpret_cast<f16x8*>(&sh.u.main.q[hh * kPitch + 8 * ch]) = v;
-      }
-    }
-  }
-
-  f32x4 oacc[kOTiles];
-#pragma unroll
-  for (int t = 0; t < kOTiles; t++) oacc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  float m_run = -1e30f, l_run = 0.f;
-
-  f16* ktile = &sh.u.main.k[kw * TN * kPitch];
-  float* ksc = &sh.u.main.sc[kw * TN * 4];
-  const int gt = threadIdx.x - kw * GT;  // thread index inside the gather team
-  const f16* qrow = &sh.u.main.q[(16 * hw + c) * kPitch + 8 * g];
-
-  for (int seg_lo = tile_lo; seg_lo < tile_hi; seg_lo += SEG_TILES) {
-    const int seg_hi = min(seg_lo + SEG_TILES, tile_hi);
-    const int j0 = seg_lo * TN;
-    const int nkeys = min(seg_hi * TN, n_keys) - j0;
-    __syncthreads();  // previous segment done with sh.rows
-    for (int base = 0; base < nkeys; base += NT * kResU) {
-      if (seg_lo == tile_lo && base == 0) {
-        resolve_store<NT>(p, nkeys, base, seq_len, pos0, pg0, blk0, sh.rows);
-      } else {
-        int pos[kResU], pg[kResU], blk[kResU];
-        resolve_idx<NT>(p, b, j0, nkeys, base, pos);
-        resolve_bt<NT>(p, b, seq_len, pos, pg, blk);
-        resolve_store<NT>(p, nkeys, base, seq_len, pos, pg, blk, sh.rows);
-      }
-    }
-    __syncthreads();
-    const int rounds = (seg_hi - seg_lo + KW - 1) / KW;
-    // The tile of round rd for this key-wave group is seg_lo + rd*KW + kw;
-    // its rows start at sh.rows[(rd*KW + kw) * TN].  Keys past the segment
-    // (or past nkeys) read as row -1.
-    auto tile_valid = [&](int rd) { return seg_lo + rd * KW + kw < seg_hi; };
-    TileStage<KVFP8, TN, GT> stage;
-    auto row_of = [&](int rd, int r) -> int {
-      const int kidx = (rd * KW + kw) * TN + r;
-      const int v = sh.rows[kidx < nkeys ? kidx : 0];  // unconditional LDS read
-      return (tile_valid(rd) && kidx < nkeys) ? v : -1;
-    };
-    // global loads of round rd's tile into the register stage
-    auto issue = [&](int rd) {
-      constexpr int NCH = TileStage<KVFP8, TN, GT>::NCH;
-      constexpr int PER = TileStage<KVFP8, TN, GT>::PER;
-      constexpr int RB = KVFP8 ? kDsmlaRowBytes : kLatentDim * 2;
-      int rowu[PER];
-#pragma unroll
-      for (int u = 0; u < PER; u++) {
-        const int i = gt + u * GT;
-        const int r = i / NCH;
-        rowu[u] = (i < TN * NCH && p.n_kv_rows > 0) ? row_of(rd, r < TN ? r : 0) : -1;
-      }
-      // Every lane loads (row 0 stands in for an invalid row, so no branch
-      // guards the load) and invalid rows are zeroed afterwards: masked keys
-      // then carry finite zeros whatever the cache holds in unused pages.
-      if (p.n_kv_rows > 0) {  // uniform: an empty cache is never read
-#pragma unroll
-        for (int u = 0; u < PER; u++) {
-          const int i = gt + u * GT;
-          const int ch = i - (i / NCH) * NCH;
-          const int row = rowu[u] >= 0 ? rowu[u] : 0;
-          stage.v[u] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(p.kv) +
-                                                      (int64_t)row * RB + 16 * ch);
-        }
-      }
-      stage.bad = 0u;
-#pragma unroll
-      for (int u = 0; u < PER; u++) stage.bad |= (rowu[u] < 0 ? 1u : 0u) << u;
-    };
-    issue(0);
-    for (int rd = 0; rd < rounds; rd++) {
-      tile_store<KVFP8, TN, GT>(stage, ktile, ksc, gt);
-      // validity of this tile's keys (before the rows array can change)
-      bool valid[NB][4];
-#pragma unroll
-      for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) valid[nb][r] = row_of(rd, 16 * nb + 4 * g + r) != -1;
-      if (rd + 1 < rounds) issue(rd + 1);
-      __syncthreads();
-
-      // ---- S^T blocks ----
-      f32x4 sacc[NB];
-      float mt = -INFINITY;
-#pragma unroll
-      for (int nb = 0; nb < NB; nb++) {
-        f32x4 acc[NACC];
-#pragma unroll
-        for (int a = 0; a < NACC; a++) acc[a] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        const f16* krow = ktile + (16 * nb + c) * kPitch + 8 * g;
-#pragma unroll
-        for (int s = 0; s < kLatentDim / 32; s++) {
-          const int a = KVFP8 ? (s < 16 ? s / 4 : 4) : 0;
-          acc[a] = mfma16x16x32(*reinterpret_cast<const f16x8*>(krow + 32 * s),
-                                *reinterpret_cast<const f16x8*>(qrow + 32 * s), acc[a]);
-        }
-        f32x4 sv;
-        if constexpr (KVFP8) {
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const f32x4 s4 = *reinterpret_cast<const f32x4*>(&ksc[4 * (16 * nb + 4 * g + r)]);
-            sv[r] = acc[4][r] + s4[0] * acc[0][r] + s4[1] * acc[1][r] + s4[2] * acc[2][r] +
-                    s4[3] * acc[3][r];
-          }
-        } else {
-          sv = acc[0];
-        }
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          sv[r] = valid[nb][r] ? sv[r] : -INFINITY;
-          mt = fmaxf(mt, sv[r]);
-        }
-        sacc[nb] = sv;
-      }
-      mt = fmaxf(mt, shfl_xor_f(mt, 16));
-      mt = fmaxf(mt, shfl_xor_f(mt, 32));
-      const float m_new = fmaxf(m_run, mt);
-      const float alpha = expf(m_run - m_new);
-      float ls = 0.f;
-      float pr[NB][4];
-#pragma unroll
-      for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          pr[nb][r] = valid[nb][r] ? expf(sacc[nb][r] - m_new) : 0.f;
-          ls += pr[nb][r];
-        }
-      ls += shfl_xor_f(ls, 16);
-      ls += shfl_xor_f(ls, 32);
-      l_run = l_run * alpha + ls;
-      m_run = m_new;
-      if (__any(alpha != 1.0f)) {
-#pragma unroll
-        for (int t = 0; t < kOTiles; t++)
-#pragma unroll
-          for (int r = 0; r < 4; r++) oacc[t][r] *= alpha;
-      }
-
-      // ---- O^T += V^T P^T ----
-      // P^T operands, one per fp8 scale tile (dims 128*st .. 128*st+127)
-      constexpr int NST = KVFP8 ? 4 : 1;
-      f16x4 pb[NST][NB];
-#pragma unroll
-      for (int st = 0; st < NST; st++)
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            float v = pr[nb][r];
-            if constexpr (KVFP8) v *= ksc[4 * (16 * nb + 4 * g + r) + st];
-            pb[st][nb][r] = (f16)v;
-          }
-      // transpose-read source: lane i of its 16-lane group supplies row
-      // (4g + i/4) (+16 per block), dims 16t + 4(i%4) .. +3
-      const f16* vsrc = ktile + (4 * g + (c >> 2)) * kPitch + 4 * (c & 3);
-#pragma unroll
-      for (int t = 0; t < kOTiles; t++) {
-        const int st = KVFP8 ? t / 8 : 0;
-        if constexpr (NB == 1) {
-          const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (lds_s16x4*)(vsrc + 16 * t));
-          oacc[t] = mfma16x16x16(__builtin_bit_cast(f16x4, a), pb[st][0], oacc[t]);
-        } else {
-          const s16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (lds_s16x4*)(vsrc + 16 * t));
-          const s16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (lds_s16x4*)(vsrc + 16 * kPitch + 16 * t));
-          const f16x4 x0 = __builtin_bit_cast(f16x4, a0), x1 = __builtin_bit_cast(f16x4, a1);
-          const f16x8 av = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
-          const f16x8 bv = {pb[st][0][0], pb[st][0][1], pb[st][0][2], pb[st][0][3],
-                            pb[st][1][0], pb[st][1][1], pb[st][1][2], pb[st][1][3]};
-          oacc[t] = mfma16x16x32(av, bv, oacc[t]);
-        }
-      }
-      __syncthreads();
-    }
-  }
-
-  // ---- finalize ----
-  if constexpr (KW == 1) {
-    const int h = h0 + 16 * hw + c;
-    if (h < p.n_head) {
-      if (g == 0)
-        p.lse[(int64_t)b * p.n_head + h] = (l_run > 0.f) ? (m_run + logf(l_run)) : p.empty_lse;
-      const float inv = (l_run > 0.f) ? 1.f / l_run : 0.f;
-      f16* orow = p.o + ((int64_t)b * p.n_head + h) * kValueDim;
-#pragma unroll
-      for (int t = 0; t < kOTiles; t++) {
-        f16x4 v;
-#pragma unroll
-        for (int r = 0; r < 4; r++) v[r] = (f16)(oacc[t][r] * inv);
-        *reinterpret_cast<f16x4*>(orow + 16 * t + 4 * g) = v;
-      }
-    }
-  } else {
-    // Merge the KW key-waves (HW == 1: all waves hold the same 16 heads).
-    // Wave w owns O^T tiles [8w, 8w+8) (dims 128w .. 128w+127): every wave
-    // scales its accumulators by exp(m_w - M), writes the tiles of the other
-    // quarters to LDS, then adds the three received copies of its own
-    // quarter and stores it straight from registers.
-    constexpr int QT = kOTiles / KW;  // tiles per quarter
-    __syncthreads();
-    if (g == 0) {
-      sh.m[kw * 16 + c] = m_run;
-      sh.l[kw * 16 + c] = l_run;
-    }
-    __syncthreads();
-    float M = -1e30f;
-#pragma unroll
-    for (int k2 = 0; k2 < KW; k2++) M = fmaxf(M, sh.m[k2 * 16 + c]);
-    float L = 0.f;
-#pragma unroll
-    for (int k2 = 0; k2 < KW; k2++) {
-      const float lk = sh.l[k2 * 16 + c];
-      L += (lk > 0.f) ? lk * expf(sh.m[k2 * 16 + c] - M) : 0.f;
-    }
-    const float wgt = (l_run > 0.f) ? expf(m_run - M) : 0.f;
-#pragma unroll
-    for (int t = 0; t < kOTiles; t++) {
-      const int qd = t / QT;
-      if (qd != kw) {
-        const int slot = kw < qd ? kw : kw - 1;
-        sh.u.xbuf[qd][slot][t % QT][lane] = oacc[t] * wgt;
-      }
-    }
-    __syncthreads();
-    const bool final_out = (p.n_splits == 1);
-    const int h = h0 + c;
-    const int64_t bh = (int64_t)b * p.n_head + h;
-    const float inv = (L > 0.f) ? 1.f / L : 0.f;
-#pragma unroll
-    for (int t = 0; t < kOTiles; t++) {
-      if (t / QT == kw) {
-        f32x4 v = oacc[t] * wgt;
-#pragma unroll
-        for (int sl = 0; sl < KW - 1; sl++) v += sh.u.xbuf[kw][sl][t % QT][lane];
-        if (h < p.n_head) {
-          if (final_out) {
-            f16x4 o4;
-#pragma unroll
-            for (int r = 0; r < 4; r++) o4[r] = (f16)(v[r] * inv);
-            *reinterpret_cast<f16x4*>(p.o + bh * kValueDim + 16 * t + 4 * g) = o4;
-          } else {
-            // split partial stored normalised (|o_s| <= max|V|) in fp16
-            const int64_t ps = bh * p.n_splits + split;
-            f16x4 o4;
-#pragma unroll
-            for (int r = 0; r < 4; r++) o4[r] = (f16)(v[r] * inv);
-            *reinterpret_cast<f16x4*>(p.part_o + ps * kValueDim + 64 * (t / 4) + 16 * g +
-                                      4 * (t % 4)) = o4;
-          }
-        }
-      }
-    }
-    if (kw == 0 && g == 0 && h < p.n_head) {
-      if (final_out) {
-        p.lse[bh] = (L > 0.f) ? (M + logf(L)) : p.empty_lse;
-      } else {
-        const int64_t ps = bh * p.n_splits + split;
-        p.part_ml[ps * 2 + 0] = M;
-        p.part_ml[ps * 2 + 1] = L;
-      }
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
 // fp8_ds_mla split decode with LDS-DMA gathers.
 //
@@ -655,6 +228,12 @@ __device__ __forceinline__ int load_dword_async(const int32_t* ptr) {
   int v;
   asm volatile("global_load_dword %0, %1, off" : "=v"(v) : "v"(ptr) : "memory");
   return v;
+}
+
+// 8 e4m3 bytes -> 8 exact fp16 values
+__device__ __forceinline__ f16x8 e4m3x8(uint32_t d0, uint32_t d1) {
+  const f16x4 a = e4m3x4_to_f16x4(d0), b = e4m3x4_to_f16x4(d1);
+  return (f16x8){a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
 }
 
 // QK of one wave's 16 keys of raw fp8_ds_mla rows at cb: returns the scores
@@ -2185,6 +1764,320 @@ __global__ void __launch_bounds__(kHwThreads, 1) mla_hw_f16_kernel(MlaParams p) 
   }
 }
 
+// ---------------------------------------------------------------------------
+// Few heads (at most 32: a tensor-parallel rank's share), prefill and batches:
+// the 64-head kernels would multiply 32-56 empty heads.
+//
+// Workgroup = (token, 16 heads, key split), 4 waves; two (fp16 rows) or three
+// (fp8_ds_mla) workgroups share a CU, so that one's gather and barriers run
+// beside another's arithmetic.  Per 64-key tile:
+//   * wave w gathers keys [16 w, +16) into its own LDS region (LDS-DMA) and
+//     computes their scores for the 16 heads (Q resident in registers) as soon
+//     as its own rows have landed; P = exp(s - m_w) with the wave's own tile
+//     maximum goes to LDS in fp32, and m_w beside it; one barrier;
+//   * wave w adds V^T P^T of the 64 keys to O^T of value dims [128 w, +128)
+//     (one fp8 scale tile): P times the source wave's exp(m_w - m) and the key's
+//     scale, rounded to fp16 once; a barrier frees the tile.
+// The running max m is lazy (kPfLazyMax) and the same in every wave.
+// Region layout: 64-byte blocks, block-major (block b of key r at 1024 b + 64 r),
+// piece p of a block at p ^ few_sw(r): the QK reads (16 keys x 4 pieces) and the
+// transpose reads are free of bank conflicts, and a DMA instruction fetches a
+// block of 16 keys, 64 contiguous bytes per four lanes.  fp8 scales follow,
+// tile-major (tile t of key r at 64 t + 4 r).
+// ---------------------------------------------------------------------------
+constexpr int kFewThreads = 256;
+constexpr int kFewTile = 64;     // keys per tile
+constexpr int kFewSeg = 512;     // keys resolved per segment
+constexpr int kFewMinTokens = 64;  // fp8, at most 16 heads: shorter batches take the split decode
+
+template <bool FP8>
+struct FewSmem {
+  static constexpr int BLOCKS = FP8 ? 10 : 18;
+  static constexpr int REGION = 1024 * BLOCKS + (FP8 ? 256 : 0);
+  uint8_t rows[4][REGION];
+  float pt[16 * kFewTile];  // P[head][key], 4-key chunk (key / 4) ^ head
+  int32_t code[kFewSeg];    // cache rows of the segment's keys
+  float m[4][16];           // the waves' tile maxima
+  float l[4][16];
+  int last[4];
+};
+
+__device__ __forceinline__ int few_sw(int r) { return (4 - (r >> 2)) & 3; }
+__device__ __forceinline__ int few_pt(int c, int key) {  // key % 4 == 0
+  return c * kFewTile + ((((key >> 2) ^ c) & 15) << 2);
+}
+
+template <bool FP8>
+__global__ void __launch_bounds__(kFewThreads, FP8 ? 3 : 2) sparse_mla_few_kernel(MlaParams p) {
+  using Sm = FewSmem<FP8>;
+  constexpr int ROW = FP8 ? kDsmlaRowBytes : kLatentDim * 2;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  Sm& sh = *reinterpret_cast<Sm*>(smem_raw);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int b = token_of(blockIdx.x, gridDim.x);
+  const int h0 = blockIdx.y * 16, split = blockIdx.z;
+  const uint8_t* kv = reinterpret_cast<const uint8_t*>(p.kv);
+  const int seq_len = p.seq_lens[b];
+  constexpr float kLog2e = 1.4426950408889634f;
+  const int kps = ((p.topk + p.n_splits - 1) / p.n_splits + kFewTile - 1) / kFewTile * kFewTile;
+  const int k_lo = min(split * kps, p.topk), k_hi = min(k_lo + kps, p.topk);
+
+  // idx -> block table -> cache row of keys threadIdx.x and + 256 of a segment
+  int pos[2], pg[2], blk[2];
+  auto load_idx = [&](int seg_lo) {
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int j = seg_lo + kFewThreads * u + (int)threadIdx.x;
+      pos[u] = j < k_hi ? p.idx[(int64_t)b * p.topk + j] : -1;
+    }
+  };
+  auto load_blk = [&]() {
+    const int32_t* bt_row = p.bt + (int64_t)b * p.max_blocks;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const bool in = pos[u] >= 0 && pos[u] < seq_len;
+      pg[u] = in ? (p.page_shift >= 0 ? pos[u] >> p.page_shift : pos[u] / p.page_size) : 0;
+      blk[u] = in && pg[u] < p.max_blocks ? bt_row[pg[u]] : -1;
+    }
+  };
+  // codes of the segment into LDS; returns its tiles up to the last unmasked key
+  auto publish = [&]() {
+    int last = 0;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int64_t row = (int64_t)blk[u] * p.page_size + (pos[u] - pg[u] * p.page_size);
+      const bool in = pos[u] >= 0 && pos[u] < seq_len && pg[u] < p.max_blocks;
+      const int code = (blk[u] < 0 || row >= p.n_kv_rows) ? ((p.zero_unresolved && in) ? -2 : -1)
+                                                          : (int)row;
+      sh.code[kFewThreads * u + threadIdx.x] = code;
+      if (code != -1) last = kFewThreads * u + (int)threadIdx.x + 1;
+    }
+    last = wave_max_i32(last);
+    if (lane == 0) sh.last[w] = last;
+    lds_barrier();
+    const int n = max(max(sh.last[0], sh.last[1]), max(sh.last[2], sh.last[3]));
+    return __builtin_amdgcn_readfirstlane((n + kFewTile - 1) / kFewTile);
+  };
+  load_idx(k_lo);
+
+  // ---- Q (B operand of S^T = K Q^T): head c, scaled in fp16.  fp8: step 2 n + e
+  // (n < 8) holds dims 64 n + 16 g + 8 e .. +7, 16 + n the RoPE dims 512 + 32 n +
+  // 8 g ..; fp16: step n dims 32 n + 8 g .. ----
+  f16x8 qf[18];
+  {
+    const int h = h0 + c;
+    const f16* qrow = p.q + ((int64_t)b * p.n_head + (h < p.n_head ? h : 0)) * kLatentDim;
+#pragma unroll
+    for (int s = 0; s < 18; s++)
+      qf[s] = *reinterpret_cast<const f16x8*>(
+          qrow + (FP8 && s < 16 ? 64 * (s >> 1) + 16 * g + 8 * (s & 1) : 32 * s + 8 * g));
+  }
+  load_blk();
+  {
+    const f16 sc = (f16)p.scale_h;
+    const f16x8 sc8 = {sc, sc, sc, sc, sc, sc, sc, sc};
+#pragma unroll
+    for (int s = 0; s < 18; s++) qf[s] *= sc8;
+  }
+
+  f32x4 oacc[8];  // O^T of dims 128 w + 16 t + 4 g + r, head c
+#pragma unroll
+  for (int t = 0; t < 8; t++) oacc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  float m_run = -1e30f, l_part = 0.f;  // per head c; l: this lane's keys
+
+  uint8_t* const reg = sh.rows[w];
+  const uint8_t* const kq = reg + 64 * c + 16 * (g ^ few_sw(c));  // QK reads, + 1024 b
+
+  for (int seg_lo = k_lo; seg_lo < k_hi; seg_lo += kFewSeg) {
+    const int ntiles = publish();
+    const bool more = seg_lo + kFewSeg < k_hi;
+    for (int tile = 0; tile < ntiles; tile++) {
+      // ---- this wave's 16 rows ----
+      const int32_t* code = sh.code + kFewTile * tile + 16 * w;
+      {
+        const int row = code[lane >> 2];
+        const uint8_t* src = (row >= 0 ? kv + (int64_t)row * ROW : kZeroRow) +
+                             16 * ((lane & 3) ^ few_sw(lane >> 2));
+        unroll<Sm::BLOCKS>([&](auto bc) {
+          constexpr int bl = bc;
+          dma16_at<FP8 && bl >= 8 ? 528 + 64 * (bl - 8) : 64 * bl>(src, reg + 1024 * bl);
+        });
+        if constexpr (FP8) {
+          const int rs = code[lane & 15];
+          dma4((rs >= 0 ? kv + (int64_t)rs * ROW : kZeroRow) + 512 + 4 * (lane >> 4),
+               reg + 1024 * Sm::BLOCKS);
+        }
+      }
+      const int4 vr = *reinterpret_cast<const int4*>(code + 4 * g);
+      // the next segment's codes, one load step beside each of two gathers
+      if (more && tile == 0) load_idx(seg_lo + kFewSeg);
+      if (more && tile == 1) load_blk();
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+      // ---- scores of keys 4 g + r, head c ----
+      f32x4 sv = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (FP8) {
+        const float* sc = reinterpret_cast<const float*>(reg + 1024 * Sm::BLOCKS) + 4 * g;
+#pragma unroll
+        for (int n = 0; n < 2; n++)
+          sv = mfma16x16x32(*reinterpret_cast<const f16x8*>(kq + 1024 * (8 + n)), qf[16 + n], sv);
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          const f32x4 ks = *reinterpret_cast<const f32x4*>(sc + 16 * t);
+          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int n = 2 * t; n < 2 * t + 2; n++) {
+            const u32x4 raw = *reinterpret_cast<const u32x4*>(kq + 1024 * n);
+            acc = mfma16x16x32(e4m3x8(raw[0], raw[1]), qf[2 * n], acc);
+            acc = mfma16x16x32(e4m3x8(raw[2], raw[3]), qf[2 * n + 1], acc);
+          }
+          sv += ks * acc;
+        }
+      } else {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int n = 0; n < 18; n += 2) {
+          sv = mfma16x16x32(*reinterpret_cast<const f16x8*>(kq + 1024 * n), qf[n], sv);
+          acc = mfma16x16x32(*reinterpret_cast<const f16x8*>(kq + 1024 * (n + 1)), qf[n + 1], acc);
+        }
+        sv += acc;
+      }
+      const int vv[4] = {vr.x, vr.y, vr.z, vr.w};
+      float mt = -1e30f;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        sv[r] = vv[r] != -1 ? sv[r] : -INFINITY;  // -2: a zero row, a valid key
+        mt = fmaxf(mt, sv[r]);
+      }
+      mt = xor32_max(xor16_max(mt));
+      f32x4 pr;
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        pr[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[r], kLog2e, -mt * kLog2e));
+      *reinterpret_cast<f32x4*>(&sh.pt[few_pt(c, 16 * w + 4 * g)]) = pr;
+      if (g == 0) sh.m[w][c] = mt;
+      lds_barrier();  // P, the maxima and every wave's rows are in
+
+      // ---- running max, and the sum of this lane's p ----
+      float mw[4], M = -1e30f;
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        mw[u] = sh.m[u][c];
+        M = fmaxf(M, mw[u]);
+      }
+      if (__any(M > m_run + kPfLazyMax)) {
+        const float m_new = M > m_run + kPfLazyMax ? M : m_run;
+        const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * kLog2e);
+        m_run = m_new;
+        l_part *= alpha;
+#pragma unroll
+        for (int t = 0; t < 8; t++) oacc[t] *= alpha;
+      }
+      l_part += ((pr[0] + pr[1]) + (pr[2] + pr[3])) *
+                __builtin_amdgcn_exp2f((mt - m_run) * kLog2e);
+
+      // ---- O^T += V^T P^T: keys 32 kb + 8 g .. +7 are rows 8 (g & 1) .. of region 2 kb + g / 2 ----
+#pragma unroll
+      for (int kb = 0; kb < 2; kb++) {
+        const uint8_t* rg = sh.rows[2 * kb] + (g >> 1) * Sm::REGION;
+        const f32x4 pa = *reinterpret_cast<const f32x4*>(&sh.pt[few_pt(c, 32 * kb + 8 * g)]);
+        const f32x4 pc = *reinterpret_cast<const f32x4*>(&sh.pt[few_pt(c, 32 * kb + 8 * g + 4)]);
+        const float f = __builtin_amdgcn_exp2f(((g >> 1 ? mw[2 * kb + 1] : mw[2 * kb]) - m_run) * kLog2e);
+        f16x8 pb;
+        if constexpr (FP8) {
+          const float* sc = reinterpret_cast<const float*>(rg + 1024 * Sm::BLOCKS) + 16 * w + 8 * (g & 1);
+          const f32x4 sa = *reinterpret_cast<const f32x4*>(sc) * f;
+          const f32x4 sb = *reinterpret_cast<const f32x4*>(sc + 4) * f;
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            pb[e] = (f16)(pa[e] * sa[e]);
+            pb[4 + e] = (f16)(pc[e] * sb[e]);
+          }
+          // 8-key transpose reads: lane i of a 16-lane group points at key
+          // 8 (g & 1) + i / 2, dims 128 w + 16 t + 8 (i % 2) .. +7
+          const int r = 8 * (g & 1) + (c >> 1);
+          const uint8_t* vb = rg + 2048 * w + 64 * r + 8 * (c & 1);
+#pragma unroll
+          for (int t = 0; t < 8; t++) {
+            const s32x2 v = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+                (lds_s32x2*)(vb + 1024 * (t >> 2) + 16 * ((t & 3) ^ few_sw(r))));
+            oacc[t] = mfma16x16x32(e4m3x8((uint32_t)v[0], (uint32_t)v[1]), pb, oacc[t]);
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            pb[e] = (f16)(pa[e] * f);
+            pb[4 + e] = (f16)(pc[e] * f);
+          }
+          // 4-key reads: key 8 (g & 1) + i / 4 (+ 4), dims 128 w + 16 t + 4 (i % 4) .. +3
+          const int r = 8 * (g & 1) + (c >> 2);
+          const uint8_t* vb = rg + 4096 * w + 64 * r + 8 * (c & 1);
+#pragma unroll
+          for (int t = 0; t < 8; t++) {
+            const int pc16 = 2 * (t & 1) + ((c >> 1) & 1);
+            const s16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (lds_s16x4*)(vb + 1024 * (t >> 1) + 16 * (pc16 ^ few_sw(8 * (g & 1)))));
+            const s16x4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (lds_s16x4*)(vb + 256 + 1024 * (t >> 1) + 16 * (pc16 ^ few_sw(8 * (g & 1) + 4))));
+            const f16x4 x0 = __builtin_bit_cast(f16x4, x), x1 = __builtin_bit_cast(f16x4, y);
+            const f16x8 av = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+            oacc[t] = mfma16x16x32(av, pb, oacc[t]);
+          }
+        }
+      }
+      lds_barrier();  // the tile, P and the maxima are free
+    }
+    if (more) {
+      // every wave has left the last tile's codes (the barrier above, or the
+      // one in publish() where the segment had no tile)
+      if (ntiles < 1) load_idx(seg_lo + kFewSeg);
+      if (ntiles < 2) load_blk();
+      lds_barrier();
+    }
+  }
+
+  // ---- l of every head, then o = O / l and lse, or the split's partial ----
+  l_part = xor32_sum(xor16_sum(l_part));
+  if (g == 0) sh.l[w][c] = l_part;
+  lds_barrier();
+  const float L = (sh.l[0][c] + sh.l[1][c]) + (sh.l[2][c] + sh.l[3][c]);
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const int h = h0 + c;
+  if (h >= p.n_head) return;
+  const int64_t bh = (int64_t)b * p.n_head + h, ps = bh * p.n_splits + split;
+  if (p.n_splits == 1) {
+    f16* orow = p.o + bh * kValueDim + 128 * w;
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+      f16x4 v;
+#pragma unroll
+      for (int r = 0; r < 4; r++) v[r] = (f16)(oacc[t][r] * inv);
+      *reinterpret_cast<f16x4*>(orow + 16 * t + 4 * g) = v;
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      f16x8 o8[2];
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) o8[t >> 1][4 * (t & 1) + r] = (f16)(oacc[4 * j + t][r] * inv);
+      u32x4* dst = reinterpret_cast<u32x4*>(p.part_o + ps * kValueDim + 64 * (2 * w + j) + 16 * g);
+      dst[0] = __builtin_bit_cast(u32x4, o8[0]);
+      dst[1] = __builtin_bit_cast(u32x4, o8[1]);
+    }
+  }
+  if (w == 0 && g == 0) {
+    if (p.n_splits == 1) {
+      p.lse[bh] = (L > 0.f) ? (m_run + logf(L)) : p.empty_lse;
+    } else {
+      p.part_ml[ps * 2 + 0] = m_run;
+      p.part_ml[ps * 2 + 1] = L;
+    }
+  }
+}
+
 // Flash-decode merge of S partial states (reference :1138-1184):
 // m = max_s m_s, w_s = l_s > 0 ? exp(m_s - m) l_s : 0, o = sum w_s o_s / sum w_s
 // (o_s is the split's own normalised output, stored in fp16).
@@ -2388,7 +2281,6 @@ __global__ void __launch_bounds__(kEpiThreads) decode_epilogue_kernel(EpiArgs a)
 // ---------------------------------------------------------------------------
 // launch configuration
 // ---------------------------------------------------------------------------
-constexpr int kDecKW = 4;        // decode: key-waves per workgroup
 constexpr int kTargetWGs = 256;  // one wave of workgroups over 256 CUs
 
 constexpr int kPipeMinUnits = 8;  // 64-head workgroups from which a batch of > 32 heads
@@ -2400,28 +2292,35 @@ static bool use_dma_decode(int topk) {
   return (topk + kDmaSplitKeys - 1) / kDmaSplitKeys <= kMergeMaxSplits;
 }
 
-static int dma_decode_splits(int B, int n_head, int topk) {
-  const int hg = (n_head + 15) / 16;
-  const int units = (topk + kDecWaveKeys - 1) / kDecWaveKeys;  // 16-key units
-  int s = kTargetWGs / (B * hg > 0 ? B * hg : 1);
-  if (s >= 8) s = s / 8 * 8;
-  const int min_s = (topk + kDmaSplitKeys - 1) / kDmaSplitKeys;  // <= 128 keys per split
-  if (s < min_s) s = min_s;
-  if (s > units) s = units;
-  if (s < 1) s = 1;
-  return s;
+// Always 128 keys per split: a workgroup's waves then all have 16 keys, and the
+// chain idx -> table -> rows is the same whatever the split.  More and smaller
+// splits to fill the chip at B = 1 only left waves idle and made the merge
+// longer (us per call, 16-key splits / 32 / 64 / 128: B = 1 x 16 heads 23.2 / 16.4 /
+// 12.9 / 12.4, B = 1 x 64 heads 17.5 / 17.5 / 13.4 / 11.6).
+static int dma_decode_splits(int topk) {
+  const int s = (topk + kDmaSplitKeys - 1) / kDmaSplitKeys;
+  return s < 1 ? 1 : s;
 }
 
-static int decode_splits(int B, int n_head, int topk) {
-  const int hg = (n_head + 15) / 16;
-  const int tiles = (topk + 15) / 16;
-  int s = kTargetWGs / (B * hg > 0 ? B * hg : 1);
-  const int max_s = (tiles + kDecKW - 1) / kDecKW;  // >= one tile per key-wave
-  if (s > max_s) s = max_s;
-  if (s > kMergeMaxSplits) s = kMergeMaxSplits;
-  if (s < 1) s = 1;
-  if (s >= 8) s = s / 8 * 8;  // multiple of 8: a (token, split)'s head groups share an XCD
-  return s;
+// Key splits of `units` workgroups of `tiles` tiles each on `slots` resident
+// workgroups: the fewest rounds x (tiles per split + `fixed`, a workgroup's
+// prologue and epilogue in tiles), at least two tiles per split; one split
+// saves the merge launch (3 tiles).  A count just past a full round costs a
+// whole second one: 24 units of the 64-head fp8 kernel took 35 us with 11 splits
+// (264 workgroups on 256 CUs).
+static int pick_splits(int64_t units, int tiles, int slots, int fixed) {
+  int best = 1;
+  int64_t best_cost = -1;
+  const int max_s = tiles / 2 < kMergeMaxSplits ? tiles / 2 : kMergeMaxSplits;
+  for (int s = 1; s <= (max_s > 1 ? max_s : 1); s++) {
+    const int64_t rounds = (units * s + slots - 1) / slots;
+    const int64_t cost = rounds * ((tiles + s - 1) / s + fixed) + (s > 1 ? 3 : 0);
+    if (best_cost < 0 || cost < best_cost) {
+      best = s;
+      best_cost = cost;
+    }
+  }
+  return best;
 }
 
 // dense decode: splits of the context so that ~256 workgroups run, at least
@@ -2460,13 +2359,13 @@ static int launch_attn_f16(const MlaParams& prm, dim3 grid, hipStream_t st) {
   return check_launch("mla_attn_f16");
 }
 
-template <bool KVFP8, int HW, int KW, int NB>
-static int launch_mla(const MlaParams& prm, dim3 grid, hipStream_t st) {
-  using Smem = MlaSmem<HW, KW, NB>;
-  auto kern = sparse_mla_kernel<KVFP8, HW, KW, NB>;
-  const int rc = reserve_lds(reinterpret_cast<const void*>(kern), sizeof(Smem), "sparse_mla_decode");
+template <bool FP8>
+static int launch_few(const MlaParams& prm, dim3 grid, hipStream_t st) {
+  auto kern = sparse_mla_few_kernel<FP8>;
+  const int rc = reserve_lds(reinterpret_cast<const void*>(kern), sizeof(FewSmem<FP8>),
+                             "sparse_mla_few");
   if (rc) return rc;
-  kern<<<grid, HW * KW * 64, sizeof(Smem), st>>>(prm);
+  kern<<<grid, kFewThreads, sizeof(FewSmem<FP8>), st>>>(prm);
   return check_launch("sparse_mla_decode");
 }
 
@@ -2474,17 +2373,23 @@ static int launch_mla(const MlaParams& prm, dim3 grid, hipStream_t st) {
 
 using namespace mi355dsa;
 
-// Which kernel runs a sparse attention call, and over how many key splits:
-//  * kPipelined: the 64-head pipelined kernels (fp8:
-//    sparse_mla_prefill_fp8_ws_kernel, fp16: mla_attn_f16_kernel), workgroup
-//    = (token, 64 heads, key split), tiles streamed through an LDS ring.  Taken from 256 64-head
-//    workgroups up (one split), and for > 32 heads from kPipeMinUnits up
-//    with round(256 / units) splits of at least two 32-key tiles each;
-//  * kSplitDma: fp8 split decode with per-wave LDS-DMA gathers (16 heads per
-//    workgroup, at most 128 keys per split), for small batches;
-//  * kSplitReg: the register-staged split decode (fp16 rows, or fp8 top-k
-//    lists too long for kSplitDma).
-enum DecodeKind { kPipelined, kSplitDma, kSplitReg };
+// Which kernel runs a sparse attention call, and over how many key splits
+// (units: workgroups without a split; us per call at 20k context, topk 2048):
+//  * kPipelined: 64 heads per workgroup (fp8: sparse_mla_prefill_fp8_ws_kernel,
+//    fp16: mla_hw_f16_kernel or mla_attn_f16_kernel).  From 256 units up in one
+//    split; below that for > 32 heads from 8 units, for 17-32 heads from 32
+//    (32 tokens x 32 heads: fp8 27 against 36 kSplitDma, 34 kFewHeads; fp16 30
+//    against 35; 16 tokens: fp8 22 against 21, fp16 level).  Never for <= 16
+//    heads of fp8 rows, whose 48 empty heads cost more than the shared gather
+//    saves (2048 tokens x 16 heads: 749 us against 393 kFewHeads); fp16 rows the
+//    same (595 against 511).
+//  * kSplitDma: fp8 rows, small batches, 128 keys per split, 16 heads per
+//    workgroup.  For <= 16 heads below 64 tokens (48: 33 against 37 kFewHeads;
+//    64: 43 against 41).
+//  * kFewHeads: 16 heads per workgroup over 64-key tiles, the rest: <= 16 heads,
+//    fp16 batches too small for kPipelined (4 x 64 heads: 17 us), fp8 lists too
+//    long for kSplitDma.
+enum DecodeKind { kPipelined, kSplitDma, kFewHeads };
 struct DecodePlan {
   DecodeKind kind;
   int S;
@@ -2492,24 +2397,27 @@ struct DecodePlan {
 
 static DecodePlan plan_decode(int B, int n_head, int topk, int kv_fp8) {
   const int64_t units = (int64_t)B * ((n_head + 63) / 64);
-  if (units >= kTargetWGs) return {kPipelined, 1};
-  if (n_head > 32 && units >= kPipeMinUnits) {
-    int s = (int)((kTargetWGs + units / 2) / units);  // nearest: fewer partial second rounds
-    const int max_s = (topk + 2 * kPfTileKeys - 1) / (2 * kPfTileKeys);  // >= 2 tiles per split
-    if (s > max_s) s = max_s;
-    if (s > kMergeMaxSplits) s = kMergeMaxSplits;
-    if (s < 1) s = 1;
-    return {kPipelined, s};
+  if (n_head > 16) {
+    if (units >= kTargetWGs) return {kPipelined, 1};
+    if (units >= (n_head > 32 ? kPipeMinUnits : 4 * kPipeMinUnits))
+      return {kPipelined, pick_splits(units, (topk + kPfTileKeys - 1) / kPfTileKeys, kTargetWGs, 7)};
   }
-  if (kv_fp8 && use_dma_decode(topk)) return {kSplitDma, dma_decode_splits(B, n_head, topk)};
-  return {kSplitReg, decode_splits(B, n_head, topk)};
+  if (kv_fp8 && use_dma_decode(topk) && (n_head > 16 || B < kFewMinTokens))
+    return {kSplitDma, dma_decode_splits(topk)};
+  return {kFewHeads, pick_splits((int64_t)B * ((n_head + 15) / 16),
+                                 (topk + kFewTile - 1) / kFewTile,
+                                 (kv_fp8 ? 3 : 2) * kTargetWGs, 2)};
 }
 
 extern "C" size_t mi355_dsa_sparse_mla_workspace_size(int B, int n_head, int topk) {
   if (B <= 0 || n_head <= 0 || topk <= 0) return 0;
-  // the larger of the fp16 and fp8 split counts, so one size serves both
+  // the larger of the fp16 and fp8 split counts, so one size serves both; for few
+  // heads at least the split decode's, whichever kernel runs: the size, and with
+  // it what the allocation-free entry takes, does not depend on that choice
   const int s16 = plan_decode(B, n_head, topk, 0).S, s8 = plan_decode(B, n_head, topk, 1).S;
-  const int S = s16 > s8 ? s16 : s8;
+  int S = s16 > s8 ? s16 : s8;
+  if (n_head <= 32 && (int64_t)B < kTargetWGs && use_dma_decode(topk) && dma_decode_splits(topk) > S)
+    S = dma_decode_splits(topk);
   if (S <= 1) return 0;
   return (size_t)B * n_head * S * (kValueDim * sizeof(f16) + 2 * sizeof(float));
 }
@@ -2533,8 +2441,6 @@ static int mla_decode_impl(
   DSA_CHECK(max_blocks == 0 || block_table, "null block_table");
   DSA_CHECK(aligned_to(q, 16) && aligned_to(kv_cache, 16) && aligned_to(o, 8),
             "q / kv_cache / o misaligned");
-  DSA_CHECK(B <= 65535 || dense || plan_decode(B, n_head, topk, kv_fp8).kind == kPipelined,
-            "B too large");
   MlaParams prm;
   prm.q = reinterpret_cast<const f16*>(q);
   prm.kv = kv_cache;
@@ -2593,7 +2499,6 @@ static int mla_decode_impl(
     prm.part_o = reinterpret_cast<f16*>(workspace);
     prm.part_ml = reinterpret_cast<float*>(prm.part_o + (size_t)B * n_head * S * kValueDim);
   }
-  const dim3 grid(S, (n_head + 15) / 16, B);
   int rc;
   if (plan.kind == kPipelined) {
     const dim3 pgrid(B, (n_head + 63) / 64, S);
@@ -2616,8 +2521,8 @@ static int mla_decode_impl(
     sparse_mla_decode_dma_kernel<<<dim3((unsigned)nwg), kDmaThreads, sizeof(DmaSmem), st>>>(prm);
     rc = check_launch("sparse_mla_decode");
   } else {
-    rc = kv_fp8 ? launch_mla<true, 1, kDecKW, 1>(prm, grid, st)
-                : launch_mla<false, 1, kDecKW, 1>(prm, grid, st);
+    const dim3 fgrid(B, (n_head + 15) / 16, S);
+    rc = kv_fp8 ? launch_few<true>(prm, fgrid, st) : launch_few<false>(prm, fgrid, st);
   }
   if (rc != MI355_DSA_OK || S == 1) return rc;
   if (epi) {  // the fused merge + W_UV epilogue of a layer step

@@ -99,7 +99,7 @@ def test_decode_invalid_entries(ops, dev):
 UNRESOLVED = [
     # B, H, fp8, topk: kernel path -> rule for a position below seq_len on a bad block
     (4, 64, True, 2048),    # fp8 split decode (LDS-DMA kernel): zero key
-    (2, 64, False, 1024),   # fp16 split decode (register-staged kernel): zero key
+    (2, 64, False, 1024),   # fp16 split decode (16-head workgroups): zero key
     (16, 64, True, 2048),   # fp8 pipelined kernel with 16 key splits: zero key
     (16, 64, False, 2048),  # fp16 pipelined kernel with 16 key splits: zero key
     (300, 64, True, 256),   # fp8 prefill configuration: zero key (64 heads)
@@ -211,6 +211,27 @@ def test_lists_with_unused_tiles(ops, dev, fp8, H):
     for b in range(B):
         lo, hi = VALID_SLOTS[b % len(VALID_SLOTS)]
         idx[b, (slot < lo) | (slot >= hi)] = -1
+    o, lse = run(ops, dev, q, kv, idx, bt, seq)
+    ro, rl = O.sparse_mla(q, kv, idx, bt, seq, SCALE)
+    check(o, lse, ro, rl)
+
+
+FEW_HEADS = [
+    # B, H, fp8, topk: 16-head workgroups over 64-key tiles and 512-key segments,
+    # alone and split; head counts off 16, lists off the tile and the segment
+    (3, 16, False, 1), (3, 5, False, 63), (2, 16, False, 65), (2, 24, False, 513),
+    (1, 64, False, 2048), (5, 40, False, 1100), (600, 16, False, 130), (64, 16, True, 2048),
+    (70, 16, True, 64), (600, 3, True, 577), (300, 8, True, 1025), (800, 16, True, 300),
+]
+
+
+@pytest.mark.parametrize("case", FEW_HEADS, ids=["B%dH%d%sK%d" % (b, h, "fp8" if f else "fp16", k)
+                                                for b, h, f, k in FEW_HEADS])
+def test_few_heads(ops, dev, case):
+    B, H, fp8, topk = case
+    seqs = [1 + (37 * i + 900) % 2200 for i in range(B)]
+    q, kv, idx, bt, seq = make(80 + B + topk, B, H, 40, 64, fp8, topk, seqs, invalid_frac=0.1)
+    q *= 4  # scores far enough apart for the running maximum to move
     o, lse = run(ops, dev, q, kv, idx, bt, seq)
     ro, rl = O.sparse_mla(q, kv, idx, bt, seq, SCALE)
     check(o, lse, ro, rl)
