@@ -127,7 +127,7 @@ struct LayerIdxArgs {
   int n_tiles;
 };
 
-template <bool KFP8>
+template <bool KFP8, int PPB>
 __global__ void __launch_bounds__(256) decode_layer_indexer_kernel(LayerIdxArgs a) {
   int id = blockIdx.x;
   if (id < a.pro.lat_wgs) {  // the latent-cache write
@@ -150,7 +150,7 @@ __global__ void __launch_bounds__(256) decode_layer_indexer_kernel(LayerIdxArgs 
   id = blockIdx.x;
   if (id < a.n_pro) return;
   const int i = id - a.n_pro;
-  indexer_logits_block<KFP8, true>(a.idx, i % a.n_tiles, i / a.n_tiles, a.nk);
+  indexer_logits_block<KFP8, true, PPB>(a.idx, i % a.n_tiles, i / a.n_tiles, a.nk);
 }
 
 }  // namespace
@@ -300,14 +300,22 @@ extern "C" int mi355_dsa_decode_layer_indexer(
   a.nk.T = T;
   a.nk.dst = idx_cache;
   a.n_pro = (int)n_pro;
-  a.n_tiles = (max_kv + kIdxPPB - 1) / kIdxPPB;
+  const int ppb = idx_decode_ppb(B, max_kv);
+  a.n_tiles = (max_kv + ppb - 1) / ppb;
   const int64_t total = n_pro + (int64_t)a.n_tiles * B;
   DSA_CHECK(total < ((int64_t)1 << 31), "decode_layer_indexer: grid too large");
   hipStream_t st = as_stream(stream);
-  if (idx_fp8)
-    decode_layer_indexer_kernel<true><<<dim3((unsigned)total), 256, 0, st>>>(a);
-  else
-    decode_layer_indexer_kernel<false><<<dim3((unsigned)total), 256, 0, st>>>(a);
+  auto launch = [&](auto kernel) { kernel<<<dim3((unsigned)total), 256, 0, st>>>(a); };
+  if (ppb == kIdxPPB) {
+    if (idx_fp8) launch(decode_layer_indexer_kernel<true, kIdxPPB>);
+    else launch(decode_layer_indexer_kernel<false, kIdxPPB>);
+  } else if (ppb == kIdxPPBMid) {
+    if (idx_fp8) launch(decode_layer_indexer_kernel<true, kIdxPPBMid>);
+    else launch(decode_layer_indexer_kernel<false, kIdxPPBMid>);
+  } else {
+    if (idx_fp8) launch(decode_layer_indexer_kernel<true, kIdxPPBSmall>);
+    else launch(decode_layer_indexer_kernel<false, kIdxPPBSmall>);
+  }
   DSA_LAUNCH_CHECK("decode_layer_indexer");
   return MI355_DSA_OK;
 }

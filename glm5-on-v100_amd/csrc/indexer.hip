@@ -32,12 +32,13 @@ namespace mi355dsa {
 // ===========================================================================
 // decode / generic kernel: the workgroup body is indexer_logits_block
 // (indexer_decode.h), shared with the fused decode-layer launch.
-// A workgroup of 4 waves owns 1024 positions of one token row; a wave scores
+// A workgroup of 4 waves owns 1024 positions of one token row (512 or 128 in
+// launches that would leave CUs idle, idx_decode_ppb); a wave scores
 // 16 keys per MFMA group (S = Q . K^T, M = 16 heads x 2 tiles, N = 16 keys,
 // K = 128), keys loaded straight from HBM into B-operand registers (no LDS),
 // double buffered.
 // ===========================================================================
-template <bool KFP8>
+template <bool KFP8, int PPB>
 __global__ void __launch_bounds__(kIdxWaves * 64) indexer_logits_kernel(
     const f16* __restrict__ Q, const void* __restrict__ Kv, const f16* __restrict__ W,
     const int32_t* __restrict__ block_table, const int32_t* __restrict__ seq_lens,
@@ -46,7 +47,7 @@ __global__ void __launch_bounds__(kIdxWaves * 64) indexer_logits_kernel(
   const IdxDecArgs a{Q, Kv, W, block_table, seq_lens, score, hist, n_kv_rows, max_blocks,
                      page_shift, max_kv, hist8, span};
   const IdxNewKeys none{};
-  indexer_logits_block<KFP8, false>(a, blockIdx.x, blockIdx.y, none);
+  indexer_logits_block<KFP8, false, PPB>(a, blockIdx.x, blockIdx.y, none);
 }
 
 // ===========================================================================
@@ -590,7 +591,8 @@ extern "C" int mi355_dsa_indexer_logits(
   DSA_CHECK(k_fp8 ? aligned_to(k_cache, 4) : aligned_to(k_cache, 16),
             "k_cache is misaligned");
   DSA_CHECK(B <= 65535, "B too large");
-  const dim3 grid((max_kv + kIdxPPB - 1) / kIdxPPB, B);
+  const int ppb = idx_decode_ppb(B, max_kv);
+  const dim3 grid((max_kv + ppb - 1) / ppb, B);
   const int shift = ilog2_pow2(page_size);
   hipStream_t st = as_stream(stream);
   uint32_t* h = reinterpret_cast<uint32_t*>(hist);
@@ -609,14 +611,21 @@ extern "C" int mi355_dsa_indexer_logits(
   a.max_kv = max_kv;
   a.hist8 = hist8;
   a.span = idx_span_launch(k_fp8, B, max_kv);
-  if (k_fp8)
-    indexer_logits_kernel<true><<<grid, kIdxWaves * 64, 0, st>>>(
-        a.Q, a.Kv, a.W, a.block_table, a.seq_lens, a.score, a.hist, a.n_kv_rows, a.max_blocks,
-        a.page_shift, a.max_kv, a.hist8, a.span);
-  else
-    indexer_logits_kernel<false><<<grid, kIdxWaves * 64, 0, st>>>(
-        a.Q, a.Kv, a.W, a.block_table, a.seq_lens, a.score, a.hist, a.n_kv_rows, a.max_blocks,
-        a.page_shift, a.max_kv, a.hist8, a.span);
+  auto launch = [&](auto kernel) {
+    kernel<<<grid, kIdxWaves * 64, 0, st>>>(a.Q, a.Kv, a.W, a.block_table, a.seq_lens, a.score,
+                                            a.hist, a.n_kv_rows, a.max_blocks, a.page_shift,
+                                            a.max_kv, a.hist8, a.span);
+  };
+  if (ppb == kIdxPPB) {
+    if (k_fp8) launch(indexer_logits_kernel<true, kIdxPPB>);
+    else launch(indexer_logits_kernel<false, kIdxPPB>);
+  } else if (ppb == kIdxPPBMid) {
+    if (k_fp8) launch(indexer_logits_kernel<true, kIdxPPBMid>);
+    else launch(indexer_logits_kernel<false, kIdxPPBMid>);
+  } else {
+    if (k_fp8) launch(indexer_logits_kernel<true, kIdxPPBSmall>);
+    else launch(indexer_logits_kernel<false, kIdxPPBSmall>);
+  }
   DSA_LAUNCH_CHECK("indexer_logits");
   return MI355_DSA_OK;
 }

@@ -15,7 +15,8 @@ namespace mi355dsa {
 // ===========================================================================
 constexpr int kIdxWaves = 4;
 constexpr int kIdxPPB = 1024;             // positions per workgroup
-constexpr int kIdxBlocksPerWave = kIdxPPB / 16 / kIdxWaves;  // 16
+constexpr int kIdxPPBMid = 512;           // and in launches that would leave CUs idle
+constexpr int kIdxPPBSmall = 128;         // (idx_decode_ppb)
 constexpr int kIdxGroup = 2;              // 16-key blocks per pipeline stage
 // LDS slot of one staged fp8 block: 16 rows x 132 bytes, then the padding
 // that the last DMA's lanes 16-63 fill
@@ -125,6 +126,23 @@ __host__ __device__ inline int idx_span_launch(int k_fp8, int B, int max_kv) {
   return k_fp8 && (int64_t)B * ((max_kv + kIdxPPB - 1) / kIdxPPB) >= kIdxSpanMinWorkgroups;
 }
 
+// Positions per workgroup.  A workgroup's time is a chain (block table, keys
+// stage by stage, scores, histogram flush), so a launch that leaves CUs idle
+// gains from shorter ranges; but every workgroup flushes its own histogram,
+// and the flushes of one row queue on the same hot bins, so past about two
+// launches' worth of CUs shorter ranges lose.  Measured, whole decode layer,
+// fp16 keys, us with 1024 / 512 / 128 positions: 1 row x 4k 36.4 / 32.8 /
+// 30.1, 4 x 4k 39.6 / 35.6 / 32.8, 1 x 64k 38.0 / 35.5 / 39.2, 1 x 128k
+// 39.4 / 38.4 / 48.3, 4 x 40k 41.0 / 42.3 / 48.4, 64 x 1000 (64 workgroups
+// of 1024) 87.7 / 84.4 / 80.9.
+constexpr int kIdxSmallMaxWorkgroups = 48;  // of 1024 positions
+constexpr int kIdxMidMaxWorkgroups = 128;
+inline int idx_decode_ppb(int B, int max_kv) {
+  const int64_t n = (int64_t)B * ((max_kv + kIdxPPB - 1) / kIdxPPB);
+  if (n <= kIdxSmallMaxWorkgroups) return kIdxPPBSmall;
+  return n <= kIdxMidMaxWorkgroups ? kIdxPPBMid : kIdxPPB;
+}
+
 // The step's new index keys, for a launch that also writes them to the
 // cache (the fused decode-layer launch): fp16 rows [T, 128] and their slots.
 constexpr int kIdxMaxNew = 64;
@@ -149,7 +167,7 @@ __device__ __forceinline__ void idx_key_row_store(const u32x4 raw, void* dst, in
   }
 }
 
-// Workgroup (tile, b) of the decode logits: positions [1024 tile, +1024) of
+// Workgroup (tile, b) of the decode logits: positions [PPB tile, +PPB) of
 // token row b.  With NEWK, positions whose cache row is the slot of one of
 // the step's new keys get that key written to the row first, by this
 // workgroup, so that it reads exactly what a separate store launch before it
@@ -159,19 +177,20 @@ __device__ __forceinline__ void idx_key_row_store(const u32x4 raw, void* dst, in
 // from a struct, so that the compiler keeps knowing that the score stores
 // do not alias the key loads.  Kv is not restrict: with NEWK the same rows
 // are written through nk.dst, and read after the workgroup barrier.)
-template <bool KFP8, bool NEWK>
+template <bool KFP8, bool NEWK, int PPB>
 __device__ __forceinline__ void indexer_logits_body(
     const f16* __restrict__ Q, const void* Kv, const f16* __restrict__ W,
     const int32_t* __restrict__ block_table, const int32_t* __restrict__ seq_lens,
     float* __restrict__ score, uint32_t* __restrict__ hist, int64_t n_kv_rows, int max_blocks,
     int page_shift, int max_kv, int hist8, int span, int tile, int b, const IdxNewKeys& nk) {
-  const int p_lo = tile * kIdxPPB;
-  const int p_hi = min(p_lo + kIdxPPB, max_kv);
+  constexpr bool kSpan = KFP8 && PPB == kIdxPPB;  // only such launches ask for spans
+  const int p_lo = tile * PPB;
+  const int p_hi = min(p_lo + PPB, max_kv);
   // The block-table entries of the tile's pages are loaded beside seq_len
   // (one round trip instead of two before the first key load); a tile past
   // the context reads them for nothing.
   constexpr int kNT = kIdxWaves * 64;
-  constexpr int kBtRegs = (kIdxPPB + 2 + kNT - 1) / kNT;
+  constexpr int kBtRegs = (PPB + 2 + kNT - 1) / kNT;
   const int pg0 = p_lo >> page_shift;
   const int npg = ((p_hi - 1) >> page_shift) - pg0 + 1;
   const int32_t* bt_row = block_table + (int64_t)b * max_blocks;
@@ -190,12 +209,12 @@ __device__ __forceinline__ void indexer_logits_body(
     return;
   }
 
-  __shared__ int32_t s_bt[kIdxPPB + 2];
+  __shared__ int32_t s_bt[PPB + 2];
   // level-1 counts of this workgroup's keys, two 16-bit bins per word (a
-  // workgroup counts at most 1024 keys)
+  // workgroup counts at most PPB keys)
   __shared__ uint32_t s_hist[kTopkBins / 2];
   // fp8 span path: per wave, two stages of kIdxGroup staged blocks
-  __shared__ __align__(16) uint8_t s_span[KFP8 ? kIdxWaves * 2 * kIdxGroup * kIdxSpanSlot : 16];
+  __shared__ __align__(16) uint8_t s_span[kSpan ? kIdxWaves * 2 * kIdxGroup * kIdxSpanSlot : 16];
   __shared__ int32_t s_new[NEWK ? 2 * kIdxMaxNew : 1];  // slots, then "this workgroup reads it"
   const int page = 1 << page_shift;
 #pragma unroll
@@ -286,8 +305,9 @@ __device__ __forceinline__ void indexer_logits_body(
   };
 
   KeyFrag cur[kIdxGroup], nxt[kIdxGroup];
-  constexpr int n_groups = kIdxBlocksPerWave / kIdxGroup;
-  static_assert(n_groups >= 2, "the span path's vmcnt waits assume two stages or more");
+  constexpr int n_groups = PPB / 16 / kIdxWaves / kIdxGroup;
+  static_assert(n_groups >= 1 && PPB <= 1024, "whole stages; 16-bit counts");
+  static_assert(!kSpan || n_groups >= 2, "the span path's vmcnt waits assume two stages or more");
   // wave w owns blocks w, w+4, w+8, ... ; stage i covers its blocks
   // [i*kIdxGroup, (i+1)*kIdxGroup) in that order.
   auto blk_of = [&](int stage, int j) { return (stage * kIdxGroup + j) * kIdxWaves + wave; };
@@ -322,10 +342,10 @@ __device__ __forceinline__ void indexer_logits_body(
   // >= 16 rows that the cache holds whole (its row count
   // a multiple of the page), 16-byte aligned: the 16 keys of a block are 16
   // consecutive rows, one 2112-byte span.
-  const bool span_ok = KFP8 && span && page_shift >= 4 && n_kv_rows > 0 &&
+  const bool span_ok = kSpan && span && page_shift >= 4 && n_kv_rows > 0 &&
                        (n_kv_rows & (page - 1)) == 0 &&
                        ((uintptr_t)Kv & 15) == 0;
-  if (KFP8 && span_ok && p_lo + kIdxPPB <= max_kv) {
+  if (kSpan && span_ok && p_lo + PPB <= max_kv) {
     // Whole workgroup inside the row.  Each block's span goes to LDS by
     // LDS-DMA in three instructions: bytes [0, 1024) and [1024, 2048), 16
     // per lane, and [2048, 2112), 4 per lane from lanes 0-15 (lanes 16-63
@@ -390,7 +410,7 @@ __device__ __forceinline__ void indexer_logits_body(
         for (int j = 0; j < kIdxGroup; j++) okc[j] = okn[j];
       }
     }
-  } else if (p_lo + kIdxPPB <= max_kv && n_kv_rows > 0) {
+  } else if (p_lo + PPB <= max_kv && n_kv_rows > 0) {
     // Whole workgroup inside the row: no branch around any global load or
     // store.  Every lane stores its key's score (the four lanes of a key
     // write the same bits), so the waits before a stage's MFMAs count
@@ -494,10 +514,10 @@ __device__ __forceinline__ void indexer_logits_body(
   }
 }
 
-template <bool KFP8, bool NEWK>
+template <bool KFP8, bool NEWK, int PPB>
 __device__ __forceinline__ void indexer_logits_block(const IdxDecArgs& a, int tile, int b,
                                                      const IdxNewKeys& nk) {
-  indexer_logits_body<KFP8, NEWK>(a.Q, a.Kv, a.W, a.block_table, a.seq_lens, a.score, a.hist,
+  indexer_logits_body<KFP8, NEWK, PPB>(a.Q, a.Kv, a.W, a.block_table, a.seq_lens, a.score, a.hist,
                                   a.n_kv_rows, a.max_blocks, a.page_shift, a.max_kv, a.hist8,
                                   a.span, tile, b, nk);
 }

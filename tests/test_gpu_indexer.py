@@ -151,6 +151,42 @@ def test_fp8_span_and_per_key_loads_agree(ops, dev, page):
         assert torch.equal(outs[0][1][b].long(), ref)
 
 
+@pytest.mark.parametrize("max_kv,page", [(3077, 64), (2176, 256), (1024, 16), (1, 64)])
+@pytest.mark.parametrize("fp8", [False, True], ids=["fp16", "fp8"])
+def test_launch_widths_agree(ops, dev, fp8, max_kv, page):
+    """The positions per workgroup follow the launch's size (128, 512 or 1024);
+    a row's scores and histogram do not: three rows (edges of the ranges, an
+    unmapped page) alone, and repeated until each width has been taken, give
+    the same bits, and the first width is pinned against the oracle."""
+    n = -(-max_kv // 1024)
+    seqs = [max_kv, max(max_kv - 1, 0), min(max_kv, 513)]
+    q, kc, w, bt, seq = make_case(31 + max_kv, 3, -(-max_kv // page) + 2, page, fp8, True, max_kv,
+                                  seqs)
+    bt[1, bt.shape[1] // 2] = -1
+    first = None
+    for reps in (1, 1 + 48 // (3 * n), 1 + 128 // (3 * n)):
+        B = 3 * reps
+        score = torch.full((B, max_kv), 7.0, device=dev)
+        hist = torch.zeros(B, 4096, dtype=torch.int32, device=dev)
+        ops.sm70_indexer_logits(score, q.repeat(reps, 1, 1).to(dev), kc.to(dev),
+                                w.repeat(reps, 1).to(dev), bt.repeat(reps, 1).to(dev),
+                                seq.repeat(reps).to(dev), hist)
+        score, hist = score.cpu().view(reps, 3, max_kv), hist.cpu().view(reps, 3, 4096)
+        if first is None:
+            first = score[0], hist[0]
+            want, _ = O.indexer_logits(q, kc, w, bt, seq, max_kv)
+            fin = torch.isfinite(want)
+            assert torch.equal(torch.isinf(score[0]), ~fin)
+            # fp16 rows are dyadic (exact); fp8 rows scale each dot product
+            tol = 1e-5 * want[fin].abs().max().item() + 1e-6 if fp8 else 0.0
+            assert (score[0][fin] - want[fin]).abs().max().item() <= tol
+        assert torch.equal(score, first[0].expand(reps, -1, -1))
+        assert torch.equal(hist, first[1].expand(reps, -1, -1))
+        for b in range(3):
+            ref = torch.bincount((O.mono_key(score[0, b, :seqs[b]]) >> 20).long(), minlength=4096)
+            assert torch.equal(hist[0, b].long(), ref)
+
+
 def test_duplicate_keys_score_identically(ops, dev):
     g = torch.Generator().manual_seed(11)
     page, nblk = 64, 32
