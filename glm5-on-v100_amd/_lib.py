@@ -52,6 +52,9 @@ SIGNATURES = {
                                                 _c_i64, _c_int, _p, _c_int, _p, _c_int, _c_i64,
                                                 _p, _p, _p, _c_int, _c_int, _p, _p, _c_int, _p,
                                                 _c_int, _p, _p, _p]),
+    "mi355_dsa_decode_layer_indexer_spec": (_c_int, [
+        _c_int, _p, _c_int, _c_i64, _p, _c_i64, _p, _c_i64, _c_int, _p, _c_int, _p, _c_int, _c_i64,
+        _p, _p, _p, _c_int, _c_int, _p, _p, _c_int, _p, _c_int, _p, _p, _c_int, _p, _p, _p]),
     "mi355_dsa_indexer_logits": (_c_int, [_p, _c_int, _c_int, _p, _c_int, _c_int, _p, _c_int,
                                           _c_i64, _c_int, _p, _p, _c_int, _p, _p, _p]),
     "mi355_dsa_indexer_logits_packed": (_c_int, [_p, _c_int, _c_int, _p, _p, _c_int, _c_i64,

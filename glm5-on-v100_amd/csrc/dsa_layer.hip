@@ -124,10 +124,11 @@ struct LayerIdxArgs {
   int n_pro;
   IdxDecArgs idx;
   IdxNewKeys nk;
+  IdxSpecRows sp;
   int n_tiles;
 };
 
-template <bool KFP8, int PPB>
+template <bool KFP8, int PPB, int NQ>
 __global__ void __launch_bounds__(256) decode_layer_indexer_kernel(LayerIdxArgs a) {
   int id = blockIdx.x;
   if (id < a.pro.lat_wgs) {  // the latent-cache write
@@ -150,7 +151,8 @@ __global__ void __launch_bounds__(256) decode_layer_indexer_kernel(LayerIdxArgs 
   id = blockIdx.x;
   if (id < a.n_pro) return;
   const int i = id - a.n_pro;
-  indexer_logits_block<KFP8, true, PPB>(a.idx, i % a.n_tiles, i / a.n_tiles, a.nk);
+  indexer_logits_block<KFP8, true, PPB, NQ>(a.idx, i % a.n_tiles, NQ * (i / a.n_tiles), a.nk,
+                                            a.sp);
 }
 
 }  // namespace
@@ -256,13 +258,13 @@ extern "C" int mi355_dsa_decode_layer_prologue(
 // that row first, with the store's own code.  The histogram must be zero on
 // entry (mi355_dsa_decode_layer_topk leaves it so); the step's tokens are at
 // most kIdxMaxNew.
-extern "C" int mi355_dsa_decode_layer_indexer(
+static int decode_layer_indexer_impl(
     int T, void* kv_cache, int kv_fp8, int64_t kv_rows, const void* kv_c, int64_t kv_c_stride,
     const void* k_pe, int64_t k_pe_stride, int in_bf16, const void* slot_mapping, int slot_i64,
     void* idx_cache, int idx_fp8, int64_t idx_rows, const void* idx_k, const int32_t* idx_slot,
     float* score, int B, int max_kv, const void* idx_q, const void* idx_w, int idx_page_size,
     const int32_t* block_table, int max_blocks, const int32_t* seq_lens, int32_t* hist,
-    void* stream) {
+    const IdxSpecRows& sp, void* stream) {
   clear_error();
   LayerIdxArgs a{};
   int64_t n_pro = 0;
@@ -300,22 +302,76 @@ extern "C" int mi355_dsa_decode_layer_indexer(
   a.nk.T = T;
   a.nk.dst = idx_cache;
   a.n_pro = (int)n_pro;
-  const int ppb = idx_decode_ppb(B, max_kv);
+  a.sp = sp;
+  // fp16 keys, an even number of tokens per request and still more than a
+  // launch of full ranges: two tokens share a workgroup's keys
+  const int ppb2 = idx_decode_ppb(B / 2, max_kv);
+  const int nq = !idx_fp8 && sp.n % 2 == 0 && ppb2 == kIdxPPB ? 2 : 1;
+  const int ppb = nq == 2 ? ppb2 : idx_decode_ppb(B, max_kv);
   a.n_tiles = (max_kv + ppb - 1) / ppb;
-  const int64_t total = n_pro + (int64_t)a.n_tiles * B;
+  const int64_t total = n_pro + (int64_t)a.n_tiles * (B / nq);
   DSA_CHECK(total < ((int64_t)1 << 31), "decode_layer_indexer: grid too large");
   hipStream_t st = as_stream(stream);
   auto launch = [&](auto kernel) { kernel<<<dim3((unsigned)total), 256, 0, st>>>(a); };
-  if (ppb == kIdxPPB) {
-    if (idx_fp8) launch(decode_layer_indexer_kernel<true, kIdxPPB>);
-    else launch(decode_layer_indexer_kernel<false, kIdxPPB>);
+  if (nq == 2) {
+    launch(decode_layer_indexer_kernel<false, kIdxPPB, 2>);
+  } else if (ppb == kIdxPPB) {
+    if (idx_fp8) launch(decode_layer_indexer_kernel<true, kIdxPPB, 1>);
+    else launch(decode_layer_indexer_kernel<false, kIdxPPB, 1>);
   } else if (ppb == kIdxPPBMid) {
-    if (idx_fp8) launch(decode_layer_indexer_kernel<true, kIdxPPBMid>);
-    else launch(decode_layer_indexer_kernel<false, kIdxPPBMid>);
+    if (idx_fp8) launch(decode_layer_indexer_kernel<true, kIdxPPBMid, 1>);
+    else launch(decode_layer_indexer_kernel<false, kIdxPPBMid, 1>);
   } else {
-    if (idx_fp8) launch(decode_layer_indexer_kernel<true, kIdxPPBSmall>);
-    else launch(decode_layer_indexer_kernel<false, kIdxPPBSmall>);
+    if (idx_fp8) launch(decode_layer_indexer_kernel<true, kIdxPPBSmall, 1>);
+    else launch(decode_layer_indexer_kernel<false, kIdxPPBSmall, 1>);
   }
   DSA_LAUNCH_CHECK("decode_layer_indexer");
   return MI355_DSA_OK;
+}
+
+extern "C" int mi355_dsa_decode_layer_indexer(
+    int T, void* kv_cache, int kv_fp8, int64_t kv_rows, const void* kv_c, int64_t kv_c_stride,
+    const void* k_pe, int64_t k_pe_stride, int in_bf16, const void* slot_mapping, int slot_i64,
+    void* idx_cache, int idx_fp8, int64_t idx_rows, const void* idx_k, const int32_t* idx_slot,
+    float* score, int B, int max_kv, const void* idx_q, const void* idx_w, int idx_page_size,
+    const int32_t* block_table, int max_blocks, const int32_t* seq_lens, int32_t* hist,
+    void* stream) {
+  return decode_layer_indexer_impl(
+      T, kv_cache, kv_fp8, kv_rows, kv_c, kv_c_stride, k_pe, k_pe_stride, in_bf16, slot_mapping,
+      slot_i64, idx_cache, idx_fp8, idx_rows, idx_k, idx_slot, score, B, max_kv, idx_q, idx_w,
+      idx_page_size, block_table, max_blocks, seq_lens, hist, IdxSpecRows{1, nullptr, nullptr},
+      stream);
+}
+
+// The same for a speculative step: B tokens of B / n requests, block_table
+// [B / n, max_blocks] and seq_lens [B / n] per request.  The launch expands
+// them per token itself and writes the expanded tables (bt_out, sl_out) for
+// the launches that follow: the tensor operations it replaces are four
+// launches (24 requests x 2 tokens to 30k, fp8 keys: 115.2 -> 104.6 us per
+// layer).  With fp16 keys and n even, two tokens share a workgroup's key
+// loads (fp16 keys, one token / two tokens per workgroup, us per layer: 24 x 2
+// to 30k 123.2 / 113.6, 2 x 2 x 184k 67.4 / 60.7, 8 x 2 x 30k 73.1 / 68.3);
+// fp8 rows are half the bytes and the instructions bound that kernel, so the
+// lower occupancy of two rows' operands and histograms costs what the sharing
+// saves (24 x 2 to 30k 108.5 / 110.0, 32 x 2 x 8k 94.2 / 97.4), as it does in
+// small launches (1 x 2 x 4k 31.4 / 33.7).
+extern "C" int mi355_dsa_decode_layer_indexer_spec(
+    int T, void* kv_cache, int kv_fp8, int64_t kv_rows, const void* kv_c, int64_t kv_c_stride,
+    const void* k_pe, int64_t k_pe_stride, int in_bf16, const void* slot_mapping, int slot_i64,
+    void* idx_cache, int idx_fp8, int64_t idx_rows, const void* idx_k, const int32_t* idx_slot,
+    float* score, int B, int max_kv, const void* idx_q, const void* idx_w, int idx_page_size,
+    const int32_t* block_table, int max_blocks, const int32_t* seq_lens, int32_t* hist, int n,
+    int32_t* bt_out, int32_t* sl_out, void* stream) {
+  clear_error();
+  DSA_CHECK(n >= 2 && B >= 1 && B % n == 0,
+            "decode_layer_indexer_spec: B must be a multiple of n >= 2");
+  DSA_CHECK(bt_out && sl_out, "decode_layer_indexer_spec: null pointer argument");
+  DSA_CHECK(idx_page_size > 0 && max_blocks > 0 &&
+                (int64_t)max_blocks * idx_page_size == max_kv,
+            "decode_layer_indexer_spec: max_kv must be max_blocks pages");
+  return decode_layer_indexer_impl(
+      T, kv_cache, kv_fp8, kv_rows, kv_c, kv_c_stride, k_pe, k_pe_stride, in_bf16, slot_mapping,
+      slot_i64, idx_cache, idx_fp8, idx_rows, idx_k, idx_slot, score, B, max_kv, idx_q, idx_w,
+      idx_page_size, block_table, max_blocks, seq_lens, hist, IdxSpecRows{n, bt_out, sl_out},
+      stream);
 }

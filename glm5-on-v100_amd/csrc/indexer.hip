@@ -47,7 +47,8 @@ __global__ void __launch_bounds__(kIdxWaves * 64) indexer_logits_kernel(
   const IdxDecArgs a{Q, Kv, W, block_table, seq_lens, score, hist, n_kv_rows, max_blocks,
                      page_shift, max_kv, hist8, span};
   const IdxNewKeys none{};
-  indexer_logits_block<KFP8, false, PPB>(a, blockIdx.x, blockIdx.y, none);
+  indexer_logits_block<KFP8, false, PPB, 1>(a, blockIdx.x, blockIdx.y, none,
+                                            IdxSpecRows{1, nullptr, nullptr});
 }
 
 // ===========================================================================

@@ -154,6 +154,16 @@ struct IdxNewKeys {
                         // the launch also reads keys from (Kv)
 };
 
+// Rows of a speculative step: n tokens per request share the request's
+// block-table row; token j of request r (row r n + j) sees seq_lens[r] -
+// (n - 1) + j positions.  The workgroups also write the per-token tables
+// (bt_out [B, max_blocks], sl_out [B]) that the step's later launches read.
+struct IdxSpecRows {
+  int n;  // 1: block_table and seq_lens are per token already, nothing written
+  int32_t* bt_out;
+  int32_t* sl_out;
+};
+
 // One indexer-K row written as the cache's store kernel writes it: 16 lanes
 // (sub = 0..15, one DPP row, all active) per row, lane sub holding dims
 // 8 sub .. +8 of the fp16 key in raw.  dst null: nothing stored (the lanes
@@ -168,7 +178,8 @@ __device__ __forceinline__ void idx_key_row_store(const u32x4 raw, void* dst, in
 }
 
 // Workgroup (tile, b) of the decode logits: positions [PPB tile, +PPB) of
-// token row b.  With NEWK, positions whose cache row is the slot of one of
+// token rows b .. b + NQ - 1, which are tokens of one request (sp.n a multiple
+// of NQ): the keys are loaded and converted once for all of them.  With NEWK, positions whose cache row is the slot of one of
 // the step's new keys get that key written to the row first, by this
 // workgroup, so that it reads exactly what a separate store launch before it
 // would have left there.  The standalone kernel (NEWK = false) runs the same
@@ -177,13 +188,14 @@ __device__ __forceinline__ void idx_key_row_store(const u32x4 raw, void* dst, in
 // from a struct, so that the compiler keeps knowing that the score stores
 // do not alias the key loads.  Kv is not restrict: with NEWK the same rows
 // are written through nk.dst, and read after the workgroup barrier.)
-template <bool KFP8, bool NEWK, int PPB>
+template <bool KFP8, bool NEWK, int PPB, int NQ>
 __device__ __forceinline__ void indexer_logits_body(
     const f16* __restrict__ Q, const void* Kv, const f16* __restrict__ W,
     const int32_t* __restrict__ block_table, const int32_t* __restrict__ seq_lens,
     float* __restrict__ score, uint32_t* __restrict__ hist, int64_t n_kv_rows, int max_blocks,
-    int page_shift, int max_kv, int hist8, int span, int tile, int b, const IdxNewKeys& nk) {
-  constexpr bool kSpan = KFP8 && PPB == kIdxPPB;  // only such launches ask for spans
+    int page_shift, int max_kv, int hist8, int span, int tile, int b, const IdxNewKeys& nk,
+    const IdxSpecRows& sp) {
+  constexpr bool kSpan = KFP8 && PPB == kIdxPPB && NQ == 1;  // only such launches ask for spans
   const int p_lo = tile * PPB;
   const int p_hi = min(p_lo + PPB, max_kv);
   // The block-table entries of the tile's pages are loaded beside seq_len
@@ -193,26 +205,43 @@ __device__ __forceinline__ void indexer_logits_body(
   constexpr int kBtRegs = (PPB + 2 + kNT - 1) / kNT;
   const int pg0 = p_lo >> page_shift;
   const int npg = ((p_hi - 1) >> page_shift) - pg0 + 1;
-  const int32_t* bt_row = block_table + (int64_t)b * max_blocks;
+  const int req = sp.n == 1 ? b : b / sp.n;
+  const int32_t* bt_row = block_table + (int64_t)req * max_blocks;
   int32_t btv[kBtRegs];
 #pragma unroll
   for (int k = 0; k < kBtRegs; k++) {
     const int i = (int)threadIdx.x + kNT * k;
     btv[k] = (i < npg && pg0 + i < max_blocks) ? bt_row[pg0 + i] : -1;
   }
-  const int seq_len = seq_lens[b];
+  // row b + q ends at seq0 + q; the last row has the longest context
+  const int seq0 = seq_lens[req] - (sp.n - 1) + (b - req * sp.n);
+  const int seq_len = seq0 + NQ - 1;
   float* srow = score + (int64_t)b * max_kv;
+  if (sp.n > 1) {
+#pragma unroll
+    for (int k = 0; k < kBtRegs; k++) {
+      const int pg = pg0 + (int)threadIdx.x + kNT * k;
+      // a page that begins in an earlier tile is that tile's to write
+      if (pg - pg0 < npg && pg < max_blocks && ((int64_t)pg << page_shift) >= p_lo)
+#pragma unroll
+        for (int q = 0; q < NQ; q++) sp.bt_out[(int64_t)(b + q) * max_blocks + pg] = btv[k];
+    }
+    if (tile == 0 && threadIdx.x < NQ) sp.sl_out[b + threadIdx.x] = seq0 + (int)threadIdx.x;
+  }
 
   // tiles wholly past the context only need the -inf padding
   if (p_lo >= seq_len) {
-    for (int i = p_lo + threadIdx.x; i < p_hi; i += blockDim.x) srow[i] = -INFINITY;
+#pragma unroll
+    for (int q = 0; q < NQ; q++)
+      for (int i = p_lo + threadIdx.x; i < p_hi; i += blockDim.x)
+        srow[(int64_t)q * max_kv + i] = -INFINITY;
     return;
   }
 
   __shared__ int32_t s_bt[PPB + 2];
   // level-1 counts of this workgroup's keys, two 16-bit bins per word (a
   // workgroup counts at most PPB keys)
-  __shared__ uint32_t s_hist[kTopkBins / 2];
+  __shared__ uint32_t s_hist[NQ * (kTopkBins / 2)];
   // fp8 span path: per wave, two stages of kIdxGroup staged blocks
   __shared__ __align__(16) uint8_t s_span[kSpan ? kIdxWaves * 2 * kIdxGroup * kIdxSpanSlot : 16];
   __shared__ int32_t s_new[NEWK ? 2 * kIdxMaxNew : 1];  // slots, then "this workgroup reads it"
@@ -223,7 +252,7 @@ __device__ __forceinline__ void indexer_logits_body(
     if (i < npg) s_bt[i] = btv[k];
   }
   if (hist != nullptr)
-    for (int i = threadIdx.x; i < kTopkBins / 2; i += blockDim.x) s_hist[i] = 0u;
+    for (int i = threadIdx.x; i < NQ * (kTopkBins / 2); i += blockDim.x) s_hist[i] = 0u;
   if constexpr (NEWK) {
     for (int i = threadIdx.x; i < nk.T; i += blockDim.x) {
       s_new[i] = nk.slot[i];
@@ -278,22 +307,24 @@ __device__ __forceinline__ void indexer_logits_body(
   // step s, group g, slot e -> dim 32s + 8g + e (fp16 keys) or
   // idx_fp8_piece(g) + 32 (s >> 1) + 8 (s & 1) + e (fp8 keys, whose two
   // 16-byte pieces per lane start at idx_fp8_piece(g) and 32 bytes later).
-  f16x8 qa[2][4];
-  const f16* qb = Q + (int64_t)b * kIdxHeads * kIdxHeadDim;
-#pragma unroll
-  for (int t = 0; t < 2; t++)
-#pragma unroll
-    for (int s = 0; s < 4; s++)
-      qa[t][s] = *reinterpret_cast<const f16x8*>(
-          qb + (16 * t + c) * kIdxHeadDim +
-          (KFP8 ? idx_fp8_piece(g) + 32 * (s >> 1) + 8 * (s & 1) : 32 * s + 8 * g));
+  f16x8 qa[NQ][2][4];
   // head weights of this lane's D rows: heads 4g + r and 16 + 4g + r
-  float wv[2][4];
+  float wv[NQ][2][4];
 #pragma unroll
-  for (int t = 0; t < 2; t++)
+  for (int q = 0; q < NQ; q++) {
+    const f16* qb = Q + (int64_t)(b + q) * kIdxHeads * kIdxHeadDim;
 #pragma unroll
-    for (int r = 0; r < 4; r++)
-      wv[t][r] = (float)W[(int64_t)b * kIdxHeads + 16 * t + 4 * g + r];
+    for (int t = 0; t < 2; t++) {
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+        qa[q][t][s] = *reinterpret_cast<const f16x8*>(
+            qb + (16 * t + c) * kIdxHeadDim +
+            (KFP8 ? idx_fp8_piece(g) + 32 * (s >> 1) + 8 * (s & 1) : 32 * s + 8 * g));
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        wv[q][t][r] = (float)W[(int64_t)(b + q) * kIdxHeads + 16 * t + 4 * g + r];
+    }
+  }
 
   // Row of the key this lane loads for block `blk` (-1: zero key).
   auto key_row = [&](int blk) -> int64_t {
@@ -312,30 +343,45 @@ __device__ __forceinline__ void indexer_logits_body(
   // [i*kIdxGroup, (i+1)*kIdxGroup) in that order.
   auto blk_of = [&](int stage, int j) { return (stage * kIdxGroup + j) * kIdxWaves + wave; };
 
-  // Score of one 16-key block for this lane's key (the same sum in the four
+  // Scores of one 16-key block for this lane's key (the same sum in the four
   // lanes g of a key: the butterfly only reorders commutative additions).
-  auto block_score = [&](const KeyFrag& f) {
-    float v = 0.f;
+  auto block_score = [&](const KeyFrag& f, float (&v)[NQ]) {
+    f16x8 kb[4];
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < 4; s++) kb[s] = key_operand<KFP8>(f, s);
 #pragma unroll
-      for (int s = 0; s < 4; s++) acc = mfma16x16x32(qa[t][s], key_operand<KFP8>(f, s), acc);
+    for (int q = 0; q < NQ; q++) {
+      v[q] = 0.f;
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        float d = acc[r];
-        if constexpr (KFP8) d *= f.scale;
-        v += relu_mfma(d) * wv[t][r];
+      for (int t = 0; t < 2; t++) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 4; s++) acc = mfma16x16x32(qa[q][t][s], kb[s], acc);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          float d = acc[r];
+          if constexpr (KFP8) d *= f.scale;
+          v[q] += relu_mfma(d) * wv[q][t][r];
+        }
       }
+      v[q] = xor16_sum(v[q]);
+      v[q] = xor32_sum(v[q]);
     }
-    v = xor16_sum(v);
-    v = xor32_sum(v);
-    return v;
   };
 
   // one key into the level-1 count of bin key >> 20
-  auto hist_count = [&](uint32_t key) {
-    atomicAdd(&s_hist[key >> 21], 1u << ((key >> 16) & 16));
+  auto hist_count = [&](int q, uint32_t key) {
+    atomicAdd(&s_hist[q * (kTopkBins / 2) + (key >> 21)], 1u << ((key >> 16) & 16));
+  };
+  // The rows' scores of the key at position p (p inside the row): every lane
+  // of a key stores the same bits, one lane counts it.
+  auto put = [&](int p, const float (&v)[NQ]) {
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      const bool live = p < seq0 + q;
+      srow[(int64_t)q * max_kv + p] = live ? v[q] : -INFINITY;
+      if (hist != nullptr && g == 0 && live) hist_count(q, mono_key(v[q]));
+    }
   };
 
   // fp8 rows, in a launch that asks for it (idx_span_launch), in pages of
@@ -398,12 +444,13 @@ __device__ __forceinline__ void indexer_logits_body(
         f.v[1] = *reinterpret_cast<const u32x4_a4*>(rw + idx_fp8_piece(g) + 32);
         f.v[2] = f.v[3] = (u32x4){0u, 0u, 0u, 0u};
         f.scale = *reinterpret_cast<const float*>(rw + 128);
-        float v = block_score(f);
-        if (!okc[j]) v = 0.f;
-        const int p = p_lo + 16 * blk_of(st, j) + c;
-        const bool live = p < seq_len;
-        srow[p] = live ? v : -INFINITY;
-        if (hist != nullptr && g == 0 && live) hist_count(mono_key(v));
+        float v[NQ];
+        block_score(f, v);
+        if (!okc[j]) {
+#pragma unroll
+          for (int q = 0; q < NQ; q++) v[q] = 0.f;
+        }
+        put(p_lo + 16 * blk_of(st, j) + c, v);
       }
       if (st + 1 < n_groups) {
 #pragma unroll
@@ -439,12 +486,13 @@ __device__ __forceinline__ void indexer_logits_body(
       }
 #pragma unroll
       for (int j = 0; j < kIdxGroup; j++) {
-        float v = block_score(cur[j]);
-        if (rcur[j] < 0) v = 0.f;  // unmapped row: the zero key's score
-        const int p = p_lo + 16 * blk_of(st, j) + c;
-        const bool live = p < seq_len;
-        srow[p] = live ? v : -INFINITY;
-        if (hist != nullptr && g == 0 && live) hist_count(mono_key(v));
+        float v[NQ];
+        block_score(cur[j], v);
+        if (rcur[j] < 0) {  // unmapped row: the zero key's score
+#pragma unroll
+          for (int q = 0; q < NQ; q++) v[q] = 0.f;
+        }
+        put(p_lo + 16 * blk_of(st, j) + c, v);
       }
       if (st + 1 < n_groups) {
 #pragma unroll
@@ -470,16 +518,9 @@ __device__ __forceinline__ void indexer_logits_body(
       for (int j = 0; j < kIdxGroup; j++) {
         const int p0 = p_lo + 16 * blk_of(st, j);
         if (p0 < p_hi) {
-          const float v = block_score(cur[j]);
-          const int p = p0 + c;
-          if (g == 0 && p < p_hi) {
-            if (p < seq_len) {
-              srow[p] = v;
-              if (hist != nullptr) hist_count(mono_key(v));
-            } else {
-              srow[p] = -INFINITY;
-            }
-          }
+          float v[NQ];
+          block_score(cur[j], v);
+          if (g == 0 && p0 + c < p_hi) put(p0 + c, v);
         }
       }
       if (st + 1 < n_groups) {
@@ -496,17 +537,18 @@ __device__ __forceinline__ void indexer_logits_body(
     // adjacent bins go in one 64-bit atomic (half the atomics); no carry
     // crosses from the low count into the high one, since a row's counts
     // stay below 2^32.
+    // The rows' histograms are consecutive, here and in memory.
     if (hist8) {
       unsigned long long* hrow2 =
           reinterpret_cast<unsigned long long*>(hist + (int64_t)b * kTopkBins);
-      for (int i = threadIdx.x; i < kTopkBins / 2; i += blockDim.x) {
+      for (int i = threadIdx.x; i < NQ * (kTopkBins / 2); i += blockDim.x) {
         const uint32_t w2 = s_hist[i];
         const unsigned long long lo = w2 & 0xffffu, hi = w2 >> 16;
         if (w2) atomicAdd(hrow2 + i, lo | (hi << 32));
       }
     } else {  // a hist base that is not 8-byte aligned: one bin per atomic
       uint32_t* hrow = hist + (int64_t)b * kTopkBins;
-      for (int i = threadIdx.x; i < kTopkBins; i += blockDim.x) {
+      for (int i = threadIdx.x; i < NQ * kTopkBins; i += blockDim.x) {
         const uint32_t n = (s_hist[i >> 1] >> (16 * (i & 1))) & 0xffffu;
         if (n) atomicAdd(&hrow[i], n);
       }
@@ -514,12 +556,13 @@ __device__ __forceinline__ void indexer_logits_body(
   }
 }
 
-template <bool KFP8, bool NEWK, int PPB>
+template <bool KFP8, bool NEWK, int PPB, int NQ>
 __device__ __forceinline__ void indexer_logits_block(const IdxDecArgs& a, int tile, int b,
-                                                     const IdxNewKeys& nk) {
-  indexer_logits_body<KFP8, NEWK, PPB>(a.Q, a.Kv, a.W, a.block_table, a.seq_lens, a.score, a.hist,
-                                  a.n_kv_rows, a.max_blocks, a.page_shift, a.max_kv, a.hist8,
-                                  a.span, tile, b, nk);
+                                                     const IdxNewKeys& nk,
+                                                     const IdxSpecRows& sp) {
+  indexer_logits_body<KFP8, NEWK, PPB, NQ>(
+      a.Q, a.Kv, a.W, a.block_table, a.seq_lens, a.score, a.hist, a.n_kv_rows, a.max_blocks,
+      a.page_shift, a.max_kv, a.hist8, a.span, tile, b, nk, sp);
 }
 
 }  // namespace mi355dsa

@@ -23,7 +23,9 @@ second stream for the latent write and step 3 (which do not feed the
 indexer) made a captured decode layer slower (106.7 vs 96.0 us at 180k
 context), the cross-stream join costing more than the overlap hides.
 Speculative decode rows (B tokens over B / next_n requests) are expanded per
-token as the reference does (triton_mla.py:267-279).
+token as the reference does (triton_mla.py:267-279); on the fused path the
+logits launch does it (mi355_dsa_decode_layer_indexer_spec): the four tensor
+ops it replaces cost a launch each, 16.5 of 115 us per layer at 24 x 2 tokens.
 
 Prefill (sparse_attn_indexer.py:641-881 without tensor-parallel key
 sharding, then triton_mla.py:380-492 _forward_mha_sparse): per request and
@@ -193,19 +195,28 @@ class DsaLayer:
         B, R = q.shape[0], seq_lens.shape[0]
         bt = block_table.to(torch.int32)
         sl = seq_lens.to(torch.int32)
+        n = 1
         if B != R:  # spec-as-decode: per-token rows (triton_mla.py:267-279)
             assert B % R == 0, f"non-uniform decode batch: {B} tokens, {R} requests"
             n = B // R
+        hist = None
+        fusable = kv_c is not None and self._fusable(q, kv_c, k_pe, idx_k, slot_mapping)
+        step = fusable and self._indexer_fusable(q, idx_q, idx_w)
+        spec = None
+        if step and n > 1 and bt.shape[1] > 0:  # the logits launch expands the rows
+            spec = (torch.empty(B, bt.shape[1], dtype=torch.int32, device=q.device),
+                    torch.empty(B, dtype=torch.int32, device=q.device))
+        elif B != R:
             offs = torch.arange(n, device=q.device, dtype=torch.int32)
             sl = (sl.unsqueeze(1) - (n - 1) + offs).reshape(-1).contiguous()
             bt = bt.repeat_interleave(n, dim=0).contiguous()
-        hist = None
-        fusable = kv_c is not None and self._fusable(q, kv_c, k_pe, idx_k, slot_mapping)
-        if fusable and self._indexer_fusable(q, idx_q, idx_w):
+        if step:
             # one launch: both cache writes and the indexer logits; then the
             # top-k (leaving the layer's histogram zero) with q_latent beside it
             ql, idx = self._indexer_step(q, idx_q, idx_w, bt, sl, kv_c, k_pe, idx_k,
-                                         slot_mapping)
+                                         slot_mapping, spec)
+            if spec is not None:
+                bt, sl = spec
         else:
             if fusable:
                 # one launch: q_latent, both cache writes and the histogram clear
@@ -282,11 +293,14 @@ class DsaLayer:
             self._hists[key] = h
         return h[:B]
 
-    def _indexer_step(self, q, idx_q, idx_w, bt, sl, kv_c, k_pe, idx_k, slot_mapping):
+    def _indexer_step(self, q, idx_q, idx_w, bt, sl, kv_c, k_pe, idx_k, slot_mapping,
+                      spec=None):
         """mi355_dsa_decode_layer_indexer (the latent and indexer-K writes and
         the indexer logits with the histogram, one launch), then
         mi355_dsa_decode_layer_topk (the top-k, which leaves the histogram
-        zero, with q_latent run beside its select).  Returns (q_latent, idx)."""
+        zero, with q_latent run beside its select).  Returns (q_latent, idx).
+        spec: (bt [B, max_blocks], sl [B]) that the launch fills from bt / sl,
+        which are then per request (mi355_dsa_decode_layer_indexer_spec)."""
         B, H = q.shape[0], q.shape[1]
         q = _rows8(q)
         ql = torch.empty(B, H, 576, dtype=torch.float16, device=q.device)
@@ -317,14 +331,20 @@ class DsaLayer:
         uk = self.w.uk_t
         st = _stream(q)
         with torch.cuda.device(q.device):
-            _lib.call("mi355_dsa_decode_layer_indexer", B, lat.data_ptr(), int(fp8), kv_rows,
+            name, extra = "mi355_dsa_decode_layer_indexer", ()
+            if spec is not None:
+                name += "_spec"
+                extra = (B // sl.shape[0], spec[0].data_ptr(), spec[1].data_ptr())
+            _lib.call(name, B, lat.data_ptr(), int(fp8), kv_rows,
                       kv_c.data_ptr(), kv_c.stride(0), k_pe.data_ptr(), k_pe.stride(0),
                       int(kv_c.dtype == torch.bfloat16), slot.data_ptr(),
                       int(slot.dtype == torch.int64), ikc.data_ptr(), int(ik_fp8), ik_rows,
                       ik.data_ptr(), islot.data_ptr(), score.data_ptr(), B, max_kv,
                       iq.data_ptr(), iw.data_ptr(), page, bt.data_ptr(), bt.shape[1],
-                      sl.data_ptr(), hist.data_ptr(), st)
+                      sl.data_ptr(), hist.data_ptr(), *extra, st)
             self.last_score = score
+            if spec is not None:
+                sl = spec[1]
             _lib.call("mi355_dsa_decode_layer_topk", idx.data_ptr(), score.data_ptr(),
                       sl.data_ptr(), hist.data_ptr(), B, max_kv, self.topk, ws.data_ptr(),
                       ws_bytes, ql.data_ptr(), ql.stride(0), ql.stride(1), q.data_ptr(),

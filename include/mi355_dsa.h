@@ -242,6 +242,23 @@ int mi355_dsa_decode_layer_indexer(
     void* stream);
 
 /*
+ * The same for a speculative step of n >= 2 tokens per request: B tokens of
+ * B / n requests (token j of request r is row r n + j), block_table
+ * [B / n, max_blocks] and seq_lens [B / n] per request, counting the step's
+ * tokens.  Row r n + j covers seq_lens[r] - (n - 1) + j positions.  Also
+ * writes the per-token tables that the following calls take: bt_out
+ * [B, max_blocks] and sl_out [B].  max_kv must be max_blocks pages.  Results
+ * equal, bit for bit, mi355_dsa_decode_layer_indexer on the expanded tables.
+ */
+int mi355_dsa_decode_layer_indexer_spec(
+    int T, void* kv_cache, int kv_fp8, int64_t kv_rows, const void* kv_c, int64_t kv_c_stride,
+    const void* k_pe, int64_t k_pe_stride, int in_bf16, const void* slot_mapping, int slot_i64,
+    void* idx_cache, int idx_fp8, int64_t idx_rows, const void* idx_k, const int32_t* idx_slot,
+    float* score, int B, int max_kv, const void* idx_q, const void* idx_w, int idx_page_size,
+    const int32_t* block_table, int max_blocks, const int32_t* seq_lens, int32_t* hist, int n,
+    int32_t* bt_out, int32_t* sl_out, void* stream);
+
+/*
  * Indexer logits (decode and generic path):
  *   score[b,p] = sum_h relu(q[b,h,:] . K[row(b,p),:]) * w[b,h]   (p < seq_len[b])
  *   score[b,p] = -inf                                          (seq_len[b] <= p < max_kv)

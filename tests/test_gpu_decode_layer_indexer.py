@@ -108,6 +108,43 @@ def test_indexer_step_equals_separate_calls(pkg, dev, case):
         assert not L2._zero_hist(B, dev).any()
 
 
+SPEC_CASES = [
+    # B tokens, tokens per request, fp8 latent, fp8 index keys, context lengths of the requests
+    (8, 2, True, False, [5000, 2600, 4097, 1]),     # 128 positions per workgroup; an empty row
+    (9, 3, True, True, [3000, 2049, 700]),          # odd count: one row per workgroup
+    (48, 2, False, True, [1000 + 170 * r for r in range(24)]),     # 512 positions
+    (64, 4, False, False, [9999 - 301 * r for r in range(16)]),    # 1024 positions
+    (64, 2, False, True, [17003 + 31 * r for r in range(32)]),     # 1024, staged spans
+]
+
+
+@pytest.mark.parametrize("case", SPEC_CASES, ids=[f"B{c[0]}n{c[1]}-{'fp8' if c[3] else 'f16'}idx"
+                                                  for c in SPEC_CASES])
+def test_spec_step_equals_expanded_rows(pkg, dev, case):
+    """Per-request tables expanded by the logits launch: the same bits in the
+    caches, scores, top-k and q_latent as the step on per-token tables, which
+    are also what the launch writes out."""
+    (m, ops, w, lat0, ik0, q, idx_q, idx_w, kv_c, k_pe, idx_k, bt, sl,
+     slot) = _case(pkg, dev, case, seed=sum(case[4]) + case[0])
+    B, n = case[:2]
+    L1 = m.DsaLayer(w, lat0.clone(), ik0.clone())
+    ql1, idx1 = L1._indexer_step(q, idx_q, idx_w, bt, sl, kv_c, k_pe, idx_k, slot)
+    L2 = m.DsaLayer(w, lat0.clone(), ik0.clone())
+    for _ in range(2):
+        spec = (torch.full_like(bt, -9), torch.full_like(sl, -9))
+        ql2, idx2 = L2._indexer_step(q, idx_q, idx_w, bt[::n].contiguous(),
+                                     torch.tensor(case[4], dtype=torch.int32, device=dev), kv_c,
+                                     k_pe, idx_k, slot, spec)
+        torch.cuda.synchronize()
+        assert torch.equal(spec[0], bt) and torch.equal(spec[1], sl)
+        assert torch.equal(L1.latent_cache.view(torch.uint8), L2.latent_cache.view(torch.uint8))
+        assert torch.equal(L1.idx_k_cache.view(torch.uint8), L2.idx_k_cache.view(torch.uint8))
+        assert torch.equal(L1.last_score.view(torch.int32), L2.last_score.view(torch.int32))
+        assert torch.equal(idx1, idx2)
+        assert torch.equal(ql1.view(torch.int16), ql2.view(torch.int16))
+        assert not L2._zero_hist(B, dev).any()
+
+
 def test_indexer_step_histogram(pkg, lib, dev):
     """The fused launch's histogram (before the top-k consumes it) equals the
     standalone logits launch's."""
