@@ -68,6 +68,7 @@ struct MlaParams {
   // dims writes 32 contiguous bytes
   f16* part_o;
   float* part_ml;  // [B, H, S, 2]   per-split (m_s, l_s)
+  int share;  // dense: splits divided by the lengths (dense_share)
   int B, n_head, topk, max_blocks, page_size, n_splits;
   int page_shift;  // log2(page_size) when it is a power of two, else -1
   int64_t n_kv_rows;
@@ -1534,22 +1535,116 @@ __device__ __forceinline__ float hw_pv_f16(const f32x16& s, float ml, uint32_t s
   return ls;
 }
 
+constexpr int kMergeMaxSplits = 128;  // key splits of one token at most
+
+// Dense decode, split contexts: the B * S split slots go to the tokens by their
+// lengths, kps keys each (a multiple of the tile), the smallest kps tried that
+// needs no more slots and no more than kMergeMaxSplits per token, and at most
+// the equal split of the whole width, which always fits.  Every wave that needs
+// the division computes it from seq_lens (B <= 128 tokens, two per lane): the
+// host does not know the lengths.  With one split count for all tokens, 4
+// requests of 32k, 26k, 20k and 14k left 28 % of the workgroups without keys
+// (attention 37.0 -> 33.4 us; whole calls, ragged to a quarter of the longest,
+// 64 heads: 4 x 32k 46.9 -> 44.3 us, 2 x 128k 76.6 -> 69.4; 32 heads, 8 x 32k
+// 59.8 -> 55.2).  Taken above kMergeBatch splits: below that more tokens share
+// the chip, the lengths even out over it and the division costs what it saves
+// (16 x 16k ragged 63.6 / 60.5, 40 x 6500 ragged 64.3 / 65.8, 48 x 5000 equal
+// 72.3 / 74.2).
+struct DenseShare {
+  int kps;
+  int n[2], off[2];  // of tokens lane and 64 + lane: splits, first slot
+  __device__ __forceinline__ int n_of(int b) const {
+    const int lo = __builtin_amdgcn_readlane(n[0], b & 63);
+    const int hi = __builtin_amdgcn_readlane(n[1], b & 63);
+    return b < 64 ? lo : hi;
+  }
+  __device__ __forceinline__ int off_of(int b) const {
+    const int lo = __builtin_amdgcn_readlane(off[0], b & 63);
+    const int hi = __builtin_amdgcn_readlane(off[1], b & 63);
+    return b < 64 ? lo : hi;
+  }
+};
+
+__device__ __forceinline__ DenseShare dense_share(const int32_t* seq_lens, int B, int width, int S) {
+  const int lane = threadIdx.x & 63;
+  int len[2], total = 0, longest = 0;
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const int b = lane + 64 * j;
+    len[j] = b < B ? max(0, min(width, seq_lens[b])) : 0;
+    total += (len[j] + kPfTileKeys - 1) / kPfTileKeys;  // in tiles: no overflow
+    longest = max(longest, len[j]);
+  }
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) {
+    total += __shfl_xor(total, m);
+    longest = max(longest, __shfl_xor(longest, m));
+  }
+  const int slots = B * S;
+  const int most = (width + S * kPfTileKeys - 1) / (S * kPfTileKeys);  // tiles, the equal split
+  int kt = max((total + slots - 1) / slots,
+               (longest + kMergeMaxSplits * kPfTileKeys - 1) / (kMergeMaxSplits * kPfTileKeys));
+  kt = min(max(__builtin_amdgcn_readfirstlane(kt), 1), most);
+  DenseShare r;
+  int incl[2];
+  while (true) {
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      r.n[j] = (len[j] + kt * kPfTileKeys - 1) / (kt * kPfTileKeys);
+      incl[j] = r.n[j];
+    }
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+      const int u0 = __shfl_up(incl[0], m), u1 = __shfl_up(incl[1], m);
+      if (lane >= m) {
+        incl[0] += u0;
+        incl[1] += u1;
+      }
+    }
+    const int n0 = __builtin_amdgcn_readlane(incl[0], 63);
+    incl[1] += n0;
+    if (kt >= most || __builtin_amdgcn_readlane(incl[1], 63) <= slots) break;
+    kt = min(kt + max(kt >> 4, 1), most);
+  }
+  r.kps = kt * kPfTileKeys;
+  r.off[0] = incl[0] - r.n[0];
+  r.off[1] = incl[1] - r.n[1];
+  return r;
+}
+
 __global__ void __launch_bounds__(kHwThreads, 1) mla_hw_f16_kernel(MlaParams p) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   HwSmem& sh = *reinterpret_cast<HwSmem*>(smem_raw);
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int hw = w & 1, kw = w >> 1;
   const int c = lane & 31, hf = lane >> 5;
-  const int b = token_of(blockIdx.x, gridDim.x);
+  int b = token_of(blockIdx.x, gridDim.x);
   const int hbase = blockIdx.y * 64;
-  const int split = blockIdx.z;
+  int split = blockIdx.z;
+  int kps = 0;
+  int64_t ps0 = 0;  // the split's partial of head h: ps0 + h * ps_h
+  int ps_h = p.n_splits;
+  if (p.share) {
+    const DenseShare ds = dense_share(p.seq_lens, p.B, p.topk, p.n_splits);
+    const int slot = (int)(blockIdx.x + gridDim.x * blockIdx.z);
+    const uint64_t in0 = __ballot(slot >= ds.off[0] && slot < ds.off[0] + ds.n[0]);
+    const uint64_t in1 = __ballot(slot >= ds.off[1] && slot < ds.off[1] + ds.n[1]);
+    if ((in0 | in1) == 0) return;  // more slots than splits
+    b = in0 != 0 ? __builtin_ctzll(in0) : 64 + __builtin_ctzll(in1);
+    split = slot - ds.off_of(b);
+    kps = ds.kps;
+    ps_h = ds.n_of(b);
+    ps0 = (int64_t)ds.off_of(b) * p.n_head + split;
+  } else {
+    ps0 = (int64_t)b * p.n_head * p.n_splits + split;
+  }
   const uint8_t* kv = reinterpret_cast<const uint8_t*>(p.kv);
   const int seq_len = p.seq_lens[b];
   constexpr float kLog2e = 1.4426950408889634f;
 
   const int n_keys = p.idx ? p.topk : max(0, min(p.topk, seq_len));
-  const int kps = ((n_keys + p.n_splits - 1) / p.n_splits + kPfTileKeys - 1) / kPfTileKeys *
-                  kPfTileKeys;
+  if (kps == 0)
+    kps = ((n_keys + p.n_splits - 1) / p.n_splits + kPfTileKeys - 1) / kPfTileKeys * kPfTileKeys;
   const int k_lo = min(split * kps, n_keys);
   const int k_hi = min(k_lo + kps, n_keys);
 
@@ -1710,7 +1805,7 @@ __global__ void __launch_bounds__(kHwThreads, 1) mla_hw_f16_kernel(MlaParams p) 
   const int h = hbase + 32 * hw + c;
   const int64_t bh = (int64_t)b * p.n_head + h;
   const bool final_out = p.n_splits == 1;
-  const int64_t ps = bh * p.n_splits + split;
+  const int64_t ps = ps0 + (int64_t)h * ps_h;
   auto finish = [&](auto tc) {  // tiles t and t + 1, one 64-dim chunk
     constexpr int t = decltype(tc)::value;
     u32x2 q2[2][4];  // dims 32 (t + tt) + 8 a + 4 hf .. +3
@@ -2084,7 +2179,6 @@ __global__ void __launch_bounds__(kFewThreads, FP8 ? 3 : 2) sparse_mla_few_kerne
 // One workgroup per (token, head), 128 threads x 4 dims.  Splits are taken
 // 16 at a time with every (m, l) pair and partial row of the batch loaded
 // together (one memory latency per batch), combined online across batches.
-constexpr int kMergeMaxSplits = 128;
 constexpr int kMergeBatch = 16;
 
 // Merged outputs of NU (token, head, position) units: unit j is (bh[j], i[j]),
@@ -2093,15 +2187,15 @@ constexpr int kMergeBatch = 16;
 // (m[j], l[j]) for the lse.  The loads of all NU units in a batch of splits
 // are issued before any of them is combined; each unit's arithmetic is the
 // same whatever NU is.
+// merge_range sums splits [s_lo, s_hi) without the division.
 template <int NU>
-__device__ __forceinline__ void merge_units(const f16* __restrict__ part_o,
+__device__ __forceinline__ void merge_range(const f16* __restrict__ part_o,
                                             const float* __restrict__ part_ml,
-                                            const int64_t (&bh)[NU], int n_splits,
-                                            const int (&i)[NU], f16x4 (&o4)[NU], float (&m)[NU],
-                                            float (&l)[NU]) {
+                                            const int64_t (&bh)[NU], int n_splits, int s_lo,
+                                            int s_hi, const int (&i)[NU], f32x4 (&acc)[NU],
+                                            float (&m)[NU], float (&l)[NU]) {
   const f32x2* ml[NU];
   const f16* po[NU];
-  f32x4 acc[NU];
 #pragma unroll
   for (int j = 0; j < NU; j++) {
     ml[j] = reinterpret_cast<const f32x2*>(part_ml + bh[j] * n_splits * 2);
@@ -2110,7 +2204,7 @@ __device__ __forceinline__ void merge_units(const f16* __restrict__ part_o,
     l[j] = 0.f;
     acc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
   }
-  for (int s0 = 0; s0 < n_splits; s0 += kMergeBatch) {
+  for (int s0 = s_lo; s0 < s_hi; s0 += kMergeBatch) {
     f32x2 mlv[NU][kMergeBatch];
     f16x4 hv[NU][kMergeBatch];
 #pragma unroll
@@ -2118,8 +2212,8 @@ __device__ __forceinline__ void merge_units(const f16* __restrict__ part_o,
 #pragma unroll
       for (int u = 0; u < kMergeBatch; u++) {
         const int s = s0 + u;
-        mlv[j][u] = (s < n_splits) ? ml[j][s] : (f32x2){-1e30f, 0.f};
-        hv[j][u] = (s < n_splits) ? *reinterpret_cast<const f16x4*>(po[j] + (int64_t)s * kValueDim)
+        mlv[j][u] = (s < s_hi) ? ml[j][s] : (f32x2){-1e30f, 0.f};
+        hv[j][u] = (s < s_hi) ? *reinterpret_cast<const f16x4*>(po[j] + (int64_t)s * kValueDim)
                                   : (f16x4){0, 0, 0, 0};
       }
     }
@@ -2146,6 +2240,16 @@ __device__ __forceinline__ void merge_units(const f16* __restrict__ part_o,
       m[j] = mb;
     }
   }
+}
+
+template <int NU>
+__device__ __forceinline__ void merge_units(const f16* __restrict__ part_o,
+                                            const float* __restrict__ part_ml,
+                                            const int64_t (&bh)[NU], int n_splits,
+                                            const int (&i)[NU], f16x4 (&o4)[NU], float (&m)[NU],
+                                            float (&l)[NU]) {
+  f32x4 acc[NU];
+  merge_range<NU>(part_o, part_ml, bh, n_splits, 0, n_splits, i, acc, m, l);
 #pragma unroll
   for (int j = 0; j < NU; j++) {
     const float inv = (l[j] > 0.f) ? 1.f / l[j] : 0.f;
@@ -2179,6 +2283,65 @@ __global__ void __launch_bounds__(128) sparse_mla_merge_kernel(
   merge_units<1>(part_o, part_ml, bh, n_splits, i, o4, m, l);
   *reinterpret_cast<f16x4*>(O + bh[0] * kValueDim + merge_dim(i[0])) = o4[0];
   if (threadIdx.x == 0) LSE[bh[0]] = (l[0] > 0.f) ? (m[0] + logf(l[0])) : empty_lse;
+}
+
+// The merge of a dense call: 4 x 128 threads per (token, head), group g taking
+// the g-th quarter of the splits, so that the batches of a token with up to 128
+// splits run side by side (a memory latency each: 4 x 8k, 63 splits, 8.1 -> 5.4
+// us); the groups' sums are combined in LDS in group order.  For calls of more
+// than kMergeBatch splits, at most 15 tokens x 64 heads; with more units the
+// larger workgroups cost more than the one batch (48 tokens: 7.3 -> 31 us).
+// share_lens: the sequence lengths where the splits were divided by
+// dense_share, else null.
+constexpr int kDenseMergeGroups = 4;
+__global__ void __launch_bounds__(128 * kDenseMergeGroups) dense_mla_merge_kernel(
+    const f16* __restrict__ part_o, const float* __restrict__ part_ml, f16* __restrict__ O,
+    float* __restrict__ LSE, int n_splits, float empty_lse, int n_head,
+    const int32_t* __restrict__ share_lens, int B, int width) {
+  __shared__ f32x4 s_acc[kDenseMergeGroups - 1][128];
+  __shared__ float s_m[kDenseMergeGroups], s_l[kDenseMergeGroups];
+  const int64_t bh0 = blockIdx.x;
+  int64_t unit[1] = {bh0};  // its partials: n_splits rows from row unit * n_splits
+  if (share_lens != nullptr) {
+    const DenseShare ds = dense_share(share_lens, B, width, n_splits);
+    const int b = (int)(bh0 / n_head);
+    const int64_t base = (int64_t)ds.off_of(b) * n_head;
+    part_o += base * kValueDim;
+    part_ml += base * 2;
+    unit[0] = bh0 - (int64_t)b * n_head;
+    n_splits = ds.n_of(b);
+  }
+  const int g = threadIdx.x >> 7;
+  const int i[1] = {(int)threadIdx.x & 127};
+  const int per = (n_splits + kDenseMergeGroups - 1) / kDenseMergeGroups;
+  const int s_lo = min(g * per, n_splits), s_hi = min(s_lo + per, n_splits);
+  f32x4 acc[1];
+  float m[1], l[1];
+  merge_range<1>(part_o, part_ml, unit, n_splits, s_lo, s_hi, i, acc, m, l);
+  if (g > 0) s_acc[g - 1][i[0]] = acc[0];
+  if (i[0] == 0) {
+    s_m[g] = m[0];
+    s_l[g] = l[0];
+  }
+  __syncthreads();
+  if (g > 0) return;
+  float M = m[0];
+#pragma unroll
+  for (int k = 1; k < kDenseMergeGroups; k++) M = fmaxf(M, s_m[k]);
+  float w = l[0] > 0.f ? expf(m[0] - M) : 0.f, L = l[0] * w;
+  f32x4 o = acc[0] * w;
+#pragma unroll
+  for (int k = 1; k < kDenseMergeGroups; k++) {
+    w = s_l[k] > 0.f ? expf(s_m[k] - M) : 0.f;
+    L += s_l[k] * w;
+    o += s_acc[k - 1][i[0]] * w;
+  }
+  const float inv = (L > 0.f) ? 1.f / L : 0.f;
+  f16x4 o4;
+#pragma unroll
+  for (int r = 0; r < 4; r++) o4[r] = (f16)(o[r] * inv);
+  *reinterpret_cast<f16x4*>(O + bh0 * kValueDim + merge_dim(i[0])) = o4;
+  if (i[0] == 0) LSE[bh0] = (L > 0.f) ? (M + logf(L)) : empty_lse;
 }
 
 // Fused epilogue of a decode layer step: the split merge and the o @ W_UV
@@ -2344,8 +2507,11 @@ static int dense_splits(int B, int n_head, int max_kv) {
 // dense 4 x 4k 24.8 / 26.2; 16 tiles, 64 tokens, 58.0 / 57.5; dense 4 x 32k ragged
 // 47.9 / 45.5; 64 tiles, 200 tokens, 134.3 / 116.6).
 constexpr int kHwMinTiles = 16;
+static bool use_hw_f16(int topk, int n_splits) {
+  return (topk + n_splits - 1) / n_splits > (kHwMinTiles - 1) * kPfTileKeys;
+}
 static int launch_attn_f16(const MlaParams& prm, dim3 grid, hipStream_t st) {
-  if ((prm.topk + prm.n_splits - 1) / prm.n_splits > (kHwMinTiles - 1) * kPfTileKeys) {
+  if (use_hw_f16(prm.topk, prm.n_splits)) {
     const int rc = reserve_lds(reinterpret_cast<const void*>(mla_hw_f16_kernel), sizeof(HwSmem),
                                "mla_hw_f16");
     if (rc) return rc;
@@ -2468,6 +2634,7 @@ static int mla_decode_impl(
   // read a zero row that keeps score 0 (:970-992, :762-771)
   prm.zero_unresolved = (dense || !(B >= 32 && n_head <= 16)) ? 1 : 0;
   prm.xcd_map = 0;
+  prm.share = 0;
   hipStream_t st = as_stream(stream);
 
   if (dense) {
@@ -2481,11 +2648,18 @@ static int mla_decode_impl(
       prm.part_o = reinterpret_cast<f16*>(workspace);
       prm.part_ml = reinterpret_cast<float*>(prm.part_o + (size_t)B * n_head * S * kValueDim);
     }
+    prm.share = S > kMergeBatch && use_hw_f16(topk, S);
     int rc = launch_attn_f16(prm, dim3(B, (n_head + 63) / 64, S), st);
     if (rc != MI355_DSA_OK || S == 1) return rc;
-    sparse_mla_merge_kernel<<<dim3((unsigned)((int64_t)B * n_head)), 128, 0, st>>>(
-        prm.part_o, prm.part_ml, prm.o, prm.lse, S, prm.empty_lse, n_head, 0);
-    return check_launch("sparse_mla_merge");
+    if (S <= kMergeBatch) {
+      sparse_mla_merge_kernel<<<dim3((unsigned)((int64_t)B * n_head)), 128, 0, st>>>(
+          prm.part_o, prm.part_ml, prm.o, prm.lse, S, prm.empty_lse, n_head, 0);
+      return check_launch("sparse_mla_merge");
+    }
+    dense_mla_merge_kernel<<<dim3((unsigned)((int64_t)B * n_head)), 128 * kDenseMergeGroups, 0,
+                             st>>>(prm.part_o, prm.part_ml, prm.o, prm.lse, S, prm.empty_lse,
+                                   n_head, prm.share ? seq_lens : nullptr, B, topk);
+    return check_launch("dense_mla_merge");
   }
 
   const DecodePlan plan = plan_decode(B, n_head, topk, kv_fp8);

@@ -66,6 +66,27 @@ def test_dense_decode(ops, dev, case):
         check(o, lse, r16, l16)
 
 
+SHARED = [
+    # H, seqs: the split slots go to the tokens by length (16 tiles or more per slot)
+    (32, [12000, 0, 1, 31, 33, 480, 512, 513, 5000, 64, 2000, 11999]),
+    (96, [20300, 7, 300]),              # two 64-head groups
+    (32, [21100, 40, 40, 0, 40, 33]),   # one token takes more splits than the equal share
+    (64, [30000, 30000]),               # equal lengths: the equal split
+]
+
+
+@pytest.mark.parametrize("H,seqs", SHARED, ids=[f"B{len(s)}H{h}" for h, s in SHARED])
+def test_splits_by_length(ops, dev, H, seqs):
+    page = 64
+    mb = (max(seqs) + page - 1) // page
+    q, kv, bt, seq = make(20 + len(seqs), len(seqs), H, mb + 8, page, seqs, mb)
+    bt[0, 3] = -1  # an unresolvable page: zero keys
+    o, lse = run(ops, dev, q, kv, bt, seq)
+    assert not torch.isnan(o).any() and not torch.isnan(lse).any()
+    ro, rl = O.mla_decode(q, kv, bt, seq, SCALE)
+    check(o, lse, ro, rl)
+
+
 def test_unresolvable_rows_are_zero_keys(ops, dev):
     """Positions below seq_len on a -1 block are zero keys with score 0, as
     in the reference (sm70_mla_decode.cu:762-771)."""
