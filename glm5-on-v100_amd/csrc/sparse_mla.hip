@@ -1879,6 +1879,11 @@ __global__ void __launch_bounds__(kHwThreads, 1) mla_hw_f16_kernel(MlaParams p) 
 // transpose reads are free of bank conflicts, and a DMA instruction fetches a
 // block of 16 keys, 64 contiguous bytes per four lanes.  fp8 scales follow,
 // tile-major (tile t of key r at 64 t + 4 r).
+// Bound: the gather's latency (a tile's rows are one round trip, hidden only by
+// the other workgroups of the CU) and, for fp8 rows, the conversions of every row
+// for 16 heads' products.  2048 tokens x 16 heads: fp8 749 us with the 64-head
+// kernel -> 393, fp16 595 -> 511; 32 tokens x 16 heads fp16 36.8 -> 30.0
+// us a call (the kernel before kept one tile in flight).
 // ---------------------------------------------------------------------------
 constexpr int kFewThreads = 256;
 constexpr int kFewTile = 64;     // keys per tile

@@ -10,7 +10,7 @@ decode plan can pick for an fp8 cache:
            and the split merge (the headline configuration)
   dma_h16  B=3, 16 heads, top-512: the LDS-DMA split decode, one head group
   pipe     B=16, 64 heads: the 64-head pipelined kernel with 16 key splits
-  regst    B=2, 16 heads, top-17408: the register-staged split decode
+  regst    B=2, 16 heads, top-17408: the 16-head kernel, split (lists too long for the DMA decode)
   prefill  B=256, 64 heads: the pipelined prefill kernel, one split
   c4       the last 4096-token launch of the 64k causal prefill
 
