@@ -180,6 +180,26 @@ def test_decode_topk_one_launch_workspace(pkg, dev):
         assert torch.equal(idx.cpu(), cref.topk_rows(s, seq_t, 2048))
 
 
+@pytest.mark.parametrize("W", [4096, 4224, 30000])
+@pytest.mark.parametrize("kind", ["randn", "ties", "narrow", "mixed"])
+def test_decode_topk_one_group_rows(pkg, dev, kind, W):
+    """Rows of one 4096-position group (selected in LDS) beside rows at its
+    edges, with a bad histogram among them, in rows wider than they are."""
+    g = torch.Generator().manual_seed(W)
+    for K in (1, 700, 2048):
+        seq_t = torch.tensor([4096, 4095, min(4097, W), K + 1, K, 3000, min(W, 9000)],
+                             dtype=torch.int32)
+        s = scores(kind, len(seq_t), W, g)
+        h = hist_of(s, seq_t)
+        h[5] = 0
+        ws = torch.full((pkg._lib.lib().mi355_dsa_decode_topk_workspace_size(len(seq_t), W, K),),
+                        0xFF, dtype=torch.uint8, device=dev)
+        for _ in range(2):
+            idx = torch.full((len(seq_t), K), 123, dtype=torch.int32, device=dev)
+            _decode_topk_abi(pkg, idx, s.to(dev), seq_t.to(dev), h.to(dev), K, ws)
+            assert torch.equal(idx.cpu(), cref.topk_rows(s, seq_t, K)), K
+
+
 def test_decode_topk_one_launch_graph_replays(pkg, dev):
     """One-launch decode top-k captured in a HIP graph: every replay, with the
     scores and histograms rewritten in place between replays and an eager
