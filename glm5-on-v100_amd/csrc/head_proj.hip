@@ -19,9 +19,9 @@
 // k (KW, partial sums reduced through LDS), so both shapes of the layer give
 // 512 workgroups per call: W_UK_T (K = 128, N = 512) as NW = 4, and W_UV
 // (K = 512, N = 128) as KW = 4.  Large T is split over a second grid axis.
-// Prefill calls (T >= 512) take a wide variant that covers a head's whole N
-// per workgroup, so each token fragment is loaded once per wave and feeds
-// eight MFMAs.  Both compute D^T = W^T X^T, so a lane stores four
+// Prefill calls and larger batches take a wide variant that covers a head's
+// whole N per workgroup, so each token fragment is loaded once per wave and
+// feeds eight MFMAs.  Both compute D^T = W^T X^T, so a lane stores four
 // consecutive output columns of one token.  Accumulation is fp32; out is
 // rounded to fp16 once (RNE).
 #include <algorithm>
@@ -47,8 +47,19 @@ __global__ __launch_bounds__(256) void head_proj_kernel(HpArgs a) {
 // columns are copied inside the token loop.
 constexpr int kHpWideKb = 4;     // 32-wide k blocks per wave (K = 128 KW)
 constexpr int kHpWideNt = 8;     // column tiles per wave
-constexpr int kHpWideMinT = 512; // tokens from which a call takes the wide kernel
-constexpr int kHpWideWgs = 512;  // workgroups per call (two per CU)
+// A call takes the wide kernel from 512 tokens, and from 192 (head, 16-token
+// tile) units: there the decode-shaped kernel reads each weight column block
+// once per tile and feeds one MFMA per fragment.  us per call, decode-shaped /
+// wide, W_UV and W_UK: 64 heads, 32 tokens (128 units) 7.4 / 7.7 and 7.7 / 8.5; 48
+// tokens 10.5 / 7.8 and 10.9 / 8.7; 256 tokens 29.0 / 10.6 and 30.3 / 14.4; 16 heads,
+// 128 tokens (128 units) 6.9 / 7.4 and 7.0 / 8.0; 256 tokens 12.0 / 7.5 and 12.1 / 8.4.
+constexpr int kHpWideMinT = 512;
+constexpr int kHpWideMinUnits = 192;
+// Workgroups per call: one per CU.  Each loads its head's weight (128 KB), so two
+// per CU doubled that and halved the tokens behind it (64 heads, us with 512 /
+// 256: W_UV 128 tokens 12.0 / 8.6, 1024 23.0 / 21.2, 4096 78.8 / 77.4; W_UK 17.8 /
+// 14.4 at 256 tokens, 35.2 / 32.2 at 1024; 16 heads, 1024 tokens 13.4 / 9.9).
+constexpr int kHpWideWgs = 256;
 
 template <int NW, int KW, bool TAIL>
 __global__ __launch_bounds__(256) void head_proj_wide_kernel(HpArgs a) {
@@ -209,7 +220,7 @@ extern "C" int mi355_dsa_head_proj(void* out, int64_t out_tok_stride, int64_t ou
   // many tokens: the wide kernel (whole head per workgroup) when the shape
   // fits it; K = 128 KW and N a multiple of its column span
   const int wide_cols = (4 / KW) * kHpWideNt * 16;
-  if (T >= kHpWideMinT && K == 32 * kHpWideKb * KW && N % wide_cols == 0 && a.out8 &&
+  if ((T >= kHpWideMinT || (int64_t)H * ((T + 15) / 16) >= kHpWideMinUnits) && K == 32 * kHpWideKb * KW && N % wide_cols == 0 && a.out8 &&
       2 * tail <= 256) {
     a.n_blocks = N / wide_cols;
     const int gxw = H * a.n_blocks;

@@ -99,3 +99,21 @@ def test_every_token_written(pkg, dev):
     pkg.dsa_layer.head_proj(out, q, w.uk_t, 64)
     assert not torch.isnan(out).any()
     assert torch.equal(out.cpu(), O.q_latent(q.cpu(), uk).to(torch.float16))
+
+
+@pytest.mark.parametrize("H,T", [(64, 32), (64, 33), (64, 48), (64, 65), (16, 176), (16, 177),
+                                 (16, 193), (12, 256), (1, 511), (1, 513)])
+def test_wide_batches_equal_small_calls(pkg, dev, H, T):
+    """Batches at the edges of the wide kernel's range (192 units of a head and
+    16 tokens, 512 tokens) and of its token chunks: every token's outputs are,
+    bit for bit, those of calls of 16 tokens, which take the other kernel."""
+    g = torch.Generator().manual_seed(H * 1000 + T)
+    w, _, _ = weights(pkg, dev, g, H, 128, 128, False)
+    q = torch.randn(T, H, 192, generator=g).to(torch.float16).to(dev)
+    o = torch.randn(T, H, 512, generator=g).to(torch.float16).to(dev)
+    ql, out = pkg.dsa_layer.q_latent(q, w), pkg.dsa_layer.v_up(o, w)
+    for t in range(0, T, 16):
+        assert torch.equal(ql[t:t + 16].view(torch.int16),
+                           pkg.dsa_layer.q_latent(q[t:t + 16], w).view(torch.int16))
+        assert torch.equal(out[t:t + 16].view(torch.int16),
+                           pkg.dsa_layer.v_up(o[t:t + 16], w).view(torch.int16))
