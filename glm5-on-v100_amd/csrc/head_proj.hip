@@ -220,8 +220,8 @@ extern "C" int mi355_dsa_head_proj(void* out, int64_t out_tok_stride, int64_t ou
   // many tokens: the wide kernel (whole head per workgroup) when the shape
   // fits it; K = 128 KW and N a multiple of its column span
   const int wide_cols = (4 / KW) * kHpWideNt * 16;
-  if ((T >= kHpWideMinT || (int64_t)H * ((T + 15) / 16) >= kHpWideMinUnits) && K == 32 * kHpWideKb * KW && N % wide_cols == 0 && a.out8 &&
-      2 * tail <= 256) {
+  const bool many = T >= kHpWideMinT || (int64_t)H * ((T + 15) / 16) >= kHpWideMinUnits;
+  if (many && K == 32 * kHpWideKb * KW && N % wide_cols == 0 && a.out8 && 2 * tail <= 256) {
     a.n_blocks = N / wide_cols;
     const int gxw = H * a.n_blocks;
     const int tiles = (T + 15) / 16;
