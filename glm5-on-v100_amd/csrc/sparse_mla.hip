@@ -2470,16 +2470,49 @@ static int dma_decode_splits(int topk) {
   return s < 1 ? 1 : s;
 }
 
-// Key splits of `units` workgroups of `tiles` tiles each on `slots` resident
-// workgroups: the fewest rounds x (tiles per split + `fixed`, a workgroup's
-// prologue and epilogue in tiles), at least two tiles per split; one split
-// saves the merge launch (3 tiles).  A count just past a full round costs a
-// whole second one: 24 units of the 64-head fp8 kernel took 35 us with 11 splits
-// (264 workgroups on 256 CUs).
-static int pick_splits(int64_t units, int tiles, int slots, int fixed) {
+// Key splits that the workspace of a sparse call has room for, by the cache's row
+// type.  The size query and what the allocation-free entry takes follow from
+// this rule alone and not from the kernel that plan_decode picks, so callers'
+// buffers do not change with the plans.  1: the call is not split: a split's O is
+// rounded to fp16 before the merge, and a call that fills the chip without
+// splits keeps O in one fp32 accumulation.
+static int split_room(int B, int n_head, int topk, int kv_fp8) {
+  const int64_t units = (int64_t)B * ((n_head + 63) / 64);    // workgroups of 64 heads
+  const int64_t units16 = (int64_t)B * ((n_head + 15) / 16);  // and of 16
+  if (units >= kTargetWGs) return 1;
+  const int max64 = (topk + 63) / 64 < kMergeMaxSplits ? (topk + 63) / 64 : kMergeMaxSplits;
+  int s;
+  if (n_head > 32 && units >= kPipeMinUnits) {
+    s = (int)((kTargetWGs + units / 2) / units);  // about one round; at least 64 keys each
+    if (s > max64) s = max64;
+    return s < 1 ? 1 : s;
+  }
+  s = (int)(kTargetWGs / units16);
+  if (kv_fp8 && use_dma_decode(topk)) {  // at most 128 keys per split, at least 16
+    if (s >= 8) s = s / 8 * 8;
+    const int s128 = (topk + kDmaSplitKeys - 1) / kDmaSplitKeys;
+    const int s16 = (topk + kDecWaveKeys - 1) / kDecWaveKeys;
+    if (s < s128) s = s128;
+    if (s > s16) s = s16;
+    return s < 1 ? 1 : s;
+  }
+  if (s > max64) s = max64;
+  if (s >= 8) s = s / 8 * 8;
+  return s < 1 ? 1 : s;
+}
+
+// Key splits, at most `room`, of `units` workgroups of `tiles` tiles each on
+// `slots` resident workgroups: the fewest rounds x (tiles per split + `fixed`,
+// a workgroup's prologue and epilogue in tiles), at least two tiles per split;
+// one split saves the merge launch (3 tiles).  A count just past a full round
+// costs a whole second one: 24 units of the 64-head fp8 kernel took 35 us with
+// 11 splits (264 workgroups on 256 CUs).  us per call at the count taken / at the
+// best of 1, 2, 3, 4, 6 and 8, topk 2048, fp8 rows and 16 heads: 64 tokens 42.5 /
+// 40.8, 100 59.0 / 58.2, 128 67.8 / 67.5, 200 99.3 / 96.9, 255 106.9 / 106.2.
+static int pick_splits(int64_t units, int tiles, int slots, int fixed, int room) {
   int best = 1;
   int64_t best_cost = -1;
-  const int max_s = tiles / 2 < kMergeMaxSplits ? tiles / 2 : kMergeMaxSplits;
+  const int max_s = tiles / 2 < room ? tiles / 2 : room;
   for (int s = 1; s <= (max_s > 1 ? max_s : 1); s++) {
     const int64_t rounds = (units * s + slots - 1) / slots;
     const int64_t cost = rounds * ((tiles + s - 1) / s + fixed) + (s > 1 ? 3 : 0);
@@ -2550,16 +2583,24 @@ using namespace mi355dsa;
 //    fp16: mla_hw_f16_kernel or mla_attn_f16_kernel).  From 256 units up in one
 //    split; below that for > 32 heads from 8 units, for 17-32 heads from 32
 //    (32 tokens x 32 heads: fp8 27 against 36 kSplitDma, 34 kFewHeads; fp16 30
-//    against 35; 16 tokens: fp8 22 against 21, fp16 level).  Never for <= 16
-//    heads of fp8 rows, whose 48 empty heads cost more than the shared gather
-//    saves (2048 tokens x 16 heads: 749 us against 393 kFewHeads); fp16 rows the
-//    same (595 against 511).
+//    against 35; 16 tokens: fp8 22 against 21, fp16 level).  For <= 16 heads, whose
+//    48 empty heads cost more than the shared gather saves, only calls that are
+//    not split (split_room) and fit one round, from 257 keys: the list is then one
+//    workgroup's chain, and theirs is shorter (us, kFewHeads / kPipelined: fp16 130
+//    tokens x 2048 keys 123 / 90, 200 132 / 100, 200 x 512 41 / 39, 200 x 256 23.2 /
+//    23.5, 200 x 128 15.9 / 16.9; fp8 256 x 2048 126 / 116, 256 x 512 40 / 36).
 //  * kSplitDma: fp8 rows, small batches, 128 keys per split, 16 heads per
 //    workgroup.  For <= 16 heads below 64 tokens (48: 33 against 37 kFewHeads;
 //    64: 43 against 41).
 //  * kFewHeads: 16 heads per workgroup over 64-key tiles, the rest: <= 16 heads,
 //    fp16 batches too small for kPipelined (4 x 64 heads: 17 us), fp8 lists too
 //    long for kSplitDma.
+// Calls that are not split keep O in one fp32 accumulation.  us per call with the
+// splits that would fill the chip best / whole: fp16 16 heads, 129 tokens 85 / 89,
+// 300 103 / 117; 32 heads, 65 tokens 51 / 82, 128 76 / 90, 170 105 / 98; fp8 16
+// heads, 300 tokens 93 / 116, 800 195 / 216, 1000 227 / 217, 2500 523 / 476, 4096
+// 880 / 761.
+constexpr int kWholeMinKeys = 256;
 enum DecodeKind { kPipelined, kSplitDma, kFewHeads };
 struct DecodePlan {
   DecodeKind kind;
@@ -2568,27 +2609,29 @@ struct DecodePlan {
 
 static DecodePlan plan_decode(int B, int n_head, int topk, int kv_fp8) {
   const int64_t units = (int64_t)B * ((n_head + 63) / 64);
+  const int room8 = split_room(B, n_head, topk, 1), room16 = split_room(B, n_head, topk, 0);
+  const bool whole = (kv_fp8 ? room8 : room16) == 1;
+  const int room = whole ? 1 : (room8 > room16 ? room8 : room16);  // what the workspace holds
   if (n_head > 16) {
     if (units >= kTargetWGs) return {kPipelined, 1};
     if (units >= (n_head > 32 ? kPipeMinUnits : 4 * kPipeMinUnits))
-      return {kPipelined, pick_splits(units, (topk + kPfTileKeys - 1) / kPfTileKeys, kTargetWGs, 7)};
+      return {kPipelined, pick_splits(units, (topk + kPfTileKeys - 1) / kPfTileKeys, kTargetWGs, 7,
+                                      room)};
   }
   if (kv_fp8 && use_dma_decode(topk) && (n_head > 16 || B < kFewMinTokens))
     return {kSplitDma, dma_decode_splits(topk)};
+  if (whole && topk > kWholeMinKeys && units > kTargetWGs / 2 && units <= kTargetWGs)
+    return {kPipelined, 1};
   return {kFewHeads, pick_splits((int64_t)B * ((n_head + 15) / 16),
                                  (topk + kFewTile - 1) / kFewTile,
-                                 (kv_fp8 ? 3 : 2) * kTargetWGs, 2)};
+                                 (kv_fp8 ? 3 : 2) * kTargetWGs, 2, room)};
 }
 
 extern "C" size_t mi355_dsa_sparse_mla_workspace_size(int B, int n_head, int topk) {
   if (B <= 0 || n_head <= 0 || topk <= 0) return 0;
-  // the larger of the fp16 and fp8 split counts, so one size serves both; for few
-  // heads at least the split decode's, whichever kernel runs: the size, and with
-  // it what the allocation-free entry takes, does not depend on that choice
-  const int s16 = plan_decode(B, n_head, topk, 0).S, s8 = plan_decode(B, n_head, topk, 1).S;
-  int S = s16 > s8 ? s16 : s8;
-  if (n_head <= 32 && (int64_t)B < kTargetWGs && use_dma_decode(topk) && dma_decode_splits(topk) > S)
-    S = dma_decode_splits(topk);
+  // the larger of the fp16 and fp8 counts, so one size serves both
+  const int s16 = split_room(B, n_head, topk, 0), s8 = split_room(B, n_head, topk, 1);
+  const int S = s16 > s8 ? s16 : s8;
   if (S <= 1) return 0;
   return (size_t)B * n_head * S * (kValueDim * sizeof(f16) + 2 * sizeof(float));
 }

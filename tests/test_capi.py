@@ -90,6 +90,47 @@ def test_sparse_workspace_size(lib):
     assert lib.mi355_dsa_sparse_mla_workspace_size(4096, 64, 2048) == 0
 
 
+def sparse_splits(B, H, topk, fp8):
+    """Key splits that the sparse decode's workspace has room for."""
+    units64, units16 = B * -(-H // 64), B * -(-H // 16)
+    if units64 >= 256:  # every CU has 64 heads of a token
+        return 1
+    if H > 32 and units64 >= 8:
+        return max(1, min((256 + units64 // 2) // units64, -(-topk // 64), 128))
+    s = 256 // units16
+    if fp8 and -(-topk // 128) <= 128:
+        s = s // 8 * 8 if s >= 8 else s
+        return max(1, min(max(s, -(-topk // 128)), -(-topk // 16)))
+    s = min(s, -(-topk // 64), 128)
+    return max(1, s // 8 * 8 if s >= 8 else s)
+
+
+def test_sparse_workspace_sizes_over_the_range(lib):
+    """The workspace is part of the interface: its size is a rule on the call's
+    sizes, whichever kernels run, so that a caller's buffers keep fitting."""
+    for topk in (1, 64, 65, 128, 129, 300, 512, 2048, 2112, 4096, 16384, 17408):
+        for H in (1, 8, 16, 17, 32, 33, 64, 65, 96, 128):
+            for B in [*range(1, 300), 400, 513, 600, 800, 1000, 2500, 3333, 4096]:
+                S = max(sparse_splits(B, H, topk, True), sparse_splits(B, H, topk, False))
+                want = B * H * S * (512 * 2 + 2 * 4) if S > 1 else 0
+                assert lib.mi355_dsa_sparse_mla_workspace_size(B, H, topk) == want, (B, H, topk)
+
+
+@pytest.mark.parametrize("B,H,fits", [(170, 64, True), (85, 128, True), (255, 64, True),
+                                      (513, 16, True), (600, 16, True), (800, 16, True),
+                                      (4096, 16, True), (2500, 8, True), (127, 16, True),
+                                      (128, 16, False), (255, 16, False)])
+def test_noalloc_limit(pkg, lib, B, H, fits):
+    """Which top-2048 calls the allocation-free entry takes (the refusal comes
+    before any other check)."""
+    need = lib.mi355_dsa_sparse_mla_workspace_size(B, H, 2048)
+    assert (need <= lib.mi355_dsa_sparse_mla_noalloc_max_bytes()) == fits
+    if not fits or need == 0:
+        rc = lib.mi355_dsa_sparse_mla_decode_noalloc(None, None, None, B, H, None, 1, 0, 64, None,
+                                                     2048, None, 1, None, 0.1, None)
+        assert rc == 1 and ("maximum" in _err(pkg)) == (not fits)
+
+
 def test_sparse_rejects_small_workspace(pkg, lib):
     rc = lib.mi355_dsa_sparse_mla_decode(16, 16, 16, 4, 64, 16, 0, 100, 64, 16, 2048,
                                          16, 4, 16, 0.1, 16, 10, None)

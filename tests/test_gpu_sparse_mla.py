@@ -237,6 +237,39 @@ def test_few_heads(ops, dev, case):
     check(o, lse, ro, rl)
 
 
+WHOLE = [
+    # B, H, fp8: calls that fill the chip without splitting the keys (from 129
+    # 16-head or 171 64-head workgroups of fp16 rows, from 256 tokens of fp8 rows)
+    (130, 16, False), (255, 8, False), (66, 32, False), (200, 24, False), (300, 16, False),
+    (172, 64, False), (172, 64, True), (256, 16, True), (257, 16, True), (600, 16, True),
+    (800, 8, True), (256, 16, False),
+]
+
+
+@pytest.mark.parametrize("B,H,fp8", WHOLE, ids=["B%dH%d%s" % (b, h, "fp8" if f else "fp16")
+                                                for b, h, f in WHOLE])
+def test_whole_lists_keep_fp32_sums(pkg, lib, dev, B, H, fp8):
+    """No partial sums go through the (fp16) workspace: it stays untouched, and
+    where its size is 0 the call takes none."""
+    topk = 2048
+    q, kv, idx, bt, seq = make(120 + B, B, H, 60, 64, fp8, topk, [3000] * B, shared_bt=True)
+    need = lib.mi355_dsa_sparse_mla_workspace_size(B, H, topk)
+    ws = torch.full((need + 16,), 0x5A, dtype=torch.uint8, device=dev)
+    o = torch.full((B, H, 512), float("nan"), dtype=torch.float16, device=dev)
+    lse = torch.full((B, H), float("nan"), device=dev)
+    args = [x.to(dev) for x in (q, kv, idx, bt, seq)]
+    pkg._lib.call("mi355_dsa_sparse_mla_decode", o.data_ptr(), lse.data_ptr(), args[0].data_ptr(),
+                  B, H, args[1].data_ptr(), int(fp8), 60 * 64, 64, args[2].data_ptr(), topk,
+                  args[3].data_ptr(), bt.shape[1], args[4].data_ptr(), SCALE,
+                  ws.data_ptr() if need else None, need, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert bool((ws == 0x5A).all())
+    some = torch.tensor(sorted({0, 1, B // 2, B - 2, B - 1}))
+    ro, rl = O.sparse_mla(q[some], kv, idx[some], bt[some], seq[some], SCALE)
+    check(o.float().cpu()[some], lse.cpu()[some], ro, rl)
+    assert not torch.isnan(o).any() and not torch.isnan(lse).any()
+
+
 PIPE_SPLIT = [
     # seed, B, H, fp8, topk, seqs: batches of 8..255 tokens at > 32 heads run the
     # 64-head pipelined kernels with round(256 / (B * ceil(H / 64))) key splits
