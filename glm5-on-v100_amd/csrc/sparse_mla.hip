@@ -2591,7 +2591,15 @@ using namespace mi355dsa;
 //    23.5, 200 x 128 15.9 / 16.9; fp8 256 x 2048 126 / 116, 256 x 512 40 / 36).
 //  * kSplitDma: fp8 rows, small batches, 128 keys per split, 16 heads per
 //    workgroup.  For <= 16 heads below 64 tokens (48: 33 against 37 kFewHeads;
-//    64: 43 against 41).
+//    64: 43 against 41), and for short lists as long as its workgroups, which
+//    are many short chains, stay few.  <= 16 heads: up to three rounds of them, one
+//    for at most 256 keys, where the other kernel does not split; 17-32 heads: two,
+//    one for at most 128 keys (us, kSplitDma / the kernel otherwise taken: 16 heads,
+//    64 tokens x 512 keys 16.0 / 20.5, 128 x 512 25.8 / 29.2, 200 x 512 (800
+//    workgroups) 40.6 / 40.3, 64 x 1024 25.3 / 27.7, 128 x 256 17.3 / 20.5, 160 x
+//    256 (320) 23.6 / 21.3, 200 x 128 11.7 / 16.0; 32 heads, 32 x 512 14.7 / 20.5, 64 x
+//    512 23.0 / 23.9, 100 x 512 (800) 36.2 / 29.6, 100 x 128 10.8 / 16.6, 200 x 64
+//    (400) 17.0 / 15.0).
 //  * kFewHeads: 16 heads per workgroup over 64-key tiles, the rest: <= 16 heads,
 //    fp16 batches too small for kPipelined (4 x 64 heads: 17 us), fp8 lists too
 //    long for kSplitDma.
@@ -2612,13 +2620,19 @@ static DecodePlan plan_decode(int B, int n_head, int topk, int kv_fp8) {
   const int room8 = split_room(B, n_head, topk, 1), room16 = split_room(B, n_head, topk, 0);
   const bool whole = (kv_fp8 ? room8 : room16) == 1;
   const int room = whole ? 1 : (room8 > room16 ? room8 : room16);  // what the workspace holds
+  const bool dma = kv_fp8 && use_dma_decode(topk);
+  const int64_t dma_wgs = (int64_t)B * ((n_head + 15) / 16) * dma_decode_splits(topk);
   if (n_head > 16) {
     if (units >= kTargetWGs) return {kPipelined, 1};
-    if (units >= (n_head > 32 ? kPipeMinUnits : 4 * kPipeMinUnits))
+    const bool short_lists =
+        dma && n_head <= 32 && dma_wgs <= (topk > kDmaSplitKeys ? 2 : 1) * kTargetWGs;
+    if (units >= (n_head > 32 ? kPipeMinUnits : 4 * kPipeMinUnits) && !short_lists)
       return {kPipelined, pick_splits(units, (topk + kPfTileKeys - 1) / kPfTileKeys, kTargetWGs, 7,
                                       room)};
   }
-  if (kv_fp8 && use_dma_decode(topk) && (n_head > 16 || B < kFewMinTokens))
+  if (dma && (n_head > 16 || B < kFewMinTokens ||
+              (units < kTargetWGs &&
+               dma_wgs <= (topk > 2 * kDmaSplitKeys ? 3 : 1) * kTargetWGs)))
     return {kSplitDma, dma_decode_splits(topk)};
   if (whole && topk > kWholeMinKeys && units > kTargetWGs / 2 && units <= kTargetWGs)
     return {kPipelined, 1};

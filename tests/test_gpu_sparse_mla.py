@@ -237,6 +237,25 @@ def test_few_heads(ops, dev, case):
     check(o, lse, ro, rl)
 
 
+SHORT_FP8 = [
+    # B, H, topk around the lines between the 16-head split decode and the other
+    # kernels: its workgroups B x ceil(H / 16) x ceil(topk / 128) at one, two and three
+    # rounds of 256, lists of one and of two splits, 255 and 256 tokens
+    (64, 16, 512), (192, 16, 512), (193, 16, 512), (128, 16, 256), (129, 16, 256), (255, 16, 128), (255, 8, 385), (256, 16, 64),
+    (64, 32, 512), (65, 32, 512), (128, 32, 128), (129, 32, 128), (128, 32, 129), (32, 24, 2048),
+    (200, 20, 64),
+]
+
+
+@pytest.mark.parametrize("B,H,topk", SHORT_FP8, ids=["B%dH%dK%d" % c for c in SHORT_FP8])
+def test_short_fp8_lists(ops, dev, B, H, topk):
+    seqs = [1 + (53 * i + 400) % 1900 for i in range(B)]
+    q, kv, idx, bt, seq = make(200 + B + topk, B, H, 40, 64, True, topk, seqs, invalid_frac=0.05)
+    o, lse = run(ops, dev, q, kv, idx, bt, seq)
+    ro, rl = O.sparse_mla(q, kv, idx, bt, seq, SCALE)
+    check(o, lse, ro, rl)
+
+
 WHOLE = [
     # B, H, fp8: calls that fill the chip without splitting the keys (from 129
     # 16-head or 171 64-head workgroups of fp16 rows, from 256 tokens of fp8 rows)
