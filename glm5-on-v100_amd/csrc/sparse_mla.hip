@@ -69,6 +69,7 @@ struct MlaParams {
   f16* part_o;
   float* part_ml;  // [B, H, S, 2]   per-split (m_s, l_s)
   int share;  // dense: splits divided by the lengths (dense_share)
+  float lazy_max;  // of the 64-head fp8 kernel: kPfLazyMax, or 0
   int B, n_head, topk, max_blocks, page_size, n_splits;
   int page_shift;  // log2(page_size) when it is a power of two, else -1
   int64_t n_kv_rows;
@@ -512,7 +513,12 @@ __global__ void __launch_bounds__(kDmaThreads) sparse_mla_decode_dma_kernel(MlaP
 // max is lazy: O and l are rescaled only when a head's tile max exceeds the
 // running max by more than kPfLazyMax, so p = exp(s - m) <= e^8 (well inside
 // fp16) and rescales are rare; o = O / l and lse = m + ln l are unchanged by
-// the choice of m.
+// the choice of m.  For fp8_ds_mla rows it is p times the key's tile scale that
+// is rounded to fp16: finite for tile scales up to 65504 / e^8 = 22 (latents up
+// to 9,850).  Batches of at most 32 heads, which the split decode with its p <= 1
+// shares, keep the exact running max (lazy_max = 0) and its range, tile scales
+// up to 65504 (us per call lazy / exact at 32 heads: 32 tokens 27.1 / 28.7, 64 42.2 /
+// 45.2, 200 102 / 110).
 // ---------------------------------------------------------------------------
 constexpr int kPfWaves = 8;
 constexpr int kPfThreads = 64 * kPfWaves;
@@ -949,7 +955,7 @@ __device__ __forceinline__ void ws_sm_role(const MlaParams& p, const WsCtx& x, W
     mt = fmaxf(mt, dppf<0xB1>(mt));  // quad_perm [1,0,3,2]
     mt = fmaxf(mt, dppf<0x4E>(mt));  // quad_perm [2,3,0,1]
     float alpha = 1.f;
-    if (mt > m_run + kPfLazyMax) {
+    if (mt > m_run + p.lazy_max) {
       const float m_new = fmaxf(m_run, mt);
       alpha = __expf(m_run - m_new);
       l_run *= alpha;
@@ -1873,7 +1879,8 @@ __global__ void __launch_bounds__(kHwThreads, 1) mla_hw_f16_kernel(MlaParams p) 
 //   * wave w adds V^T P^T of the 64 keys to O^T of value dims [128 w, +128)
 //     (one fp8 scale tile): P times the source wave's exp(m_w - m) and the key's
 //     scale, rounded to fp16 once; a barrier frees the tile.
-// The running max m is lazy (kPfLazyMax) and the same in every wave.
+// The running max m is the same in every wave; lazy (kPfLazyMax) for fp16 rows,
+// exact for fp8 rows, whose P times the tile scale must stay inside fp16.
 // Region layout: 64-byte blocks, block-major (block b of key r at 1024 b + 64 r),
 // piece p of a block at p ^ few_sw(r): the QK reads (16 keys x 4 pieces) and the
 // transpose reads are free of bank conflicts, and a DMA instruction fetches a
@@ -1911,6 +1918,7 @@ template <bool FP8>
 __global__ void __launch_bounds__(kFewThreads, FP8 ? 3 : 2) sparse_mla_few_kernel(MlaParams p) {
   using Sm = FewSmem<FP8>;
   constexpr int ROW = FP8 ? kDsmlaRowBytes : kLatentDim * 2;
+  constexpr float kLazy = FP8 ? 0.f : kPfLazyMax;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Sm& sh = *reinterpret_cast<Sm*>(smem_raw);
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2066,8 +2074,8 @@ __global__ void __launch_bounds__(kFewThreads, FP8 ? 3 : 2) sparse_mla_few_kerne
         mw[u] = sh.m[u][c];
         M = fmaxf(M, mw[u]);
       }
-      if (__any(M > m_run + kPfLazyMax)) {
-        const float m_new = M > m_run + kPfLazyMax ? M : m_run;
+      if (__any(M > m_run + kLazy)) {
+        const float m_new = M > m_run + kLazy ? M : m_run;
         const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * kLog2e);
         m_run = m_new;
         l_part *= alpha;
@@ -2697,6 +2705,7 @@ static int mla_decode_impl(
   prm.zero_unresolved = (dense || !(B >= 32 && n_head <= 16)) ? 1 : 0;
   prm.xcd_map = 0;
   prm.share = 0;
+  prm.lazy_max = kv_fp8 && n_head <= 32 && B < kTargetWGs ? 0.f : kPfLazyMax;
   hipStream_t st = as_stream(stream);
 
   if (dense) {

@@ -237,6 +237,52 @@ def test_few_heads(ops, dev, case):
     check(o, lse, ro, rl)
 
 
+LARGE_SCALES = [
+    # B, H, topk: the 16-head kernel split and whole, the 64-head kernel below 33
+    # heads, the 128-key split decode
+    (64, 16, 2048), (100, 8, 1024), (300, 16, 2048), (40, 32, 2048), (100, 24, 2048), (8, 16, 2048),
+]
+
+
+@pytest.mark.parametrize("B,H,topk", LARGE_SCALES, ids=["B%dH%dK%d" % c for c in LARGE_SCALES])
+def test_large_tile_scales(ops, dev, B, H, topk):
+    """Tile scales of 32-128 (latents up to 57,344) and one key per token that scores
+    7.2-7.5 above the others: p times the scale stays finite in fp16 only while
+    p is taken against the true maximum (e^7.2 x 64 does not fit).  Scores come from
+    one RoPE dim alone.  Bound: P and o are each rounded to fp16 once (2^-11),
+    partials once more: 2^-9 sum(p |v|) / sum(p), the same attention on |v|."""
+    g = torch.Generator().manual_seed(B + topk)
+    page, ctx = 64, 2560
+    n = ctx  # every token's cache pages are the same
+    code = torch.randint(0, 255, (n, 512), generator=g, dtype=torch.int32).to(torch.uint8)
+    code[(code & 0x7F) == 0x7F] = 0x7E
+    scale = torch.exp2(torch.randint(5, 8, (n, 4), generator=g).float())
+    rope = torch.zeros(n, 64, dtype=torch.float16)
+    rope[:, 0] = torch.rand(n, generator=g) * 0.3
+    peaks = torch.randperm(n, generator=g)[:B]
+    rope[peaks, 0] = 7.5
+    def rows(c):
+        return torch.cat([c, scale.view(torch.uint8), rope.view(torch.uint8)], 1).view(-1, page, 656)
+    q = torch.zeros(B, H, 576, dtype=torch.float16)
+    q[:, :, 512] = 1 / SCALE
+    bt = torch.arange(ctx // page, dtype=torch.int32).expand(B, -1).contiguous()
+    seq = torch.full((B,), ctx, dtype=torch.int32)
+    others = torch.ones(n, dtype=torch.bool)
+    others[peaks] = False
+    others = others.nonzero().flatten()
+    idx = torch.empty(B, topk, dtype=torch.int32)
+    for b in range(B):
+        pick = others[torch.randperm(len(others), generator=g)[:topk - 1]]
+        idx[b] = torch.cat([pick, peaks[b:b + 1]]).sort().values.to(torch.int32)
+    o, lse = run(ops, dev, q, rows(code), idx, bt, seq)
+    assert torch.isfinite(o).all()
+    some = torch.tensor(sorted({0, 1, B // 3, B // 2, B - 1}))
+    ro, rl = O.sparse_mla(q[some], rows(code), idx[some], bt[some], seq[some], SCALE)
+    bound, _ = O.sparse_mla(q[some], rows(code & 0x7F), idx[some], bt[some], seq[some], SCALE)
+    assert ((o[some] - ro).abs() <= 2 ** -9 * bound).all()
+    assert (lse[some] - rl).abs().max().item() <= LSE_ATOL
+
+
 SHORT_FP8 = [
     # B, H, topk around the lines between the 16-head split decode and the other
     # kernels: its workgroups B x ceil(H / 16) x ceil(topk / 128) at one, two and three
