@@ -694,6 +694,9 @@ int launch_ring(const VaArgs& a0, int num_seqs, int max_q_len, hipStream_t st) {
   const int rc = reserve_lds(reinterpret_cast<const void*>(kern), lds, "varlen_attention");
   if (rc) return rc;
   VaArgs a = a0;
+  // scale 0 (equal weights): a masked score is -inf and needs a factor above 0
+  // to stay one (any other score below 1e31 then counts less than 1e-7)
+  if (fabsf(a.scale_log2) < FLT_MIN) a.scale_log2 = FLT_MIN;
   a.n_qtiles = (max_q_len + QROWS - 1) / QROWS;
   if (a.n_qtiles == 0) return MI355_DSA_OK;
   // pair-major order where it leaves no XCD idle (a multiple of 8 pairs, or

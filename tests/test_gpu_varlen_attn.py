@@ -110,6 +110,19 @@ def test_equal_scores_closed_form(pkg, dev):
         torch.testing.assert_close(out[t], v[ks:ks + n].float().mean(0), rtol=2e-3, atol=1e-3)
 
 
+@pytest.mark.parametrize("scale", [0.0, -0.0, 1e-40])
+@pytest.mark.parametrize("dims", [(192, 128), (64, 64), (256, 256)])
+def test_zero_scale_is_equal_weights(pkg, dev, dims, scale):
+    """softmax_scale 0 weighs every visible key equally; masked keys stay out."""
+    cu_q, cu_k = [0, 64, 100, 231], [0, 300, 330, 461]
+    for dtype in (torch.float16, torch.bfloat16):
+        q, k, v = make(11, cu_q, cu_k, 4, *dims, dtype)
+        for causal in (True, False):
+            out, lse = run(pkg, dev, q, k, v, cu_q, cu_k, scale, causal)
+            ro, rl = O.varlen_attention(q, k, v, cu_q, cu_k, scale, causal)
+            check(out, lse, ro, rl, dtype)
+
+
 # (q_len, k_len) around the ring kernel's 32-key steps and 128-row tiles (and
 # its three-step prologue); H = 3 takes the plain grid order, H = 8 whole
 # (sequence, head) pairs per XCD
