@@ -3,7 +3,8 @@
 Usage: python glm5-on-v100_amd/build.py   (or __graft_entry__.build())
 
 Each csrc/*.hip is compiled to an object in _build/ (in parallel), then the
-objects are linked into <package>/libmi355_dsa.so.  hipcc cross-compiles
+objects are linked into <package>/libmi355_dsa.so.  Kernels that rely on a
+property of the generated code are checked for it (check_kernels).  hipcc cross-compiles
 gfx950 code without a GPU.
 """
 from __future__ import annotations
@@ -11,6 +12,7 @@ from __future__ import annotations
 import concurrent.futures as cf
 import glob
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -44,13 +46,69 @@ def compile_flags() -> list[str]:
     ]
 
 
+# Kernels of each source whose generated code the build checks (check_kernels):
+# those that hold values in accumulation registers named in inline asm, which
+# the compiler does not know to be in use.
+OWN_AGPRS = {"sparse_mla.hip": ["mla_hw_f16_kernel"]}
+
+
+def _body(asm: str, kernel: str) -> tuple[str, list[str]]:
+    """The symbol and the assembly lines of the one kernel whose name holds `kernel`."""
+    names = [n for n in re.findall(r"^(_Z\w+):", asm, re.M)
+             if kernel in n and f"\n\t.amdhsa_kernel {n}\n" in asm]
+    if len(names) != 1:
+        raise RuntimeError(f"{kernel}: {len(names)} kernels of that name in the assembly")
+    start = asm.index(f"\n{names[0]}:")
+    return names[0], asm[start:asm.index(".Lfunc_end", start)].split("\n")
+
+
+def _usage(asm: str, symbol: str, key: str) -> int:
+    """An entry of the kernel's metadata (".vgpr_spill_count" and the like)."""
+    for block in asm[asm.index("amdhsa.kernels:"):].split("\n  - ")[1:]:
+        if re.search(rf"\.name:\s+{re.escape(symbol)}\s", block):
+            return int(re.search(rf"{re.escape(key)}:\s+(\d+)", block).group(1))
+    raise RuntimeError(f"{symbol}: no metadata")
+
+
+def check_kernels(asm: str, own_agprs: list[str]) -> None:
+    """Raises unless every kernel of `own_agprs` is as its inline asm needs it:
+    nothing spilled, no scratch memory, at most 256 other registers, and no
+    instruction that the compiler placed names an accumulation register."""
+    for kernel in own_agprs:
+        symbol, lines = _body(asm, kernel)
+        agprs = _usage(asm, symbol, ".agpr_count")
+        used = {k: _usage(asm, symbol, k) for k in
+                (".vgpr_spill_count", ".sgpr_spill_count", ".private_segment_fixed_size")}
+        if any(used.values()) or _usage(asm, symbol, ".vgpr_count") - agprs > 256:
+            raise RuntimeError(f"{kernel}: spills or too many registers: {used}")
+        in_asm = False
+        for line in lines:
+            if "#ASMSTART" in line or "#ASMEND" in line:
+                in_asm = "#ASMSTART" in line
+                continue
+            code = line.split(";")[0].strip()
+            if not in_asm and re.search(r"\s(?:\S*,\s*)*a(?:\d+|\[\d+:\d+\])", code):
+                raise RuntimeError(f"{kernel}: the compiler uses an accumulation register: {code}")
+
+
 def _compile(src: str) -> str:
-    obj = os.path.join(BUILD_DIR, os.path.basename(src).replace(".hip", ".o"))
+    name = os.path.basename(src)
+    obj = os.path.join(BUILD_DIR, name.replace(".hip", ".o"))
     cmd = [hipcc(), *compile_flags(), "-c", src, "-o", obj]
+    if name in OWN_AGPRS:  # the assembly that the object is made from, beside it
+        cmd.append("-save-temps=obj")
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stdout}\n{r.stderr}")
+    if name in OWN_AGPRS:
+        with open(asm_path(name)) as f:
+            check_kernels(f.read(), OWN_AGPRS[name])
     return obj
+
+
+def asm_path(name: str) -> str:
+    """Where the build leaves the device assembly of a checked source."""
+    return os.path.join(BUILD_DIR, name.replace(".hip", f"-hip-amdgcn-amd-amdhsa-{ARCH}.s"))
 
 
 TESTKIT_SRC = os.path.join(PKG_DIR, "..", "tests", "hip", "quant_exhaustive.hip")

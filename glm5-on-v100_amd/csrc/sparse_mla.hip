@@ -1390,7 +1390,8 @@ constexpr int kHwAhead = 3;                                      // LDS reads ah
 // needs the other 256 for Q, scores, P and the operands in flight: left to it,
 // O moved between the two files every round and Q spilled.  It never
 // allocates an accumulation register itself in a kernel that does not exceed
-// 256 VGPRs (hw_own_agprs, once a round, lists them all as overwritten).
+// 256 VGPRs (hw_own_agprs, once a round, lists them all as overwritten); the
+// build reads the generated code for that and fails otherwise (check_kernels).
 #define HW_AGPRS \
   "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", \
   "a14", "a15", "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", \
