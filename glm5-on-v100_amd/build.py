@@ -50,6 +50,9 @@ def compile_flags() -> list[str]:
 # those that hold values in accumulation registers named in inline asm, which
 # the compiler does not know to be in use.
 OWN_AGPRS = {"sparse_mla.hip": ["mla_hw_f16_kernel"]}
+# Kernels that must not spill: a reload in a loop waits for all of the wave's
+# memory operations, gathers in flight included.
+NO_SPILLS = {"sparse_mla.hip": ["sparse_mla_prefill_fp8_ws_kernel"]}
 
 
 def _body(asm: str, kernel: str) -> tuple[str, list[str]]:
@@ -70,17 +73,21 @@ def _usage(asm: str, symbol: str, key: str) -> int:
     raise RuntimeError(f"{symbol}: no metadata")
 
 
-def check_kernels(asm: str, own_agprs: list[str]) -> None:
-    """Raises unless every kernel of `own_agprs` is as its inline asm needs it:
-    nothing spilled, no scratch memory, at most 256 other registers, and no
-    instruction that the compiler placed names an accumulation register."""
-    for kernel in own_agprs:
+def check_kernels(asm: str, own_agprs: list[str], no_spills: list[str] = []) -> None:
+    """Raises unless no kernel of either list spills or uses scratch memory, and
+    every kernel of `own_agprs` is as its inline asm needs it: at most 256 other
+    registers, and no instruction that the compiler placed names an accumulation
+    register."""
+    for kernel in [*own_agprs, *no_spills]:
         symbol, lines = _body(asm, kernel)
-        agprs = _usage(asm, symbol, ".agpr_count")
         used = {k: _usage(asm, symbol, k) for k in
                 (".vgpr_spill_count", ".sgpr_spill_count", ".private_segment_fixed_size")}
-        if any(used.values()) or _usage(asm, symbol, ".vgpr_count") - agprs > 256:
-            raise RuntimeError(f"{kernel}: spills or too many registers: {used}")
+        if any(used.values()):
+            raise RuntimeError(f"{kernel}: spills: {used}")
+        if kernel not in own_agprs:
+            continue
+        if _usage(asm, symbol, ".vgpr_count") - _usage(asm, symbol, ".agpr_count") > 256:
+            raise RuntimeError(f"{kernel}: too many registers")
         in_asm = False
         for line in lines:
             if "#ASMSTART" in line or "#ASMEND" in line:
@@ -102,7 +109,7 @@ def _compile(src: str) -> str:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stdout}\n{r.stderr}")
     if name in OWN_AGPRS:
         with open(asm_path(name)) as f:
-            check_kernels(f.read(), OWN_AGPRS[name])
+            check_kernels(f.read(), OWN_AGPRS[name], NO_SPILLS.get(name, []))
     return obj
 
 

@@ -777,6 +777,8 @@ __device__ __forceinline__ void ws_qk_role(const MlaParams& p, const WsCtx& x, W
   for (int seg_lo = x.k_lo; seg_lo < x.k_hi; seg_lo += kSegKeys) {
     const int nkeys = min(x.k_hi - seg_lo, kSegKeys);
     const int ntiles = ws_resolve(p, x, seg_lo, nkeys, sh);
+    // (known, the compiler reads K beside the MFMAs rather than before them)
+    __builtin_assume(ntiles >= 1);
     lds_barrier();  // tile 0 landed
     for (int s = -1; s < ntiles; s++) {
       f32x4 v[2][4];
@@ -851,12 +853,23 @@ __device__ __forceinline__ void ws_pv_role(const MlaParams& p, const WsCtx& x, W
       const bool dma = s + 3 < ntiles;
       if (s >= 1) pv(s - 1);
       if (dma) {
+        // tile s + 2 has landed: with one tile of a wave in flight the call is as
+        // fast on random rows and faster on shared ones than with two (us, 64
+        // heads: batch of 172 91.8 / 93.9, prefill of 4096 1458 / 1482)
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         // the slot of tile s - 1: this wave's own PV reads of it have returned
         // (and nothing of the refill is scheduled into the PV above, where
         // the O accumulators hold the registers)
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        ws_dma_nope(kv, sh.rows + (s + 3) * kPfTileKeys, sh.ring[(s + 3) % kWsRing], pw, lane);
+        // The refill's addresses come from an opaque lane, so that none is kept
+        // over the PV: there it was one register too many, and its reload from
+        // scratch waited for every memory operation inside the loop (us, 64 heads:
+        // 172 tokens 102.4 -> 91.8, 100 70.0 -> 65.6, prefill of 4096 level).
+        int l = lane;
+        asm volatile("" : "+v"(l));
+        ws_dma_nope(kv, sh.rows + (s + 3) * kPfTileKeys, sh.ring[(s + 3) % kWsRing], pw, l);
       }
       lds_barrier();
       ws_wait_pv(dma);  // tile s + 2 landed (this wave's part)

@@ -32,7 +32,7 @@ def asm(build):
 
 
 def test_this_tree_passes(build, asm):
-    build.check_kernels(asm, build.OWN_AGPRS[NAME])
+    build.check_kernels(asm, build.OWN_AGPRS[NAME], build.NO_SPILLS[NAME])
 
 
 @pytest.mark.parametrize("line", ["v_accvgpr_write_b32 a7, v3", "v_accvgpr_read_b32 v3, a255",
@@ -49,14 +49,15 @@ def test_an_accumulation_register_of_the_compilers(build, asm, line):
 
 @pytest.mark.parametrize("key", [".vgpr_spill_count", ".sgpr_spill_count",
                                  ".private_segment_fixed_size"])
-def test_spills_and_scratch(build, asm, key):
+@pytest.mark.parametrize("own,none", [([KERNEL], []), ([], [KERNEL])], ids=["own", "none"])
+def test_spills_and_scratch(build, asm, key, own, none):
     symbol, _ = build._body(asm, KERNEL)
     head, _, meta = asm.partition("amdhsa.kernels:")
     blocks = meta.split("\n  - ")
     i = next(i for i, b in enumerate(blocks) if re.search(rf"\.name:\s+{symbol}\s", b))
     blocks[i] = re.sub(rf"{re.escape(key)}:(\s+)\d+", rf"{key}:\g<1>4", blocks[i])
     with pytest.raises(RuntimeError, match="spills"):
-        build.check_kernels(head + "amdhsa.kernels:" + "\n  - ".join(blocks), [KERNEL])
+        build.check_kernels(head + "amdhsa.kernels:" + "\n  - ".join(blocks), own, none)
 
 
 def test_a_missing_kernel(build, asm):
