@@ -52,7 +52,7 @@ def compile_flags() -> list[str]:
 OWN_AGPRS = {"sparse_mla.hip": ["mla_hw_f16_kernel"]}
 # Kernels that must not spill: a reload in a loop waits for all of the wave's
 # memory operations, gathers in flight included.
-NO_SPILLS = {"sparse_mla.hip": ["sparse_mla_prefill_fp8_ws_kernel"]}
+NO_SPILLS = {"sparse_mla.hip": ["sparse_mla_prefill_fp8_ws_kernel", "sparse_mla_few_kernelILb0E"]}
 
 
 def _body(asm: str, kernel: str) -> tuple[str, list[str]]:

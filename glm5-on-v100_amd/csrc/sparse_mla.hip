@@ -1902,9 +1902,12 @@ __global__ void __launch_bounds__(kHwThreads, 1) mla_hw_f16_kernel(MlaParams p) 
 // tile-major (tile t of key r at 64 t + 4 r).
 // Bound: the gather's latency (a tile's rows are one round trip, hidden only by
 // the other workgroups of the CU) and, for fp8 rows, the conversions of every row
-// for 16 heads' products.  2048 tokens x 16 heads: fp8 749 us with the 64-head
-// kernel -> 393, fp16 595 -> 511; 32 tokens x 16 heads fp16 36.8 -> 30.0
-// us a call (the kernel before kept one tile in flight).
+// for 16 heads' products.  The source waves' maxima are read from LDS: picked by
+// the lane from an array they went through scratch memory in every tile.  us,
+// 64-head kernel / maxima in scratch / in LDS: 2048 tokens x 16 heads fp8 674 /
+// 382 / 333, fp16 825 / 507 / 397; 32 x 16 fp16 35.6 (one tile in flight) / 27.5 /
+// 26.7; 100 x 16 fp8 69.0 / 61.7 / 57.4.  (The fp8 variant's 11 spilled registers are
+// reloaded outside the tile loop.)
 // ---------------------------------------------------------------------------
 constexpr int kFewThreads = 256;
 constexpr int kFewTile = 64;     // keys per tile
@@ -2082,12 +2085,9 @@ __global__ void __launch_bounds__(kFewThreads, FP8 ? 3 : 2) sparse_mla_few_kerne
       lds_barrier();  // P, the maxima and every wave's rows are in
 
       // ---- running max, and the sum of this lane's p ----
-      float mw[4], M = -1e30f;
+      float M = -1e30f;
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        mw[u] = sh.m[u][c];
-        M = fmaxf(M, mw[u]);
-      }
+      for (int u = 0; u < 4; u++) M = fmaxf(M, sh.m[u][c]);
       if (__any(M > m_run + kLazy)) {
         const float m_new = M > m_run + kLazy ? M : m_run;
         const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * kLog2e);
@@ -2105,7 +2105,7 @@ __global__ void __launch_bounds__(kFewThreads, FP8 ? 3 : 2) sparse_mla_few_kerne
         const uint8_t* rg = sh.rows[2 * kb] + (g >> 1) * Sm::REGION;
         const f32x4 pa = *reinterpret_cast<const f32x4*>(&sh.pt[few_pt(c, 32 * kb + 8 * g)]);
         const f32x4 pc = *reinterpret_cast<const f32x4*>(&sh.pt[few_pt(c, 32 * kb + 8 * g + 4)]);
-        const float f = __builtin_amdgcn_exp2f(((g >> 1 ? mw[2 * kb + 1] : mw[2 * kb]) - m_run) * kLog2e);
+        const float f = __builtin_amdgcn_exp2f((sh.m[2 * kb + (g >> 1)][c] - m_run) * kLog2e);
         f16x8 pb;
         if constexpr (FP8) {
           const float* sc = reinterpret_cast<const float*>(rg + 1024 * Sm::BLOCKS) + 16 * w + 8 * (g & 1);
@@ -2529,8 +2529,8 @@ static int split_room(int B, int n_head, int topk, int kv_fp8) {
 // one split saves the merge launch (3 tiles).  A count just past a full round
 // costs a whole second one: 24 units of the 64-head fp8 kernel took 35 us with
 // 11 splits (264 workgroups on 256 CUs).  us per call at the count taken / at the
-// best of 1, 2, 3, 4, 6 and 8, topk 2048, fp8 rows and 16 heads: 64 tokens 42.5 /
-// 40.8, 100 59.0 / 58.2, 128 67.8 / 67.5, 200 99.3 / 96.9, 255 106.9 / 106.2.
+// best of 1, 2, 3, 4, 6 and 8, topk 2048, fp8 rows and 16 heads: 64 tokens 43.3 /
+// 36.4, 100 56.9 / 52.6, 128 61.8 / 60.1, 200 90.5 / 87.6, 255 98.5 / 94.0.
 static int pick_splits(int64_t units, int tiles, int slots, int fixed, int room) {
   int best = 1;
   int64_t best_cost = -1;
@@ -2604,32 +2604,32 @@ using namespace mi355dsa;
 //  * kPipelined: 64 heads per workgroup (fp8: sparse_mla_prefill_fp8_ws_kernel,
 //    fp16: mla_hw_f16_kernel or mla_attn_f16_kernel).  From 256 units up in one
 //    split; below that for > 32 heads from 8 units, for 17-32 heads from 32
-//    (32 tokens x 32 heads: fp8 27 against 36 kSplitDma, 34 kFewHeads; fp16 30
-//    against 35; 16 tokens: fp8 22 against 21, fp16 level).  For <= 16 heads, whose
-//    48 empty heads cost more than the shared gather saves, only calls that are
+//    (32 tokens x 32 heads: fp8 27 against 37 kSplitDma, 32 kFewHeads; fp16 30
+//    against 35; 16 tokens: fp8 23 against 22, fp16 level).  For <= 16 heads, whose
+//    48 empty heads cost more than the shared gather saves (2048 tokens x 16 heads,
+//    us, kFewHeads / kPipelined: fp8 347 / 675, fp16 391 / 591), only calls that are
 //    not split (split_room) and fit one round, from 257 keys: the list is then one
-//    workgroup's chain, and theirs is shorter (us, kFewHeads / kPipelined: fp16 130
-//    tokens x 2048 keys 123 / 90, 200 132 / 100, 200 x 512 41 / 39, 200 x 256 23.2 /
-//    23.5, 200 x 128 15.9 / 16.9; fp8 256 x 2048 126 / 116, 256 x 512 40 / 36).
+//    workgroup's chain, and theirs is shorter (fp16 130 tokens x 2048 keys 118 / 92,
+//    200 126 / 106, 200 x 512 39.2 / 37.4, 200 x 256 22.4 / 24.0, 200 x 128 14.9 /
+//    16.9; fp8 256 x 2048 120 / 106, 256 x 512 38 / 34).
 //  * kSplitDma: fp8 rows, small batches, 128 keys per split, 16 heads per
-//    workgroup.  For <= 16 heads below 64 tokens (48: 33 against 37 kFewHeads;
-//    64: 43 against 41), and for short lists as long as its workgroups, which
+//    workgroup.  For <= 16 heads below 64 tokens (48: 32 against 33 kFewHeads;
+//    64: 41 against 39), and for short lists as long as its workgroups, which
 //    are many short chains, stay few.  <= 16 heads: up to three rounds of them, one
 //    for at most 256 keys, where the other kernel does not split; 17-32 heads: two,
 //    one for at most 128 keys (us, kSplitDma / the kernel otherwise taken: 16 heads,
-//    64 tokens x 512 keys 16.0 / 20.5, 128 x 512 25.8 / 29.2, 200 x 512 (800
-//    workgroups) 40.6 / 40.3, 64 x 1024 25.3 / 27.7, 128 x 256 17.3 / 20.5, 160 x
-//    256 (320) 23.6 / 21.3, 200 x 128 11.7 / 16.0; 32 heads, 32 x 512 14.7 / 20.5, 64 x
-//    512 23.0 / 23.9, 100 x 512 (800) 36.2 / 29.6, 100 x 128 10.8 / 16.6, 200 x 64
-//    (400) 17.0 / 15.0).
+//    64 tokens x 512 keys 15.8 / 19.8, 128 x 512 25.1 / 26.6, 200 x 512 (800
+//    workgroups) 40.5 / 37.2, 64 x 1024 24.2 / 25.0, 128 x 256 17.2 / 19.8, 160 x
+//    256 (320) 23.3 / 20.5, 200 x 128 11.4 / 15.4; 32 heads, 32 x 512 14.4 / 20.5, 64 x
+//    512 22.6 / 24.1, 100 x 512 (800) 35.9 / 30.6, 100 x 128 10.2 / 16.8, 200 x 64
+//    (400) 17.0 / 14.8).
 //  * kFewHeads: 16 heads per workgroup over 64-key tiles, the rest: <= 16 heads,
-//    fp16 batches too small for kPipelined (4 x 64 heads: 17 us), fp8 lists too
+//    fp16 batches too small for kPipelined (4 x 64 heads: 16.6 us), fp8 lists too
 //    long for kSplitDma.
 // Calls that are not split keep O in one fp32 accumulation.  us per call with the
-// splits that would fill the chip best / whole: fp16 16 heads, 129 tokens 85 / 89,
-// 300 103 / 117; 32 heads, 65 tokens 51 / 82, 128 76 / 90, 170 105 / 98; fp8 16
-// heads, 300 tokens 93 / 116, 800 195 / 216, 1000 227 / 217, 2500 523 / 476, 4096
-// 880 / 761.
+// best split of up to four / whole: fp16 16 heads, 129 tokens 76 / 90, 300 89 / 99,
+// 600 153 / 173; 32 heads, 65 tokens 51 / 81, 128 76 / 91, 170 105 / 97; fp8 16 heads,
+// 300 tokens 79 / 103, 800 171 / 191, 1000 194 / 194, 2500 458 / 410, 4096 751 / 651.
 constexpr int kWholeMinKeys = 256;
 enum DecodeKind { kPipelined, kSplitDma, kFewHeads };
 struct DecodePlan {
