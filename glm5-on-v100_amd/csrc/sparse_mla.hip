@@ -1561,8 +1561,8 @@ constexpr int kMergeMaxSplits = 128;  // key splits of one token at most
 // lengths, kps keys each (a multiple of the tile), the smallest kps tried that
 // needs no more slots and no more than kMergeMaxSplits per token, and at most
 // the equal split of the whole width, which always fits.  Every wave that needs
-// the division computes it from seq_lens (B <= 128 tokens, two per lane): the
-// host does not know the lengths.  With one split count for all tokens, 4
+// the division computes it from seq_lens (a token per lane, B <= kShareMaxTokens):
+// the host does not know the lengths.  With one split count for all tokens, 4
 // requests of 32k, 26k, 20k and 14k left 28 % of the workgroups without keys
 // (attention 37.0 -> 33.4 us; whole calls, ragged to a quarter of the longest,
 // 64 heads: 4 x 32k 46.9 -> 44.3 us, 2 x 128k 76.6 -> 69.4; 32 heads, 8 x 32k
@@ -1570,31 +1570,18 @@ constexpr int kMergeMaxSplits = 128;  // key splits of one token at most
 // the chip, the lengths even out over it and the division costs what it saves
 // (16 x 16k ragged 63.6 / 60.5, 40 x 6500 ragged 64.3 / 65.8, 48 x 5000 equal
 // 72.3 / 74.2).
+constexpr int kShareMaxTokens = 64;
 struct DenseShare {
   int kps;
-  int n[2], off[2];  // of tokens lane and 64 + lane: splits, first slot
-  __device__ __forceinline__ int n_of(int b) const {
-    const int lo = __builtin_amdgcn_readlane(n[0], b & 63);
-    const int hi = __builtin_amdgcn_readlane(n[1], b & 63);
-    return b < 64 ? lo : hi;
-  }
-  __device__ __forceinline__ int off_of(int b) const {
-    const int lo = __builtin_amdgcn_readlane(off[0], b & 63);
-    const int hi = __builtin_amdgcn_readlane(off[1], b & 63);
-    return b < 64 ? lo : hi;
-  }
+  int n, off;  // of token lane: splits, first slot
+  __device__ __forceinline__ int n_of(int b) const { return __builtin_amdgcn_readlane(n, b); }
+  __device__ __forceinline__ int off_of(int b) const { return __builtin_amdgcn_readlane(off, b); }
 };
 
 __device__ __forceinline__ DenseShare dense_share(const int32_t* seq_lens, int B, int width, int S) {
   const int lane = threadIdx.x & 63;
-  int len[2], total = 0, longest = 0;
-#pragma unroll
-  for (int j = 0; j < 2; j++) {
-    const int b = lane + 64 * j;
-    len[j] = b < B ? max(0, min(width, seq_lens[b])) : 0;
-    total += (len[j] + kPfTileKeys - 1) / kPfTileKeys;  // in tiles: no overflow
-    longest = max(longest, len[j]);
-  }
+  const int len = lane < B ? max(0, min(width, seq_lens[lane])) : 0;
+  int total = (len + kPfTileKeys - 1) / kPfTileKeys, longest = len;  // in tiles: no overflow
 #pragma unroll
   for (int m = 1; m < 64; m <<= 1) {
     total += __shfl_xor(total, m);
@@ -1606,29 +1593,20 @@ __device__ __forceinline__ DenseShare dense_share(const int32_t* seq_lens, int B
                (longest + kMergeMaxSplits * kPfTileKeys - 1) / (kMergeMaxSplits * kPfTileKeys));
   kt = min(max(__builtin_amdgcn_readfirstlane(kt), 1), most);
   DenseShare r;
-  int incl[2];
+  int incl;
   while (true) {
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-      r.n[j] = (len[j] + kt * kPfTileKeys - 1) / (kt * kPfTileKeys);
-      incl[j] = r.n[j];
-    }
+    r.n = (len + kt * kPfTileKeys - 1) / (kt * kPfTileKeys);
+    incl = r.n;
 #pragma unroll
     for (int m = 1; m < 64; m <<= 1) {
-      const int u0 = __shfl_up(incl[0], m), u1 = __shfl_up(incl[1], m);
-      if (lane >= m) {
-        incl[0] += u0;
-        incl[1] += u1;
-      }
+      const int u = __shfl_up(incl, m);
+      if (lane >= m) incl += u;
     }
-    const int n0 = __builtin_amdgcn_readlane(incl[0], 63);
-    incl[1] += n0;
-    if (kt >= most || __builtin_amdgcn_readlane(incl[1], 63) <= slots) break;
+    if (kt >= most || __builtin_amdgcn_readlane(incl, 63) <= slots) break;
     kt = min(kt + max(kt >> 4, 1), most);
   }
   r.kps = kt * kPfTileKeys;
-  r.off[0] = incl[0] - r.n[0];
-  r.off[1] = incl[1] - r.n[1];
+  r.off = incl - r.n;
   return r;
 }
 
@@ -1647,10 +1625,9 @@ __global__ void __launch_bounds__(kHwThreads, 1) mla_hw_f16_kernel(MlaParams p) 
   if (p.share) {
     const DenseShare ds = dense_share(p.seq_lens, p.B, p.topk, p.n_splits);
     const int slot = (int)(blockIdx.x + gridDim.x * blockIdx.z);
-    const uint64_t in0 = __ballot(slot >= ds.off[0] && slot < ds.off[0] + ds.n[0]);
-    const uint64_t in1 = __ballot(slot >= ds.off[1] && slot < ds.off[1] + ds.n[1]);
-    if ((in0 | in1) == 0) return;  // more slots than splits
-    b = in0 != 0 ? __builtin_ctzll(in0) : 64 + __builtin_ctzll(in1);
+    const uint64_t in = __ballot(slot >= ds.off && slot < ds.off + ds.n);
+    if (in == 0) return;  // more slots than splits
+    b = __builtin_ctzll(in);
     split = slot - ds.off_of(b);
     kps = ds.kps;
     ps_h = ds.n_of(b);
@@ -2733,7 +2710,7 @@ static int mla_decode_impl(
       prm.part_o = reinterpret_cast<f16*>(workspace);
       prm.part_ml = reinterpret_cast<float*>(prm.part_o + (size_t)B * n_head * S * kValueDim);
     }
-    prm.share = S > kMergeBatch && use_hw_f16(topk, S);
+    prm.share = S > kMergeBatch && B <= kShareMaxTokens && use_hw_f16(topk, S);
     int rc = launch_attn_f16(prm, dim3(B, (n_head + 63) / 64, S), st);
     if (rc != MI355_DSA_OK || S == 1) return rc;
     if (S <= kMergeBatch) {
