@@ -232,6 +232,12 @@ __device__ __forceinline__ float relu_mfma(float d) {
   asm("v_max_f32 %0, 0, %1" : "=v"(r) : "v"(d));
   return r;
 }
+// The same against the lowest finite value: NaN and -inf become it, +inf stays.
+__device__ __forceinline__ float finite_low_mfma(float d) {
+  float r;
+  asm("v_max_f32 %0, 0xff7fffff, %1" : "=v"(r) : "v"(d));
+  return r;
+}
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) v = fmaxf(v, shfl_xor_f(v, m));

@@ -954,13 +954,17 @@ __device__ __forceinline__ void ws_sm_role(const MlaParams& p, const WsCtx& x, W
 #pragma unroll
       for (int q = 1; q < 4; q++) s4[hf] += sq[q][hf];
     }
-    if (masked) {  // wave-uniform: most tiles hold no masked key
+    // wave-uniform: most tiles hold no masked key.  The batches that the split
+    // decode shares (exact maximum) take a NaN score as masked, as it does.
+    if (masked || p.lazy_max == 0.f) {
       const int4 vr0 = *reinterpret_cast<const int4*>(trows + 8 * kq);
       const int4 vr1 = *reinterpret_cast<const int4*>(trows + 8 * kq + 4);
       const int vv[8] = {vr0.x, vr0.y, vr0.z, vr0.w, vr1.x, vr1.y, vr1.z, vr1.w};
 #pragma unroll
-      for (int k = 0; k < 8; k++)  // -2: zero row, a valid key
-        s4[k >> 2][k & 3] = vv[k] != -1 ? s4[k >> 2][k & 3] : -INFINITY;
+      for (int k = 0; k < 8; k++) {  // -2: zero row, a valid key
+        const float x = s4[k >> 2][k & 3];
+        s4[k >> 2][k & 3] = vv[k] != -1 && (x == x || p.lazy_max > 0.f) ? x : -INFINITY;
+      }
     }
     float mt = -1e30f;
 #pragma unroll
@@ -1482,7 +1486,7 @@ struct HwSmem {
   int32_t rows[kSegKeys];
   float m[2][64], l[2][64];           // [key group][head]
   int tmask[kSegKeys / kPfTileKeys];  // tile of the segment holds a masked key (row -1)
-  int last[kHwWaves];
+  int last[kHwWaves], bad[kHwWaves];
 };
 static_assert(sizeof(HwSmem) <= 160 * 1024, "one workgroup per CU");
 static_assert(offsetof(HwSmem, m) >= kHwWaves * 8 * 64 * 64, "the O exchange ends below m and l");
@@ -1661,9 +1665,14 @@ __global__ void __launch_bounds__(kHwThreads, 1) mla_hw_f16_kernel(MlaParams p) 
   }
 
   // O^T tile t: dims 32 t + 8 a + 4 hf + r (element 4 a + r), head c
-  hw_own_agprs();
-  unroll<256>([&](auto i) { hw_zero<i>(); });
-  float m_run = -1e30f, l_part = 0.f;  // l: this lane's keys only
+  float m_run, l_part;  // l: this lane's keys only
+  auto clear = [&]() {
+    hw_own_agprs();
+    unroll<256>([&](auto i) { hw_zero<i>(); });
+    m_run = -1e30f;
+    l_part = 0.f;
+  };
+  clear();
 
   // LDS addresses within a slot
   const uint32_t lds0 = (uint32_t)(uintptr_t)(&sh.ring[kw][0][0]);
@@ -1718,7 +1727,10 @@ __global__ void __launch_bounds__(kHwThreads, 1) mla_hw_f16_kernel(MlaParams p) 
     // later would drain the tiles in flight
     __builtin_amdgcn_s_waitcnt(0x0f70);
   }
-  for (int seg_lo = k_lo; seg_lo < k_hi; seg_lo += kSegKeys) {
+  // NaN scores count as masked.  They show as a NaN row sum, and the keys are
+  // then run again with every score tested, so the usual pass tests none.
+  bool safe = false;
+  for (int seg_lo = k_lo;;) {
     for (int t0 = 0; t0 < ntiles; t0 += 2) {
       const int tile = t0 + kw, par = (t0 >> 1) & 1;
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1745,6 +1757,10 @@ __global__ void __launch_bounds__(kHwThreads, 1) mla_hw_f16_kernel(MlaParams p) 
             if (rc.w == -1) s[4 * a + 3] = -INFINITY;
           }
         }
+        if (safe) {
+#pragma unroll
+          for (int e = 0; e < 16; e++) s[e] = s[e] == s[e] ? s[e] : -INFINITY;
+        }
         float mt = fmaxf(s[0], s[1]);
 #pragma unroll
         for (int e = 2; e < 16; e++) mt = fmaxf(mt, s[e]);
@@ -1762,20 +1778,27 @@ __global__ void __launch_bounds__(kHwThreads, 1) mla_hw_f16_kernel(MlaParams p) 
         hw_own_agprs();
       }
     }
-    if (seg_lo + kSegKeys < k_hi) {
-      resolve_idx<kHwThreads>(p, b, seg_lo + kSegKeys, min(k_hi - seg_lo - kSegKeys, kSegKeys), 0, pos);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last round's DMA past the end too
-      lds_barrier();  // rows, flags and the ring are free
-      ntiles = start_segment(seg_lo + kSegKeys);
-      __builtin_amdgcn_s_waitcnt(0x0f70);
+    seg_lo += kSegKeys;
+    if (seg_lo >= k_hi) {
+      const int bad = !safe && __any(l_part != l_part);
+      if (lane == 0) sh.bad[w] = bad;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_barrier();  // the ring is idle
+      if (!__builtin_amdgcn_readfirstlane(sh.bad[0] | sh.bad[1] | sh.bad[2] | sh.bad[3])) break;
+      safe = true;
+      seg_lo = k_lo;
+      clear();
     }
+    resolve_idx<kHwThreads>(p, b, seg_lo, min(k_hi - seg_lo, kSegKeys), 0, pos);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last round's DMA past the end too
+    lds_barrier();  // rows, flags and the ring are free
+    ntiles = start_segment(seg_lo);
+    __builtin_amdgcn_s_waitcnt(0x0f70);
   }
 
   // ---- merge the key groups: wave (hw, kw) finishes dims [256 kw, +256) of
   // its heads and hands the other half to wave (hw, 1 - kw) ----
   const float l_own = l_part + __shfl_xor(l_part, 32, 64);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  lds_barrier();  // the ring is idle
   if (hf == 0) {
     sh.m[kw][32 * hw + c] = m_run;
     sh.l[kw][32 * hw + c] = l_own;
@@ -1871,7 +1894,8 @@ __global__ void __launch_bounds__(kHwThreads, 1) mla_hw_f16_kernel(MlaParams p) 
 //     (one fp8 scale tile): P times the source wave's exp(m_w - m) and the key's
 //     scale, rounded to fp16 once; a barrier frees the tile.
 // The running max m is the same in every wave; lazy (kPfLazyMax) for fp16 rows,
-// exact for fp8 rows, whose P times the tile scale must stay inside fp16.
+// exact for fp8 rows, whose P times the tile scale must stay inside fp16.  A NaN score
+// counts as masked, as in the split decode (2048 tokens x 16 heads fp8 337 -> 341 us).
 // Region layout: 64-byte blocks, block-major (block b of key r at 1024 b + 64 r),
 // piece p of a block at p ^ few_sw(r): the QK reads (16 keys x 4 pieces) and the
 // transpose reads are free of bank conflicts, and a DMA instruction fetches a
@@ -2049,7 +2073,8 @@ __global__ void __launch_bounds__(kFewThreads, FP8 ? 3 : 2) sparse_mla_few_kerne
       float mt = -1e30f;
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        sv[r] = vv[r] != -1 ? sv[r] : -INFINITY;  // -2: a zero row, a valid key
+        // -2: a zero row, a valid key; a NaN score counts as masked (p = 0 too)
+        sv[r] = vv[r] != -1 ? finite_low_mfma(sv[r]) : -INFINITY;
         mt = fmaxf(mt, sv[r]);
       }
       mt = xor32_max(xor16_max(mt));

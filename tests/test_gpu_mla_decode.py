@@ -71,7 +71,8 @@ SHARED = [
     (32, [12000, 0, 1, 31, 33, 480, 512, 513, 5000, 64, 2000, 11999]),
     (96, [20300, 7, 300]),              # two 64-head groups
     (32, [21100, 40, 40, 0, 40, 33]),   # one token takes more splits than the equal share
-    (64, [30000, 30000]),               # equal lengths: the equal split
+    (64, [30000, 30000]),               # fewer tiles: not divided by length
+    (64, [31000, 31000, 31000, 31000]),  # equal lengths: the equal split
 ]
 
 
@@ -85,6 +86,33 @@ def test_splits_by_length(ops, dev, H, seqs):
     assert not torch.isnan(o).any() and not torch.isnan(lse).any()
     ro, rl = O.mla_decode(q, kv, bt, seq, SCALE)
     check(o, lse, ro, rl)
+
+
+@pytest.mark.parametrize("H,seqs", [(64, [31000, 5000, 31000, 200]), (32, [6000] * 20),
+                                    (64, [600] * 300), (64, [30000, 5000])],
+                         ids=["shared-splits", "splits", "whole", "few-tiles"])
+def test_nan_scores_are_masked(ops, dev, H, seqs):
+    """A key with a NaN RoPE element is left out, a query with one sees no key."""
+    page, B = 64, len(seqs)
+    mb = (max(seqs) + page - 1) // page
+    q, kv, bt, seq = make(40 + B, B, H, mb + 8, page, seqs, mb)
+    bad = kv.clone()
+    some = torch.tensor([0, 1])
+    # the oracle has no masking by value: a key as far below the others as fp16 goes
+    # weighs nothing
+    q[:, :, 512] = 8.0
+    for t in (kv, bad):
+        t.view(-1, 576)[:, 512] = 0
+    kv.view(-1, 576)[::7, 512] = -60000.0
+    bad.view(-1, 576)[::7, 512] = float("nan")
+    ro, rl = O.mla_decode(q[some], kv, bt[some], seq[some], SCALE)
+    q[1, H - 1, 5] = float("nan")
+    o, lse = run(ops, dev, q, bad, bt, seq)
+    assert (o[1, H - 1] == 0).all() and torch.isneginf(lse[1, H - 1])
+    ro[1, H - 1], rl[1, H - 1] = o[1, H - 1], lse[1, H - 1]
+    check(o[some], lse[some], ro, rl)
+    assert torch.isfinite(o).all()
+
 
 
 def test_unresolvable_rows_are_zero_keys(ops, dev):

@@ -457,3 +457,38 @@ def test_c3_full_size(ops, pkg, dev):
     seq_c = torch.full((B,), n, dtype=torch.int32)
     ro, rl = O.sparse_mla(d["q"].cpu(), kv_c, idx_c, bt_c, seq_c, d["scale"])
     check(o.float().cpu(), lse.cpu(), ro, rl)
+
+
+NAN_SCORES = [
+    # B, H, fp8, topk: whole-head waves (split, whole, two segments), 16-head
+    # workgroups of both row types, the 64-head fp8 kernel below 33 heads, the
+    # fp8 split decode
+    (100, 64, False, 2048), (256, 64, False, 700), (256, 70, False, 2112), (4, 64, False, 1024),
+    (140, 16, False, 130), (64, 16, True, 2048), (300, 16, True, 700), (100, 24, True, 2048),
+    (8, 16, True, 512),
+]
+
+
+@pytest.mark.parametrize("B,H,fp8,topk", NAN_SCORES,
+                         ids=["B%dH%d%sK%d" % (b, h, "fp8" if f else "fp16", k)
+                              for b, h, f, k in NAN_SCORES])
+def test_nan_scores_are_masked(ops, dev, B, H, fp8, topk):
+    """A key with a NaN RoPE element is left out, a query with one sees no key."""
+    q, kv, idx, bt, seq = make(300 + B, B, H, 60, 64, fp8, topk, [3000] * B, shared_bt=True)
+    rows = kv.view(60 * 64, -1)
+    rope = rows[:, 528:].view(torch.float16) if fp8 else rows[:, 512:]
+    rope[::7, 3] = float("nan")
+    pos = idx.clamp(min=0).long()
+    phys = bt[0].long()[pos // 64] * 64 + pos % 64
+    keep = torch.where((idx >= 0) & (phys % 7 == 0), -1, idx)
+    assert (keep != idx).any()
+    some = torch.tensor(sorted({0, 1, B // 2, B - 1}))
+    ro, rl = O.sparse_mla(q[some], kv, keep[some], bt[some], seq[some], SCALE,
+                          empty_lse=-1e30 if B >= 32 and H <= 16 else None,
+                          zero_unresolved=not (B >= 32 and H <= 16))
+    q[1, H - 1, 5] = float("nan")
+    o, lse = run(ops, dev, q, kv, idx, bt, seq)
+    assert (o[1, H - 1] == 0).all() and lse[1, H - 1] <= -1e30
+    ro[1, H - 1], rl[1, H - 1] = o[1, H - 1], lse[1, H - 1]
+    check(o[some], lse[some], ro, rl)
+    assert torch.isfinite(o).all()
