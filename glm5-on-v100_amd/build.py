@@ -52,7 +52,9 @@ def compile_flags() -> list[str]:
 OWN_AGPRS = {"sparse_mla.hip": ["mla_hw_f16_kernel"]}
 # Kernels that must not spill: a reload in a loop waits for all of the wave's
 # memory operations, gathers in flight included.
-NO_SPILLS = {"sparse_mla.hip": ["sparse_mla_prefill_fp8_ws_kernel", "sparse_mla_few_kernelILb0E"]}
+NO_SPILLS = {"sparse_mla.hip": ["sparse_mla_prefill_fp8_ws_kernel", "sparse_mla_few_kernelILb0E"],
+             "varlen_attn.hip": [f"varlen_attn_ring_kernelILb{t}ELi{d}E" for t in (0, 1)
+                                 for d in (192, 128, 64)]}
 
 
 def _body(asm: str, kernel: str) -> tuple[str, list[str]]:
@@ -102,14 +104,15 @@ def _compile(src: str) -> str:
     name = os.path.basename(src)
     obj = os.path.join(BUILD_DIR, name.replace(".hip", ".o"))
     cmd = [hipcc(), *compile_flags(), "-c", src, "-o", obj]
-    if name in OWN_AGPRS:  # the assembly that the object is made from, beside it
+    checked = name in OWN_AGPRS or name in NO_SPILLS
+    if checked:  # the assembly that the object is made from, beside it
         cmd.append("-save-temps=obj")
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stdout}\n{r.stderr}")
-    if name in OWN_AGPRS:
+    if checked:
         with open(asm_path(name)) as f:
-            check_kernels(f.read(), OWN_AGPRS[name], NO_SPILLS.get(name, []))
+            check_kernels(f.read(), OWN_AGPRS.get(name, []), NO_SPILLS.get(name, []))
     return obj
 
 

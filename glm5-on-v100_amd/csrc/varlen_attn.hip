@@ -358,6 +358,12 @@ int launch_va(const VaArgs& a0, int num_seqs, int max_q_len, hipStream_t st) {
 // 5.9 ms, the grouped MFMA / VALU order 5.66 ms (the compiler's own order put
 // the exponentials before the MFMAs).  Measured level: 2 K reads ahead instead
 // of 3, two steps per loop iteration, groups of 4-16 query tiles per pair.
+// Sequences of one or two steps are all prologue and epilogue.  Addresses of the
+// NaN pass and of the outputs kept over the loop spilled 22 registers there, and
+// the flags between the waves went by flat loads: 16 x 64 tokens, 64 heads, fp16 22.0
+// us with the two-stage kernel, 26.3 so, 21.2 without either (8 x 500 115 -> 106 us;
+// one workgroup over 4000 keys 98 -> 100).  A branch around the step past the last one
+// slows such long single workgroups by another 4 %.
 // ---------------------------------------------------------------------------
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -511,10 +517,10 @@ __global__ void __launch_bounds__(kVaThreads, 2) varlen_attn_ring_kernel(VaArgs 
   };
 
   // the ring's first three steps
-  auto prologue = [&]() {
+  auto prologue = [&](int first) {
 #pragma unroll
     for (int i = 0; i < 3; i++)
-      if (i < n) issue(i);
+      if (i < n) issue(first + i);
   };
   auto max16 = [&](const f32x16& x) {
     float m = fmaxf(x[0], x[1]);
@@ -522,7 +528,7 @@ __global__ void __launch_bounds__(kVaThreads, 2) varlen_attn_ring_kernel(VaArgs 
     for (int e = 2; e < 16; e++) m = fmaxf(m, x[e]);
     return xor32_max(m);
   };
-  prologue();
+  prologue(0);
   // Q completes here, beside the first steps.  The compiler does not count
   // the DMAs issued by inline asm, so a wait for Q left to the loop would
   // drain the steps in flight.
@@ -639,25 +645,33 @@ __global__ void __launch_bounds__(kVaThreads, 2) varlen_attn_ring_kernel(VaArgs 
       s = sn;
     }
     if (safe) break;
-    volatile int* redo = reinterpret_cast<int*>(smem_raw);  // the ring is idle here
+    // the flags lie past the waves' output rows
     const int bad = __any(l_part != l_part);  // of all 64 lanes
+    lds_barrier();  // the ring is idle
+    if (lane == 0) *(__attribute__((address_space(3))) int*)(lds0 + 256 * DV + 4 * w) = bad;
     lds_barrier();
-    if (lane == 0) redo[w] = bad;
+    const u32x4 redo = *(const __attribute__((address_space(3))) u32x4*)(lds0 + 256 * DV);
+    if (__builtin_amdgcn_readfirstlane(redo[0] | redo[1] | redo[2] | redo[3]) == 0) break;
     lds_barrier();
-    if (!(redo[0] | redo[1] | redo[2] | redo[3])) break;
-    lds_barrier();
-    prologue();
+    // (a first step that the compiler does not know: no address of this rare
+    // pass is kept from the first one, in registers that the loop needs)
+    int first = 0;
+    asm volatile("" : "+s"(first));
+    prologue(first);
   }
 
   // ---- outputs: lane c's query, dims 32 t + 8 u + 4 hf .. +3, turned into
   // whole rows in the wave's part of the idle ring (16-byte piece j of row r
   // at j ^ (r & 7)), so that every store writes full rows ----
+  // (an opaque lane, so that no address of the outputs is kept over the loop)
+  int ln = lane;
+  asm volatile("" : "+v"(ln));
+  const int co = ln & 31, ho = ln >> 5, qo = q0 + 32 * w + co;
   float l = l_part;
   l += __shfl_xor(l, 32, 64);
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  if (a.lse != nullptr && hf == 0 && qi < q_len)
-    a.lse[(int64_t)h * a.total_q + qs + qi] = l > 0.f ? m_run * a.scale + logf(l) : -INFINITY;
-  lds_barrier();
+  if (a.lse != nullptr && ho == 0 && qo < q_len)
+    a.lse[(int64_t)h * a.total_q + qs + qo] = l > 0.f ? m_run * a.scale + logf(l) : -INFINITY;
   constexpr int NP16 = DV / 8;  // 16-byte pieces of an output row
   unsigned char* const ow = smem_raw + w * (32 * 2 * DV);
 #pragma unroll
@@ -666,12 +680,12 @@ __global__ void __launch_bounds__(kVaThreads, 2) varlen_attn_ring_kernel(VaArgs 
     for (int u = 0; u < 4; u++) {
       const u32x2 pk = {pack16<BF16>(oacc[t][4 * u] * inv, oacc[t][4 * u + 1] * inv),
                         pack16<BF16>(oacc[t][4 * u + 2] * inv, oacc[t][4 * u + 3] * inv)};
-      *reinterpret_cast<u32x2*>(ow + c * (2 * DV) + 16 * ((4 * t + u) ^ (c & 7)) + 8 * hf) = pk;
+      *reinterpret_cast<u32x2*>(ow + co * (2 * DV) + 16 * ((4 * t + u) ^ (co & 7)) + 8 * ho) = pk;
     }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own rows
 #pragma unroll
   for (int u = 0; u < NP16 / 2; u++) {
-    const int r = (64 / NP16) * u + lane / NP16, j = lane % NP16;
+    const int r = (64 / NP16) * u + ln / NP16, j = ln % NP16;
     const u32x4 x = *reinterpret_cast<const u32x4*>(ow + r * (2 * DV) + 16 * (j ^ (r & 7)));
     const int i = q0 + 32 * w + r;
     if (i >= q_len) continue;
