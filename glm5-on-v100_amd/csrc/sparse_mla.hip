@@ -954,17 +954,20 @@ __device__ __forceinline__ void ws_sm_role(const MlaParams& p, const WsCtx& x, W
 #pragma unroll
       for (int q = 1; q < 4; q++) s4[hf] += sq[q][hf];
     }
-    // wave-uniform: most tiles hold no masked key.  The batches that the split
-    // decode shares (exact maximum) take a NaN score as masked, as it does.
-    if (masked || p.lazy_max == 0.f) {
+    // The batches that the split decode shares (exact maximum) take a NaN score
+    // as masked, as it does: p = 0 (200 tokens x 32 heads 95.9 -> 97.7 us; with the
+    // masked keys' selects 103).
+    if (p.lazy_max == 0.f) {
+#pragma unroll
+      for (int k = 0; k < 8; k++) s4[k >> 2][k & 3] = finite_low_mfma(s4[k >> 2][k & 3]);
+    }
+    if (masked) {  // wave-uniform: most tiles hold no masked key
       const int4 vr0 = *reinterpret_cast<const int4*>(trows + 8 * kq);
       const int4 vr1 = *reinterpret_cast<const int4*>(trows + 8 * kq + 4);
       const int vv[8] = {vr0.x, vr0.y, vr0.z, vr0.w, vr1.x, vr1.y, vr1.z, vr1.w};
 #pragma unroll
-      for (int k = 0; k < 8; k++) {  // -2: zero row, a valid key
-        const float x = s4[k >> 2][k & 3];
-        s4[k >> 2][k & 3] = vv[k] != -1 && (x == x || p.lazy_max > 0.f) ? x : -INFINITY;
-      }
+      for (int k = 0; k < 8; k++)  // -2: zero row, a valid key
+        s4[k >> 2][k & 3] = vv[k] != -1 ? s4[k >> 2][k & 3] : -INFINITY;
     }
     float mt = -1e30f;
 #pragma unroll
