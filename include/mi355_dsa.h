@@ -380,7 +380,7 @@ int mi355_dsa_sparse_mla_decode(void* o, float* lse, const void* q, int B,
  * mi355_dsa_sparse_mla_noalloc_max_bytes() bytes (32 MiB) per device, held
  * from the library's load until the process ends; a call needing more
  * (mi355_dsa_sparse_mla_workspace_size(B, n_head, topk) larger than that,
- * e.g. B >= 128 at 16 heads and topk 2048; no 64-head shape at topk 2048)
+ * e.g. at topk 2048 16 heads at B 128-255, 32 heads at 64-255; no call above 32)
  * returns MI355_DSA_EINVAL and
  * launches nothing.  Every call on one device shares that device's array:
  * calls that overlap on one device (different streams) race and must be
